@@ -113,6 +113,7 @@ E3Launch base_launch(atmo_handle* h) {
   L.surface_flux = h->cfg.surface_flux;
   L.surface_noncons = h->cfg.surface_noncons;
   L.cv = h->d_cv;
+  L.cv_rows = 1;
   L.cv_t = h->cfg.precision == ATMO_PREC_FP64 ? (const void*)h->d_cv : (const void*)h->d_cv32;
   L.invJ = h->d_invJ;
   L.dsplit = h->dsplit.data();
@@ -614,28 +615,33 @@ int atmo_create(const atmo_config* cfg, const atmo_geometry3d* g, atmo_handle** 
     fail(nullptr, ATMO_ERR_DEVICE, "device allocation failed");
     return cleanup_fail(ATMO_ERR_DEVICE);
   }
-  if (metric_on_device) {
-    // upload the node coordinates only and compute the metric terms here
-    double* d_xyz = nullptr;
-    Basis b(n);
-    const bool ok = hipMalloc(&d_xyz, sizeof(double) * 3 * n3 * (size_t)E) == hipSuccess &&
-                    hipMemcpy(d_xyz, g->node_coordinates, sizeof(double) * 3 * n3 * (size_t)E,
-                              hipMemcpyHostToDevice) == hipSuccess &&
-                    e3_launch_metric_terms(n, E, b.D.data(), d_xyz, h->d_cv, h->d_invJ, h->stream) &&
-                    hipGetLastError() == hipSuccess;
-    if (ok && h->d_cv32) launch_narrow_to_float(h->d_cv, h->d_cv32, (size_t)9 * n3 * E, h->stream);
-    const bool done = ok && hipStreamSynchronize(h->stream) == hipSuccess;
+  {
+    // the vectors in the caller's layout, uploaded or computed on the device
+    // from the node coordinates alone, then as the rows the stages read
+    double *d_xyz = nullptr, *d_cv9 = nullptr;
+    const size_t cb = sizeof(double) * 9 * n3 * (size_t)E, nb = sizeof(double) * n3 * (size_t)E;
+    bool ok = hipMalloc(&d_cv9, cb) == hipSuccess;
+    if (ok && metric_on_device) {
+      Basis b(n);
+      ok = hipMalloc(&d_xyz, 3 * nb) == hipSuccess &&
+           hipMemcpy(d_xyz, g->node_coordinates, 3 * nb, hipMemcpyHostToDevice) == hipSuccess &&
+           e3_launch_metric_terms(n, E, b.D.data(), d_xyz, d_cv9, h->d_invJ, h->stream);
+    } else if (ok) {
+      ok = hipMemcpy(d_cv9, g->contravariant_vectors, cb, hipMemcpyHostToDevice) == hipSuccess &&
+           hipMemcpy(h->d_invJ, g->inverse_jacobian, nb, hipMemcpyHostToDevice) == hipSuccess;
+    }
+    if (ok) {
+      e3_launch_vector_rows(d_cv9, h->d_cv, n3, E, h->stream);
+      if (h->d_cv32) launch_narrow_to_float(h->d_cv, h->d_cv32, (size_t)9 * n3 * E, h->stream);
+      ok = hipGetLastError() == hipSuccess && hipStreamSynchronize(h->stream) == hipSuccess;
+    }
     if (d_xyz) (void)hipFree(d_xyz);
-    if (!done) {
-      fail(nullptr, ATMO_ERR_DEVICE, "metric terms on the device failed");
+    if (d_cv9) (void)hipFree(d_cv9);
+    if (!ok) {
+      fail(nullptr, ATMO_ERR_DEVICE,
+           metric_on_device ? "metric terms on the device failed" : "device upload failed");
       return cleanup_fail(ATMO_ERR_DEVICE);
     }
-  } else if (hipMemcpy(h->d_cv, g->contravariant_vectors, sizeof(double) * 9 * n3 * (size_t)E,
-                       hipMemcpyHostToDevice) != hipSuccess ||
-             hipMemcpy(h->d_invJ, g->inverse_jacobian, sizeof(double) * n3 * (size_t)E,
-                       hipMemcpyHostToDevice) != hipSuccess) {
-    fail(nullptr, ATMO_ERR_DEVICE, "device upload failed");
-    return cleanup_fail(ATMO_ERR_DEVICE);
   }
   if (hipMemcpy(h->d_nbr, nbr.data(), sizeof(int32_t) * nbr.size(), hipMemcpyHostToDevice) !=
           hipSuccess ||
@@ -645,15 +651,6 @@ int atmo_create(const atmo_config* cfg, const atmo_geometry3d* g, atmo_handle** 
       hipMemset(h->d_k, 0, sb) != hipSuccess) {
     fail(nullptr, ATMO_ERR_DEVICE, "device upload failed");
     return cleanup_fail(ATMO_ERR_DEVICE);
-  }
-  if (h->d_cv32 && !metric_on_device) {
-    std::vector<float> cv32((size_t)9 * n3 * E);
-    for (size_t q = 0; q < cv32.size(); ++q) cv32[q] = (float)g->contravariant_vectors[q];
-    if (hipMemcpy(h->d_cv32, cv32.data(), sizeof(float) * cv32.size(), hipMemcpyHostToDevice) !=
-        hipSuccess) {
-      fail(nullptr, ATMO_ERR_DEVICE, "device upload failed");
-      return cleanup_fail(ATMO_ERR_DEVICE);
-    }
   }
   *out = h;
   return ATMO_OK;

@@ -89,6 +89,14 @@ __global__ __launch_bounds__(GeoShape<N>::BLOCK) void e3_metric_terms_kernel(
   invJ[g] = 1.0 / det;
 }
 
+__global__ void vector_rows_kernel(const double* __restrict__ cv, double* __restrict__ rows, int n3,
+                                   size_t total) {
+  const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;  // index into rows
+  if (q >= total) return;
+  const size_t row = q / n3, node = q - row * n3, e = row / 9, c = row - e * 9;
+  rows[q] = cv[(e * n3 + node) * 9 + c];
+}
+
 __global__ void narrow_to_float_kernel(const double* __restrict__ a, float* __restrict__ b,
                                        size_t n) {
   const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -118,6 +126,12 @@ bool e3_launch_metric_terms(int n, int n_elements, const double* D, const double
     default:
       return false;
   }
+}
+
+void e3_launch_vector_rows(const double* cv, double* rows, int n3, int n_elements, hipStream_t s) {
+  const size_t total = (size_t)9 * n3 * n_elements;
+  hipLaunchKernelGGL(vector_rows_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
+                     cv, rows, n3, total);
 }
 
 void launch_narrow_to_float(const double* a, float* b, size_t n, hipStream_t s) {

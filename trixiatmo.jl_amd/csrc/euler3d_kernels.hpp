@@ -31,9 +31,10 @@ struct E3Launch {
   int mode;  // 0 rhs, 1 RK stage
   const double* u;
   double* out;
-  double* k;              // RK register [5, nodes] (phi has no tendency)
+  double* k;              // RK register [e][5][n^3] (phi has no tendency)
   const double* cv;       // FP64 contravariant vectors (reductions)
-  const void* cv_t;       // contravariant vectors in the stage kernel's compute type
+  int cv_rows;            // cv is [e][9][n^3] (a handle's layout) instead of [e][n^3][9]
+  const void* cv_t;       // contravariant vectors [e][9][n^3] in the stage kernel's storage type
   const double* invJ;
   const double* dsplit;   // host copy of Dsplit[n*n]
   const double* weights;  // host copy of the LGL weights[n]
@@ -69,6 +70,8 @@ bool e3_launch_reduction(const E3Launch& L, int which, const double* du, double*
 // coordinates [3,n,n,n,E] (D: the n x n derivative matrix); false for n > 8
 bool e3_launch_metric_terms(int n, int n_elements, const double* D, const double* xyz,
                             double* cv, double* invJ, hipStream_t s);
+// [e][n^3][9] -> [e][9][n^3] for the n_elements elements of n3 nodes
+void e3_launch_vector_rows(const double* cv, double* rows, int n3, int n_elements, hipStream_t s);
 // b[q] = (float) a[q]
 void launch_narrow_to_float(const double* a, float* b, size_t n, hipStream_t s);
 

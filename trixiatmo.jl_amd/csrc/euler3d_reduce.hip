@@ -20,8 +20,10 @@ struct WeightTable {
 };
 
 // ---------------------------------------------------------------- reductions
-// per element: max over nodes of |Ja^d . lambda| / J summed over d
-template <int N>
+// per element: max over nodes of |Ja^d . lambda| / J summed over d.  ROWS: the
+// contravariant vectors in the handle's layout [e][9][n^3] (each entry's row
+// contiguous over the element's nodes), else the caller's [e][n^3][9]
+template <int N, bool ROWS>
 __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_max_speed(E3Params q, const double* __restrict__ u,
                                                                const double* __restrict__ cv,
                                                                const double* __restrict__ invJ,
@@ -35,7 +37,10 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_max_speed(E3Params q, cons
     const size_t g = (size_t)e * N3 + t;
     double uu[6], l[3];
     for (int v = 0; v < 6; ++v) uu[v] = u[g * 6 + v];
-    node_scaled_speeds(q, uu, cv + g * 9, fabs(invJ[g]), l);
+    if constexpr (ROWS)
+      node_scaled_speeds(q, uu, cv + (size_t)e * (9 * N3) + t, N3, fabs(invJ[g]), l);
+    else
+      node_scaled_speeds(q, uu, cv + g * 9, 1, fabs(invJ[g]), l);
     l1 = l[0];
     l2 = l[1];
     l3 = l[2];
@@ -128,9 +133,12 @@ static void launch_red(const E3Launch& L, int which, const double* du, double* p
   WeightTable wt{};
   if (which != 0)
     for (int q = 0; q < N; ++q) wt.w[q] = L.weights[q];
-  if (which == 0)
-    hipLaunchKernelGGL((e3_max_speed<N>), dim3(L.n_elements), dim3(Shape<N>::BLOCK), 0, s, L.q,
-                       L.u, L.cv, L.invJ, partial);
+  if (which == 0 && L.cv_rows)
+    hipLaunchKernelGGL((e3_max_speed<N, true>), dim3(L.n_elements), dim3(Shape<N>::BLOCK), 0, s,
+                       L.q, L.u, L.cv, L.invJ, partial);
+  else if (which == 0)
+    hipLaunchKernelGGL((e3_max_speed<N, false>), dim3(L.n_elements), dim3(Shape<N>::BLOCK), 0, s,
+                       L.q, L.u, L.cv, L.invJ, partial);
   else
     hipLaunchKernelGGL((e3_integrals<N>), dim3(L.n_elements), dim3(Shape<N>::BLOCK), 0, s, L.q,
                        wt, L.u, du, L.invJ, partial);

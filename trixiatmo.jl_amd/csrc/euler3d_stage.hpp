@@ -25,6 +25,12 @@
 // KAHAN is set).  With the background split the momentum rows carry only
 // p' = p - p_bg and (rho_avg - rho_avg,bg) [phi]; the FP64 tendency of the
 // background is added back, so the discretisation is unchanged.
+//
+// The metric terms and the RK register are kept as rows over an element's
+// nodes ([e][9][n^3] and [e][5][n^3]), so 64 lanes read 512 contiguous bytes
+// per entry instead of a stride of 72 or 40 bytes: shell 6 x 16^2 x 8 at
+// polydeg 4, 150 resident steps 101.9 against 103.0 ms (two alternating
+// runs); the other sizes within noise.
 #ifndef ATMO_EULER3D_STAGE_HPP
 #define ATMO_EULER3D_STAGE_HPP
 
@@ -412,13 +418,14 @@ __device__ __forceinline__ void face_normals(FaceNormals<N, T, EPB>& fn, int e0,
 #pragma unroll
       for (int c = 0; c < 3; ++c)
         if constexpr (LDS_CV) fn.n[ps][c] = sgn * s_cv[es * cv_stride + (3 * d + c) * N3 + node];
-        else fn.n[ps][c] = sgn * T(cv[(e * N3 + node) * 9 + 3 * d + c]);
+        else fn.n[ps][c] = sgn * T(cv[(e * 9 + 3 * d + c) * N3 + node]);
     } else {
       const int dp = info & 7;
       const T sgn = (dp % 2 == 0) ? T(1) : T(-1);  // minus the primary's outward normal
-      const G* jp = cv + (size_t)link * 9 + 3 * (dp / 2);
+      const int le = link / N3, ln = link - le * N3;
+      const G* jp = cv + ((size_t)le * 9 + 3 * (dp / 2)) * N3 + ln;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) fn.n[ps][c] = sgn * T(jp[c]);
+      for (int c = 0; c < 3; ++c) fn.n[ps][c] = sgn * T(jp[c * N3]);
     }
   }
 }
@@ -608,10 +615,10 @@ __device__ __forceinline__ FastPrim<T> load_fast_prim(const T* s_w, int node, co
 template <int N, typename T, bool KAHAN>
 __device__ __forceinline__ void stage_epilogue(
     const Acc<T, KAHAN>* acc, const Acc<T, KAHAN>* acc_nc, const T* s_sf, int ti, int tj, int tk,
-    size_t gnode, const double* __restrict__ u, double* __restrict__ out,
+    int e, size_t gnode, const double* __restrict__ u, double* __restrict__ out,
     double* __restrict__ kreg, const double* __restrict__ invJ, int mode, double rk_a,
     double rk_dt, double rk_b, double coriolis, const Background& bg, double* un) {
-  constexpr int NV = 6, N2 = Shape<N>::N2;
+  constexpr int NV = 6, N2 = Shape<N>::N2, N3 = Shape<N>::N3;
   double du[NV];
   du[0] = double(acc[0].value());
 #pragma unroll
@@ -654,10 +661,11 @@ __device__ __forceinline__ void stage_epilogue(
 #pragma unroll
     for (int v = 0; v < NV; ++v) out[gnode * NV + v] = du[v];
   } else {
+    double* kn_ = kreg + (size_t)e * ((NV - 1) * N3) + (gnode - (size_t)e * N3);
 #pragma unroll
     for (int v = 0; v < NV - 1; ++v) {
-      const double kn = rk_a * kreg[gnode * (NV - 1) + v] + rk_dt * du[v];
-      kreg[gnode * (NV - 1) + v] = kn;
+      const double kn = rk_a * kn_[v * N3] + rk_dt * du[v];
+      kn_[v * N3] = kn;
       un[v] = uo[v] + rk_b * kn;
       out[gnode * NV + v] = un[v];
     }
@@ -668,15 +676,19 @@ __device__ __forceinline__ void stage_epilogue(
 // new states un (the resident loop's next step size), reduced over the
 // element's slot of BE lanes with speed_max (exact, so any order gives the
 // max-speed reduction's value); every thread of the workgroup takes part
-template <int BE, int EPB = 1>
+template <int N, int EPB = 1>
 __device__ __forceinline__ void element_speed(const E3Params& q, bool active, const double* un,
                                               const double* __restrict__ cv64,
                                               const double* __restrict__ invJ, size_t gnode,
                                               int t, int e0, int n_valid, double (*red)[3],
                                               double* partial) {
+  constexpr int BE = Shape<N>::BLOCK, N3 = Shape<N>::N3;
   constexpr int WPS = BE / 64;  // waves per element slot
   double l[3] = {0.0, 0.0, 0.0};
-  if (active) node_scaled_speeds(q, un, cv64 + gnode * 9, fabs(invJ[gnode]), l);
+  if (active) {
+    const size_t e = e0 + t / BE;
+    node_scaled_speeds(q, un, cv64 + e * (9 * N3) + (gnode - e * N3), N3, fabs(invJ[gnode]), l);
+  }
 #pragma unroll
   for (int d = 0; d < 3; ++d)
 #pragma unroll
@@ -742,9 +754,8 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
   for (int d = 0; d < 3; ++d) {
     __syncthreads();
     if (active) {
-      s_ja[0][t] = cv[gnode * 9 + 3 * d + 0];
-      s_ja[1][t] = cv[gnode * 9 + 3 * d + 1];
-      s_ja[2][t] = cv[gnode * 9 + 3 * d + 2];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) s_ja[c][t] = cv[((size_t)e * 9 + 3 * d + c) * N3 + t];
     }
     const int stride = d == 0 ? 1 : (d == 1 ? N : N2);
     const int own_d = d == 0 ? ti : (d == 1 ? tj : tk);
@@ -816,11 +827,11 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
   __syncthreads();
   double un[6];
   if (active)
-    stage_epilogue<N, T, KAHAN>(acc, acc_nc, s_fl, ti, tj, tk, gnode, u, out, kreg, invJ, mode,
+    stage_epilogue<N, T, KAHAN>(acc, acc_nc, s_fl, ti, tj, tk, e, gnode, u, out, kreg, invJ, mode,
                                 rk_a, res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
   if (res.speed_partial) {
     __shared__ double s_red[B / 64][3];
-    element_speed<B>(q, active, un, res.cv64, invJ, gnode, t, e, 1, s_red, res.speed_partial);
+    element_speed<N>(q, active, un, res.cv64, invJ, gnode, t, e, 1, s_red, res.speed_partial);
   }
 }
 
@@ -879,7 +890,7 @@ void e3_stage_direct(
   if (active) {
     node_fields_to_lds<N, VOL, NC, T>(q, u, gnode, tl, s_w, s_phi, s_pb, bg);
 #pragma unroll
-    for (int c = 0; c < 9; ++c) s_buf[c * N3 + tl] = T(cv[gnode * 9 + c]);
+    for (int c = 0; c < 9; ++c) s_buf[c * N3 + tl] = T(cv[((size_t)e * 9 + c) * N3 + tl]);
   }
   FacePrefetch<N, EPB> pf;
   face_prefetch<N, EPB>(pf, e0, n_valid, t, u, nbr, face_info);
@@ -1022,11 +1033,11 @@ void e3_stage_direct(
   __syncthreads();
   double un[6];
   if (active)
-    stage_epilogue<N, T, KAHAN>(acc, acc_nc, s_buf, ti, tj, tk, gnode, u, out, kreg, invJ, mode,
+    stage_epilogue<N, T, KAHAN>(acc, acc_nc, s_buf, ti, tj, tk, e, gnode, u, out, kreg, invJ, mode,
                                 rk_a, res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
   if (res.speed_partial) {
     __shared__ double s_red[EPB * BE / 64][3];
-    element_speed<BE, EPB>(q, active, un, res.cv64, invJ, gnode, t, e0, n_valid, s_red,
+    element_speed<N, EPB>(q, active, un, res.cv64, invJ, gnode, t, e0, n_valid, s_red,
                            res.speed_partial);
   }
 }
