@@ -309,9 +309,9 @@ int atmo_swe_create(const atmo_swe_config* config, const atmo_geometry2d* geomet
 /* Autotuner of the stage kernels (no counterpart in the reference): times
  * every workgroup shape on the resident state (as an RK stage) and keeps the
  * fastest; `ms` (may be NULL, else room for ATMO_SWE_VARIANTS values)
- * receives the time of each shape.  Covariant form: 1, 2 or 4 waves per
- * workgroup, each with a full or a persistent grid (ATMO_SWE_VARIANTS
- * shapes).  3D Euler: one or two elements per workgroup (variants 0 and 1;
+ * receives the time of each shape.  Covariant form: node lanes of 1, 2
+ * or 4 waves per workgroup that do all the work (0..2) or share it with two
+ * more sets of waves (3..5; ATMO_SWE_VARIANTS shapes).  3D Euler: one or two elements per workgroup (variants 0 and 1;
  * the second is built for polydeg 3 and 4 of the direct volume form, elsewhere
  * variant 0 is the only shape and its time is reported as 0).  atmo_step and
  * atmo_solve tune by themselves on their first call; every shape gives

@@ -7,22 +7,41 @@
 // the 14 auxiliary rows it needs plus z / r (Trixi's node-major aux rows span
 // 208 bytes, so reading a few of them fetches the whole row), and one 2 x 2
 // basis map per face node instead of the 12 basis entries of both sides.
-// A workgroup of 64, 128 or 256 lanes holds EPB = lanes / n^2
-// elements (one lane per node); the per-node fields the two-point fluxes need
-// (state, velocity v = hv / h and covariant velocity G v formed once per node,
-// J, G, G^-1, h_s) are staged in LDS.  Volume terms are gathered per node:
-// sum_m Dsplit[own, m] (f#(own, m) + g(own, m) / 2) along both directions (the
-// symmetric f# is evaluated for each ordering, the nonconservative g is
-// non-symmetric anyway).  Face nodes are
-// then mapped to lanes: each element evaluates the interface flux of its own
+// A group of EPB elements has one lane per node (64, 128 or 256 lanes); the
+// per-node fields the fluxes need (state, velocity v = hv / h, covariant
+// velocity G v, J, G^-1, h_s, each formed once per node) are staged in LDS.
+// Volume terms are gathered per node: sum_m Dsplit[own, m] (f#(own, m) +
+// g(own, m) / 2) along both directions (the symmetric f# is evaluated for each
+// ordering, the nonconservative g is non-symmetric anyway).  Every face node
+// has a lane too: each element evaluates the interface flux of its own
 // faces in its own contravariant basis with its own auxiliary variables,
 // exactly as the reference does for each side
 // (src/solvers/dgsem_p4est/dg_2d_manifold_in_3d_covariant.jl:301-432), lifts it
 // with 1/w_end, and every node adds its face terms, applies -1/J and the
 // geometric + Coriolis source, and stores du or applies the 2N RK update
 // (per-element time step: ensemble members step with their own dt).
+//
+// Two forms of a group: the node lanes do all of it one after the other, or
+// (SPLIT) three sets of waves share it: the node lanes take the volume terms
+// of the first direction, a second set those of the second direction and a
+// third set the face nodes, whose neighbour states are on their way from the
+// start.  Both add the same sums in the same order, with every fused
+// multiply-add written out (left to itself the compiler contracts each form
+// its own way), so they give the same bits.
+//
+// What bounds it, and what each form is for (MI355X, microseconds per stage;
+// in brackets the form before, whose volume loop took about twice the
+// operations per pair, whose register reads waited for the stores before
+// them and whose neighbour reads began after the volume terms): a small mesh
+// is one chain of dependent operations per wave, so the split form, whose
+// chain is shorter, wins (polydeg 3, 2,400 nodes: 3.9 split, 5.5 not [5.6];
+// polydeg 4, 25,350 nodes: 4.7, 6.3 [7.4]); a full chip is bound by HBM, so
+// the plain form, which needs fewer waves per node, wins (polydeg 3, 1.87 M
+// nodes, 396 MB: 65.9 = 6.0 TB/s; split 71.7 [88.1]).  Between them (98,304
+// nodes: 6.5 split, 6.9 plain [7.8]) the autotuner decides.
 #include <hip/hip_runtime.h>
 
+#include "euler3d_physics.hpp"
 #include "swe_kernels.hpp"
 #include "speed_max.hpp"
 
@@ -32,197 +51,104 @@ namespace {
 
 constexpr int NV = 3, NA = 26;
 
-struct AuxV {
-  const double* a;  // 26 entries with stride `s`
-  int s;
-  __device__ __forceinline__ double at(int k) const { return a[k * s]; }
-  __device__ __forceinline__ double A(int r, int c) const { return at(r + 3 * c); }
-  __device__ __forceinline__ double B(int r, int c) const { return at(6 + r + 2 * c); }
-  __device__ __forceinline__ double J() const { return at(12); }
-  __device__ __forceinline__ double Gcov(int i, int j) const {
-    return (i == 0 && j == 0) ? at(13) : (i == 1 && j == 1) ? at(15) : at(14);
-  }
-  __device__ __forceinline__ double Gcon(int i, int j) const {
-    return (i == 0 && j == 0) ? at(16) : (i == 1 && j == 1) ? at(18) : at(17);
-  }
-  __device__ __forceinline__ double hs() const { return at(19); }
-  __device__ __forceinline__ double Gam(int k, int i, int j) const {
-    const int o = 20 + 3 * k;
-    return (i == 0 && j == 0) ? at(o) : (i == 1 && j == 1) ? at(o + 2) : at(o + 1);
-  }
-};
-
-// covariant_shallow_water_split.jl:66-80
-__device__ __forceinline__ void flux_split(const double* u, const AuxV& x, int o, double* f) {
-  const double mass = x.J() * u[1 + o];
-  f[0] = mass;
-  f[1] = mass * (u[1] / u[0]);
-  f[2] = mass * (u[2] / u[0]);
+// quotients a / h and b / h from one refined reciprocal (each within one unit
+// in the last place of the IEEE quotient, as div_nr)
+__device__ __forceinline__ void div2(double a, double b, double h, double& qa, double& qb) {
+  const double r = rcp_refined(h);
+  qa = a * r;
+  qb = b * r;
+  qa = fma(fma(-h, qa, a), r, qa);
+  qb = fma(fma(-h, qb, b), r, qb);
 }
 
-// :100-122 flux_ec
-__device__ __forceinline__ void flux_ec(const double* ul, const double* ur, const AuxV& xl,
-                                        const AuxV& xr, int o, double* f) {
-  const double mass = 0.5 * (xl.J() * ul[1 + o] + xr.J() * ur[1 + o]);
-  f[0] = mass;
-  f[1] = 0.5 * (ul[1] / ul[0] + ur[1] / ur[0]) * mass;
-  f[2] = 0.5 * (ul[2] / ul[0] + ur[2] / ur[0]) * mass;
-}
-
-__device__ __forceinline__ void flux_central(const double* ul, const double* ur, const AuxV& xl,
-                                             const AuxV& xr, int o, double* f) {
-  double fl[NV], fr[NV];
-  flux_split(ul, xl, o, fl);
-  flux_split(ur, xr, o, fr);
-#pragma unroll
-  for (int v = 0; v < NV; ++v) f[v] = 0.5 * (fl[v] + fr[v]);
-}
-
-// :157-187 flux_nonconservative_ec
-__device__ __forceinline__ void noncons_ec(double g, const double* ul, const double* ur,
-                                           const AuxV& xl, const AuxV& xr, int o, double* f) {
-  const double hl = ul[0], hr = ur[0];
-  const double vr0 = ur[1] / hr, vr1 = ur[2] / hr;
-  const double vc0 = xr.Gcov(0, 0) * vr0 + xr.Gcov(0, 1) * vr1;
-  const double vc1 = xr.Gcov(1, 0) * vr0 + xr.Gcov(1, 1) * vr1;
-  const double hs_jump = xr.hs() - xl.hs();
-  const double geo0 = 0.5 * ul[1 + o] * ((xl.Gcon(0, 0) * vc0 + xl.Gcon(0, 1) * vc1) - vr0);
-  const double geo1 = 0.5 * ul[1 + o] * ((xl.Gcon(1, 0) * vc0 + xl.Gcon(1, 1) * vc1) - vr1);
-  const double pr0 = g * xl.Gcon(0, o) * hl * (hr + hs_jump);
-  const double pr1 = g * xl.Gcon(1, o) * hl * (hr + hs_jump);
-  f[0] = 0.0;
-  f[1] = xl.J() * (geo0 + pr0);
-  f[2] = xl.J() * (geo1 + pr1);
-}
-
-__device__ __forceinline__ double max_abs_speed(double g, const double* ul, const double* ur,
-                                                const AuxV& xl, const AuxV& xr, int o) {
-  return fmax(fabs(ul[1 + o] / ul[0]) + sqrt(xl.Gcon(o, o) * ul[0] * g),
-              fabs(ur[1 + o] / ur[0]) + sqrt(xr.Gcon(o, o) * ur[0] * g));
+// J = sqrt(det G) and G^-1 = adj(G) / det G from the covariant metric tensor
+// (metric_from_gcov with the shorter quotient and root of euler3d_physics.hpp);
+// every kernel takes them from here, so each use gets the same bits
+__device__ __forceinline__ void metric_of(double g11, double g12, double g22, double& J,
+                                          double& c11, double& c12, double& c22) {
+#pragma clang fp contract(off)
+  const double det = fma(g11, g22, -(g12 * g12));
+  const double inv = div_nr(1.0, det);
+  J = sqrt_(det);
+  c11 = g22 * inv;
+  c12 = -g12 * inv;
+  c22 = g11 * inv;
 }
 
 // CovariantShallowWaterEquations2D, the standard form (covariant_shallow_water.jl:166-187):
 // contravariant flux in orientation o with the pressure term G^{io} g h^2 / 2
 __device__ __forceinline__ void flux_standard(double g, double h, double hv1, double hv2,
                                               double J, double Gi_0o, double Gi_1o, double hvo,
-                                              double* f) {
-  const double vcon = hvo / h;
+                                              double vo, double* f) {
+#pragma clang fp contract(off)
   const double grav = 0.5 * g * h * h;
   f[0] = J * hvo;
-  f[1] = J * (hv1 * vcon + Gi_0o * grav);
-  f[2] = J * (hv2 * vcon + Gi_1o * grav);
+  f[1] = J * fma(hv1, vo, Gi_0o * grav);
+  f[2] = J * fma(hv2, vo, Gi_1o * grav);
 }
 
-__device__ __forceinline__ void flux_standard(double g, const double* u, const AuxV& x, int o,
-                                              double* f) {
-  flux_standard(g, u[0], u[1], u[2], x.J(), x.Gcon(0, o), x.Gcon(1, o), u[1 + o], f);
+// what the node-local source reads of one node
+struct SourceIn {
+  double h, hv[2], v[2], vc[2];  // vc: covariant velocity G v
+  double J, c11, c12, c22, sin_lat;
+  double gam[6];  // Gamma^1_11, _12, _22, Gamma^2_11, _12, _22
+};
+
+// the Coriolis term 2 omega sin(lat) J (G^{k2} h v^1 - G^{k1} h v^2)
+__device__ __forceinline__ double coriolis(double fJ, double ck1, double ck2, const double* hv) {
+#pragma clang fp contract(off)
+  return fJ * fma(ck2, hv[0], -(ck1 * hv[1]));
 }
 
-// source_terms_geometric_coriolis of the standard form (:215-238)
-__device__ __forceinline__ void source_standard(double g, double omega, const double* u,
-                                                double sin_lat, const AuxV& a, double* s) {
-  const double h = u[0], hv[2] = {u[1], u[2]};
-  const double v[2] = {u[1] / h, u[2] / h};
-  const double grav = 0.5 * g * h * h;
-  double tau[2][2];  // h v^i v^j + G^{ij} g h^2 / 2
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) tau[i][j] = hv[i] * v[j] + grav * a.Gcon(i, j);
-  const double f = 2 * omega * sin_lat;
-  double src[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    double sg = 0.0;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) sg += a.Gam(k, i, j) * tau[i][j];
-    src[k] = sg + f * a.J() * (a.Gcon(k, 1) * hv[0] - a.Gcon(k, 0) * hv[1]);
-  }
+// source_terms_geometric_coriolis of the standard form (covariant_shallow_water.jl:215-238)
+__device__ __forceinline__ void source_standard(double g, double omega, const SourceIn& a,
+                                                double* s) {
+#pragma clang fp contract(off)
+  const double grav = 0.5 * g * a.h * a.h;
+  // tau^{ij} = h v^i v^j + G^{ij} g h^2 / 2 (symmetric)
+  const double t11 = fma(a.hv[0], a.v[0], grav * a.c11);
+  const double t12 = fma(a.hv[0], a.v[1], grav * a.c12);
+  const double t22 = fma(a.hv[1], a.v[1], grav * a.c22);
+  const double fJ = 2 * omega * a.sin_lat * a.J;
   s[0] = 0.0;
-  s[1] = -src[0];
-  s[2] = -src[1];
+  s[1] = -(fma(a.gam[0], t11, fma(2.0 * a.gam[1], t12, a.gam[2] * t22)) +
+           coriolis(fJ, a.c11, a.c12, a.hv));
+  s[2] = -(fma(a.gam[3], t11, fma(2.0 * a.gam[4], t12, a.gam[5] * t22)) +
+           coriolis(fJ, a.c12, a.c22, a.hv));
 }
 
-// surface flux (u_ll, u_rr, aux, aux) + 1/2 the nonconservative surface term
-__device__ __forceinline__ void surface_terms(const SweLaunch& L, const double* ul,
-                                              const double* ur, const AuxV& x, int o,
-                                              double* f) {
-  if (L.surface_flux == 3) {
-    // flux_lax_friedrichs of the standard form: flux_central of the standard
-    // flux plus the local Lax-Friedrichs dissipation; no nonconservative term
-    double fl[NV], fr[NV];
-    flux_standard(L.gravity, ul, x, o, fl);
-    flux_standard(L.gravity, ur, x, o, fr);
-    const double lam = max_abs_speed(L.gravity, ul, ur, x, x, o);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) f[v] = 0.5 * (fl[v] + fr[v]) + -0.5 * x.J() * lam * (ur[v] - ul[v]);
-    return;
-  }
-  if (L.surface_flux == 1) flux_central(ul, ur, x, x, o, f);
-  else flux_ec(ul, ur, x, x, o, f);
-  if (L.surface_flux != 2) {  // DissipationLocalLaxFriedrichs, equations.jl:283-290
-    const double lam = max_abs_speed(L.gravity, ul, ur, x, x, o);
-#pragma unroll
-    for (int v = 0; v < NV; ++v) f[v] += -0.5 * x.J() * lam * (ur[v] - ul[v]);
-  }
-  double g[NV];
-  if (L.surface_noncons == 0) {  // flux_nonconservative_surface_simplified, :229-250
-    g[0] = 0.0;
-    g[1] = x.J() * (L.gravity * x.Gcon(0, o) * ul[0] * ur[0]);
-    g[2] = x.J() * (L.gravity * x.Gcon(1, o) * ul[0] * ur[0]);
-  } else {
-    noncons_ec(L.gravity, ul, ur, x, x, o, g);
-  }
-#pragma unroll
-  for (int v = 0; v < NV; ++v) f[v] += 0.5 * g[v];
-}
-
-// covariant_shallow_water_split.jl:273-302 (sin_lat = z / r of the node)
-__device__ __forceinline__ void source_split(double omega, const double* u, double sin_lat,
-                                             const AuxV& a, double* s) {
-  const double hv0 = u[1], hv1 = u[2];
-  const double v0 = u[1] / u[0], v1 = u[2] / u[0];
-  const double hvv[2][2] = {{hv0 * v0, hv0 * v1}, {hv1 * v0, hv1 * v1}};
-  double hcv[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) hcv[i][j] = a.Gcov(i, 0) * hvv[0][j] + a.Gcov(i, 1) * hvv[1][j];
-  const double f = 2 * omega * sin_lat;
-  double t1[2], t2[2];
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    t1[k] = a.Gam(k, 0, 0) * hvv[0][0] + a.Gam(k, 1, 0) * hvv[1][0] + a.Gam(k, 0, 1) * hvv[0][1] +
-            a.Gam(k, 1, 1) * hvv[1][1];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-    t2[i] = a.Gam(0, i, 0) * hcv[0][0] + a.Gam(0, i, 1) * hcv[0][1] + a.Gam(1, i, 0) * hcv[1][0] +
-            a.Gam(1, i, 1) * hcv[1][1];
-  const double sg0 = 0.5 * (t1[0] - (a.Gcon(0, 0) * t2[0] + a.Gcon(0, 1) * t2[1]));
-  const double sg1 = 0.5 * (t1[1] - (a.Gcon(1, 0) * t2[0] + a.Gcon(1, 1) * t2[1]));
+// covariant_shallow_water_split.jl:273-302.  The reference's G_{ia} h v^a v^j
+// is the covariant velocity times h v^j.
+__device__ __forceinline__ void source_split(double omega, const SourceIn& a, double* s) {
+#pragma clang fp contract(off)
+  const double w11 = a.hv[0] * a.v[0], w12 = a.hv[0] * a.v[1], w22 = a.hv[1] * a.v[1];
+  const double m00 = a.vc[0] * a.hv[0], m01 = a.vc[0] * a.hv[1];
+  const double m10 = a.vc[1] * a.hv[0], m11 = a.vc[1] * a.hv[1];
+  const double t1 = fma(a.gam[0], w11, fma(2.0 * a.gam[1], w12, a.gam[2] * w22));
+  const double t2 = fma(a.gam[3], w11, fma(2.0 * a.gam[4], w12, a.gam[5] * w22));
+  const double r1 = fma(a.gam[0], m00, a.gam[1] * m01) + fma(a.gam[3], m10, a.gam[4] * m11);
+  const double r2 = fma(a.gam[1], m00, a.gam[2] * m01) + fma(a.gam[4], m10, a.gam[5] * m11);
+  const double fJ = 2 * omega * a.sin_lat * a.J;
   s[0] = 0.0;
-  s[1] = -(sg0 + f * a.J() * (a.Gcon(0, 1) * hv0 - a.Gcon(0, 0) * hv1));
-  s[2] = -(sg1 + f * a.J() * (a.Gcon(1, 1) * hv0 - a.Gcon(1, 0) * hv1));
+  s[1] = -fma(0.5, t1 - fma(a.c11, r1, a.c12 * r2), coriolis(fJ, a.c11, a.c12, a.hv));
+  s[2] = -fma(0.5, t2 - fma(a.c12, r1, a.c22 * r2), coriolis(fJ, a.c12, a.c22, a.hv));
 }
 
-// Workgroup shape: WAVES waves of 64 lanes, one lane per node, EPB = WAVES *
-// 64 / n^2 elements (n^2 <= 64); with PERSIST the grid is capped and every
-// workgroup loops over element groups with a grid stride.
+// Group of elements: WAVES waves of 64 lanes with one lane per node hold EPB =
+// WAVES * 64 / n^2 elements (n^2 <= 64)
 template <int N, int WAVES>
 struct SweShape {
   static constexpr int N2 = N * N;
-  static constexpr int BLOCK = 64 * WAVES;
-  static constexpr int EPB = BLOCK / N2;
+  static constexpr int LANES = 64 * WAVES;
+  static constexpr int EPB = LANES / N2;
   static constexpr int NF = 4 * N;  // face nodes per element
+  // passes of the face nodes over the group's lanes
+  static constexpr int PASSES = (EPB * NF + LANES - 1) / LANES;
 };
 
-// per-node fields staged in LDS: h, hv^1, hv^2, v^1, v^2 (v = hv / h), J,
-// G_11, G_12, G_22, G^11, G^12, G^22, h_s (13 doubles per node: with the
-// face buffer 8 KB per wave at polydeg 3, which leaves room for five waves
-// per SIMD)
-constexpr int kSweFields = 13;
+// per-node fields staged in LDS: h, hv^1, hv^2, v^1, v^2 (v = hv / h), J, the
+// covariant velocity (G v)_1, (G v)_2, G^11, G^12, G^22, h_s
+constexpr int kSweFields = 12;
 
 // the stage's geometry rows and face maps in their storage type GT (double, or
 // float under ATMO_PREC_FP32_GEOMETRY); a float operand widens to double in
@@ -236,6 +162,159 @@ __device__ __forceinline__ const GT* face_maps(const SweLaunch& L) {
   if constexpr (sizeof(GT) == 4) return L.fxf32; else return L.fxf;
 }
 
+// a face node's inputs from memory: the neighbour's state and the map of its
+// momentum into the own basis
+template <typename GT>
+struct FaceIn {
+  double u[NV];
+  GT M[4];
+};
+
+template <int N, int WAVES, typename GT>
+__device__ __forceinline__ bool face_load(const SweLaunch& L, int e0, int fid, FaceIn<GT>& x) {
+  using S = SweShape<N, WAVES>;
+  const int fe = fid / S::NF;
+  if (fid >= S::EPB * S::NF || e0 + fe >= L.n_elements) return false;
+  const size_t fnode = (size_t)e0 * S::NF + fid;
+  const GT* M = face_maps<GT>(L) + fnode * 4;
+  const int link = L.nbr[fnode];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) x.M[c] = M[c];
+  const double* ur = L.u + (size_t)link * NV;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) x.u[v] = ur[v];
+  return true;
+}
+
+// surface flux plus half the nonconservative surface term of one face node,
+// lifted by 1/w_end.  All of it is symmetric in the two states but for the
+// dissipation: on a face whose outward normal points along -x_o both parts
+// change sign and order, f*(own, nbr) for one side is
+//   s (f#(own, nbr) + g / 2) - J lam (nbr - own) / 2,   s = +1 or -1.
+// With one set of auxiliary variables on both sides the jump of h_s and the
+// curvature part G^-1 G v - v of flux_nonconservative_ec vanish (:157-187),
+// which leaves flux_nonconservative_surface_simplified (:229-250).
+template <int N, typename GT>
+__device__ __forceinline__ void face_flux(const SweLaunch& L, const double (*n)[N * N], int r,
+                                          const FaceIn<GT>& x, double* fs) {
+#pragma clang fp contract(off)
+  const int f = r / N, k = r - f * N, o = f >> 1;
+  const int i = f == 0 ? 0 : (f == 1 ? N - 1 : k);
+  const int j = f == 2 ? 0 : (f == 3 ? N - 1 : k);
+  const int q = i + N * j;
+  const double sgn = (f & 1) ? 1.0 : -1.0;
+  const double h = n[0][q], hv[2] = {n[1][q], n[2][q]}, v[2] = {n[3][q], n[4][q]};
+  const double J = n[5][q], c1o = n[8 + o][q], c2o = n[9 + o][q], coo = n[8 + 2 * o][q];
+  const double hvo = n[1 + o][q], vo = n[3 + o][q];
+  // neighbour state in this element's contravariant basis (contravariant2global,
+  // then global2contravariant: covariant_shallow_water.jl:140-153)
+  const double ht = x.u[0];
+  const double t1 = fma(x.M[0], x.u[1], x.M[1] * x.u[2]);
+  const double t2 = fma(x.M[2], x.u[1], x.M[3] * x.u[2]);
+  double vt1, vt2;
+  div2(t1, t2, ht, vt1, vt2);
+  const double to = o ? t2 : t1, vto = o ? vt2 : vt1;
+  double F[NV];
+  if (L.surface_flux == 3) {
+    // flux_central of the standard form; no nonconservative term
+    double fl[NV], fr[NV];
+    flux_standard(L.gravity, h, hv[0], hv[1], J, c1o, c2o, hvo, vo, fl);
+    flux_standard(L.gravity, ht, t1, t2, J, c1o, c2o, to, vto, fr);
+#pragma unroll
+    for (int c = 0; c < NV; ++c) F[c] = 0.5 * (fl[c] + fr[c]);
+  } else {
+    const double half_J = 0.5 * J;
+    const double m = half_J * (hvo + to);
+    F[0] = m;
+    if (L.surface_flux == 1) {  // flux_central of the split flux (:66-80)
+      F[1] = half_J * fma(hvo, v[0], to * vt1);
+      F[2] = half_J * fma(hvo, v[1], to * vt2);
+    } else {  // flux_ec (:100-122)
+      F[1] = 0.5 * (v[0] + vt1) * m;
+      F[2] = 0.5 * (v[1] + vt2) * m;
+    }
+    const double pr = half_J * (L.gravity * h * ht);
+    F[1] = fma(pr, c1o, F[1]);
+    F[2] = fma(pr, c2o, F[2]);
+  }
+#pragma unroll
+  for (int c = 0; c < NV; ++c) F[c] *= sgn;
+  if (L.surface_flux != 2) {  // DissipationLocalLaxFriedrichs, equations.jl:283-290
+    const double gc = L.gravity * coo;
+    const double lam = fmax(fabs(vo) + sqrt_(gc * h), fabs(vto) + sqrt_(gc * ht));
+    const double d = -0.5 * J * lam;
+    F[0] = fma(d, ht - h, F[0]);
+    F[1] = fma(d, t1 - hv[0], F[1]);
+    F[2] = fma(d, t2 - hv[1], F[2]);
+  }
+#pragma unroll
+  for (int c = 0; c < NV; ++c) fs[c] = F[c] * L.inv_w;
+}
+
+// volume terms of node q along direction o: the sums over the partners in
+// rotated order own + 1, ..., own + n - 1 (mod n), so every lane has a partner
+// in each step.  Split form: with m = J hv^o of the two nodes, 4 times the term
+// is (f#_h: 2 (m_l + m_r)), (v_l + v_r) (m_l + m_r) + m_l ((G^-1 (G v)_r) - v_r)
+// + 2 g J h G^{.o} (h_r + h_s,r - h_s,l); the powers of two are applied to the
+// sums, which rounds as applying them to each term.
+template <int N, int UNROLL>
+__device__ __forceinline__ void volume_terms(const SweLaunch& L, const double (*n)[N * N],
+                                             const double* s_ds, int q, int o, double* sum) {
+#pragma clang fp contract(off)
+  const int ti = q % N, tj = q / N;
+  const int own = o == 0 ? ti : tj, stride = o == 0 ? 1 : N;
+  sum[0] = sum[1] = sum[2] = 0.0;
+  if (L.volume_flux == 2) {
+    // weak form (dg_2d_manifold_in_3d_covariant.jl:100-130): derivative_hat of
+    // the standard flux, evaluated in place for every node of the line
+    const int base = q - own * stride;
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+      const int p = base + m * stride;
+      double f[NV];
+      flux_standard(L.gravity, n[0][p], n[1][p], n[2][p], n[5][p], n[8 + o][p], n[9 + o][p],
+                    n[1 + o][p], n[3 + o][p], f);
+      const double d = s_ds[own * N + m];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) sum[v] = fma(d, f[v], sum[v]);
+    }
+    return;
+  }
+  const double hl = n[0][q], vl0 = n[3][q], vl1 = n[4][q], Jl = n[5][q], hsl = n[11][q];
+  const double c11 = n[8][q], c12 = n[9][q], c22 = n[10][q];
+  const double ml = Jl * n[1 + o][q];
+  const double pf = 2.0 * L.gravity * Jl * hl;
+  const double p0 = pf * (o == 0 ? c11 : c12), p1 = pf * (o == 0 ? c12 : c22);
+  const bool ec = L.volume_flux == 0;
+#pragma unroll UNROLL
+  for (int j = 1; j < N; ++j) {
+    const int step = own + j >= N ? j - N : j;
+    const int p = q + step * stride;
+    const double vr0 = n[3][p], vr1 = n[4][p], vc0 = n[6][p], vc1 = n[7][p];
+    const double mr = n[5][p] * n[1 + o][p];
+    const double ms = ml + mr;
+    const double hh = n[0][p] + (n[11][p] - hsl);
+    double a0, a1;
+    if (ec) {  // flux_ec (:100-122)
+      a0 = (vl0 + vr0) * ms;
+      a1 = (vl1 + vr1) * ms;
+    } else {  // flux_central of the split flux (:66-80)
+      a0 = 2.0 * fma(ml, vl0, mr * vr0);
+      a1 = 2.0 * fma(ml, vl1, mr * vr1);
+    }
+    // flux_nonconservative_ec (:157-187) of (own, partner)
+    a0 += fma(ml, fma(c11, vc0, c12 * vc1) - vr0, p0 * hh);
+    a1 += fma(ml, fma(c12, vc0, c22 * vc1) - vr1, p1 * hh);
+    const double ds = s_ds[own * (N + 1) + step];
+    sum[0] = fma(ds, ms, sum[0]);
+    sum[1] = fma(ds, a0, sum[1]);
+    sum[2] = fma(ds, a1, sum[2]);
+  }
+  sum[0] *= 0.5;
+  sum[1] *= 0.25;
+  sum[2] *= 0.25;
+}
+
 }  // namespace
 
 // StepsizeCallback's scaled wave speeds at one node (stepsize_dg2d.jl:47-71):
@@ -243,261 +322,204 @@ __device__ __forceinline__ const GT* face_maps(const SweLaunch& L) {
 // resident step both call this one function, so their speeds agree bit for bit
 __device__ __forceinline__ void swe_node_speeds(const double* u, double gcon11, double gcon22,
                                                 double gravity, double l[2]) {
-  l[0] = fabs(u[1] / u[0]) + sqrt(gcon11 * u[0] * gravity);
-  l[1] = fabs(u[2] / u[0]) + sqrt(gcon22 * u[0] * gravity);
+#pragma clang fp contract(off)
+  double v1, v2;
+  div2(u[1], u[2], u[0], v1, v2);
+  l[0] = fabs(v1) + sqrt_(gcon11 * u[0] * gravity);
+  l[1] = fabs(v2) + sqrt_(gcon22 * u[0] * gravity);
 }
 
 // SPEED: the RK stage also writes L.speed_partial (the last stage of a
 // resident step); a variant of its own, so the other stages keep their
 // register budget
-// polydeg 3 fits five waves per SIMD (90-92 VGPRs, 8 KB of LDS per wave, no
-// spills); the other degrees keep the compiler's register choice (a five-wave
-// budget spills there)
-template <int N, int WAVES, bool PERSIST, bool SPEED, typename GT>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(N == 4 ? 5 : 1)))
+template <int N, int WAVES, bool SPLIT, bool SPEED, typename GT>
+__global__ __launch_bounds__((SPLIT ? 3 : 1) * 64 * WAVES)
+__attribute__((amdgpu_waves_per_eu(N == 4 && !SPLIT ? 5 : 1)))
 void swe_stage(SweLaunch L) {
+#pragma clang fp contract(off)
   using S = SweShape<N, WAVES>;
-  constexpr int N2 = S::N2, EPB = S::EPB, B = S::BLOCK;
+  constexpr int N2 = S::N2, EPB = S::EPB, B = S::LANES;
+  constexpr int UNROLL = SPLIT && N <= 5 ? N : 1;
   __shared__ double s_n[EPB][kSweFields][N2];
   __shared__ double s_sf[EPB][NV][S::NF];
+  __shared__ double s_d1[SPLIT ? EPB : 1][NV][N2];  // the second direction's volume terms
+  __shared__ double s_ds[N2];
 
-  const int t = threadIdx.x;
+  const int role = SPLIT ? __builtin_amdgcn_readfirstlane(threadIdx.x / B) : 0;
+  const bool node_role = role == 0, dir1_role = !SPLIT || role == 1, face_role = !SPLIT || role == 2;
+  const int t = threadIdx.x - role * B;
+  const int e0 = blockIdx.x * EPB;
   const int es = t / N2, q = t - es * N2;
   const int ti = q % N, tj = q / N;
-  const int groups = (L.n_elements + EPB - 1) / EPB;
-  for (int grp = blockIdx.x; grp < groups; grp += PERSIST ? gridDim.x : groups) {
-    const int e0 = grp * EPB;
-    const int e = e0 + es;
-    const bool active = es < EPB && e < L.n_elements;
-    if (PERSIST) __syncthreads();  // the previous group's LDS reads are done
-    if (active) {
-      const size_t g = (size_t)e * N2 + q;
-      const double* un = L.u + g * NV;
-      const GT* gg = geo_rows<GT>(L) + g;
-      const long long NN = L.n_nodes;
-      const double h = un[0], hv1 = un[1], hv2 = un[2];
-      const double v1 = hv1 / h, v2 = hv2 / h;
-      const double G11 = gg[0], G12 = gg[NN], G22 = gg[2 * NN];
-      double J, c11, c12, c22;
-      metric_from_gcov(G11, G12, G22, J, c11, c12, c22);
-      // FP32 storage: J is the stored area element rounded once; it is the
-      // same number on both sides of a face (G is not: it is expressed in each
-      // element's own basis), so the two mass fluxes there agree
-      if constexpr (sizeof(GT) == 4) J = gg[11 * NN];
-      s_n[es][0][q] = h;
-      s_n[es][1][q] = hv1;
-      s_n[es][2][q] = hv2;
-      s_n[es][3][q] = v1;
-      s_n[es][4][q] = v2;
-      s_n[es][5][q] = J;
-      s_n[es][6][q] = G11;
-      s_n[es][7][q] = G12;
-      s_n[es][8][q] = G22;
-      s_n[es][9][q] = c11;
-      s_n[es][10][q] = c12;
-      s_n[es][11][q] = c22;
-      if constexpr (sizeof(GT) == 4) s_n[es][12][q] = L.topography ? L.hs64[g] : 0.0;
-      else s_n[es][12][q] = L.topography ? gg[3 * NN] : 0.0;
-    }
-    __syncthreads();
+  const int e = e0 + es;
+  const bool active = es < EPB && e < L.n_elements;
+  const size_t g = (size_t)e * N2 + q;
+  const long long NN = L.n_nodes;
 
-    double du[NV] = {0, 0, 0};
-    if (active && L.volume_flux == 2) {
-      // weak form (dg_2d_manifold_in_3d_covariant.jl:100-130): node (i, j)
-      // gathers derivative_hat[i, m] F^1(m, j) + derivative_hat[j, m] F^2(i, m),
-      // the standard flux of every node on its two lines evaluated in place
+  // the first pass's neighbour states are loaded before anything else is waited for
+  FaceIn<GT> fin;
+  bool has_face = false;
+  if (face_role) has_face = face_load<N, WAVES, GT>(L, e0, t, fin);
+  if (dir1_role && t < N2) s_ds[t] = L.volume_flux == 2 ? L.dhat[t] : L.dsplit[t];
+  if (node_role && active) {
+    const double* un = L.u + g * NV;
+    const GT* gg = geo_rows<GT>(L) + g;
+    const double h = un[0], hv1 = un[1], hv2 = un[2];
+    const double G11 = gg[0], G12 = gg[NN], G22 = gg[2 * NN];
+    double hs = 0.0;
+    if (L.topography) {
+      if constexpr (sizeof(GT) == 4) hs = L.hs64[g];
+      else hs = gg[3 * NN];
+    }
+    double v1, v2, J, c11, c12, c22;
+    div2(hv1, hv2, h, v1, v2);
+    metric_of(G11, G12, G22, J, c11, c12, c22);
+    // FP32 storage: J is the stored area element rounded once; it is the
+    // same number on both sides of a face (G is not: it is expressed in each
+    // element's own basis), so the two mass fluxes there agree
+    if constexpr (sizeof(GT) == 4) J = gg[11 * NN];
+    s_n[es][0][q] = h;
+    s_n[es][1][q] = hv1;
+    s_n[es][2][q] = hv2;
+    s_n[es][3][q] = v1;
+    s_n[es][4][q] = v2;
+    s_n[es][5][q] = J;
+    s_n[es][6][q] = fma(G11, v1, G12 * v2);
+    s_n[es][7][q] = fma(G12, v1, G22 * v2);
+    s_n[es][8][q] = c11;
+    s_n[es][9][q] = c12;
+    s_n[es][10][q] = c22;
+    s_n[es][11][q] = hs;
+  }
+  // the node's remaining inputs: source geometry, register, step size
+  SourceIn src;
+  double kreg[NV], dt = L.rk_dt;
+  auto load_rest = [&]() {
+    if (L.source_terms) {
+      const GT* gg = geo_rows<GT>(L) + g;
 #pragma unroll
-      for (int m = 0; m < N; ++m) {
-        const int p1 = m + N * tj, p2 = ti + N * m;
-        double f1[NV], f2[NV];
-        flux_standard(L.gravity, s_n[es][0][p1], s_n[es][1][p1], s_n[es][2][p1], s_n[es][5][p1],
-                      s_n[es][9][p1], s_n[es][10][p1], s_n[es][1][p1], f1);
-        flux_standard(L.gravity, s_n[es][0][p2], s_n[es][1][p2], s_n[es][2][p2], s_n[es][5][p2],
-                      s_n[es][10][p2], s_n[es][11][p2], s_n[es][2][p2], f2);
-        const double d1 = L.dhat[ti * N + m], d2 = L.dhat[tj * N + m];
+      for (int c = 0; c < 6; ++c) src.gam[c] = gg[(4 + c) * NN];
+      src.sin_lat = gg[10 * NN];
+    }
+    if (L.mode != 0) {
 #pragma unroll
-        for (int v = 0; v < NV; ++v) du[v] += d1 * f1[v] + d2 * f2[v];
+      for (int v = 0; v < NV; ++v) kreg[v] = L.k[v * NN + g];
+      if (L.dt_member) dt = L.dt_member[L.member[e]];
+    }
+  };
+  if (SPLIT && node_role && active) load_rest();
+  __syncthreads();
+
+  double du[NV], d1[NV];
+  if (node_role && active) volume_terms<N, UNROLL>(L, s_n[es], s_ds, q, 0, du);
+  if (dir1_role && active) {
+    volume_terms<N, UNROLL>(L, s_n[es], s_ds, q, 1, d1);
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) s_d1[es][v][q] = d1[v];
+    }
+  }
+  if (!SPLIT && active) {
+    load_rest();
+#pragma unroll
+    for (int v = 0; v < NV; ++v) du[v] += d1[v];
+  }
+  if (face_role) {
+#pragma unroll
+    for (int ps = 0; ps < S::PASSES; ++ps) {
+      const int fid = t + ps * B;
+      if (ps > 0) has_face = face_load<N, WAVES, GT>(L, e0, fid, fin);
+      if (!has_face) continue;
+      const int fe = fid / S::NF, r = fid - fe * S::NF;
+      double fs[NV];
+      face_flux<N, GT>(L, s_n[fe], r, fin, fs);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) s_sf[fe][v][r] = fs[v];
+    }
+  }
+  __syncthreads();
+  if (node_role && active) {
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) du[v] += s_d1[es][v][q];
+    }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+      const bool on = f == 0 ? ti == 0 : f == 1 ? ti == N - 1 : f == 2 ? tj == 0 : tj == N - 1;
+      if (!on) continue;
+      const int k = f < 2 ? tj : ti;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) du[v] += s_sf[es][v][f * N + k];
+    }
+    src.h = s_n[es][0][q];
+    src.hv[0] = s_n[es][1][q];
+    src.hv[1] = s_n[es][2][q];
+    src.J = s_n[es][5][q];
+    const double fac = div_nr(-1.0, src.J);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) du[v] *= fac;
+    if (L.source_terms) {
+      src.v[0] = s_n[es][3][q];
+      src.v[1] = s_n[es][4][q];
+      src.vc[0] = s_n[es][6][q];
+      src.vc[1] = s_n[es][7][q];
+      src.c11 = s_n[es][8][q];
+      src.c12 = s_n[es][9][q];
+      src.c22 = s_n[es][10][q];
+      double sv[NV];
+      if (L.source_terms == 2) source_standard(L.gravity, L.rotation_rate, src, sv);
+      else source_split(L.rotation_rate, src, sv);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) du[v] += sv[v];
+    }
+    if (L.mode == 0) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) L.out[g * NV + v] = du[v];
+    } else {
+      const double uo[NV] = {src.h, src.hv[0], src.hv[1]};
+      double un[NV];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const double kn = fma(L.rk_a, kreg[v], dt * du[v]);
+        L.k[v * NN + g] = kn;
+        un[v] = fma(L.rk_b, kn, uo[v]);
       }
-    } else if (active) {
-      const double hl = s_n[es][0][q], hvl[2] = {s_n[es][1][q], s_n[es][2][q]};
-      const double vl[2] = {s_n[es][3][q], s_n[es][4][q]};
-      const double Jl = s_n[es][5][q], hsl = s_n[es][12][q];
-      const double Gi[3] = {s_n[es][9][q], s_n[es][10][q], s_n[es][11][q]};
 #pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        const int own = o == 0 ? ti : tj;
-        // the partners in rotated order own + 1, ..., own + n - 1 (mod n):
-        // every lane has a partner in each step
-#pragma unroll 1
-        for (int j = 1; j < N; ++j) {
-          const int m = own + j >= N ? own + j - N : own + j;
-          const int pq = o == 0 ? m + N * tj : ti + N * m;
-          const double hr = s_n[es][0][pq], hvr_o = s_n[es][1 + o][pq];
-          const double vr[2] = {s_n[es][3][pq], s_n[es][4][pq]};
-          // the partner's covariant velocity G v from its staged G and v
-          const double vc0 = s_n[es][6][pq] * vr[0] + s_n[es][7][pq] * vr[1];
-          const double vc1 = s_n[es][7][pq] * vr[0] + s_n[es][8][pq] * vr[1];
-          const double Jr = s_n[es][5][pq];
-          double f[NV];
-          if (L.volume_flux == 0) {  // flux_ec (:100-122)
-            const double mass = 0.5 * (Jl * hvl[o] + Jr * hvr_o);
-            f[0] = mass;
-            f[1] = 0.5 * (vl[0] + vr[0]) * mass;
-            f[2] = 0.5 * (vl[1] + vr[1]) * mass;
-          } else {  // flux_central of the split flux (:66-80)
-            const double ml = Jl * hvl[o], mr = Jr * hvr_o;
-            f[0] = 0.5 * (ml + mr);
-            f[1] = 0.5 * (ml * vl[0] + mr * vr[0]);
-            f[2] = 0.5 * (ml * vl[1] + mr * vr[1]);
-          }
-          // flux_nonconservative_ec (:157-187) of (own, partner)
-          const double hs_jump = s_n[es][12][pq] - hsl;
-          const double geo0 = 0.5 * hvl[o] * ((Gi[0] * vc0 + Gi[1] * vc1) - vr[0]);
-          const double geo1 = 0.5 * hvl[o] * ((Gi[1] * vc0 + Gi[2] * vc1) - vr[1]);
-          const double Gio0 = o == 0 ? Gi[0] : Gi[1], Gio1 = o == 0 ? Gi[1] : Gi[2];
-          const double pr0 = L.gravity * Gio0 * hl * (hr + hs_jump);
-          const double pr1 = L.gravity * Gio1 * hl * (hr + hs_jump);
-          const double g1 = Jl * (geo0 + pr0), g2 = Jl * (geo1 + pr1);
-          const double ds = L.dsplit[own * N + m];
-          du[0] += ds * f[0];
-          du[1] += ds * f[1] + 0.5 * ds * g1;
-          du[2] += ds * f[2] + 0.5 * ds * g2;
-        }
+      for (int v = 0; v < NV; ++v) L.out[g * NV + v] = un[v];
+      if constexpr (SPEED) {
+        // the node's speeds go to its first two LDS fields, which only this
+        // lane reads after the face phase and which it has read already
+        double l[2];
+        swe_node_speeds(un, s_n[es][8][q], s_n[es][10][q], L.gravity, l);
+        s_n[es][0][q] = l[0];
+        s_n[es][1][q] = l[1];
       }
     }
-    // face nodes of the group's elements, one lane each
-    const double inv_w = L.inv_w;
-    for (int fid = t; fid < EPB * S::NF; fid += B) {
-      const int fe = fid / S::NF, r = fid - fe * S::NF;
-      const int f = r / N, k = r - f * N;
-      if (e0 + fe >= L.n_elements) continue;
-      const int i = f == 0 ? 0 : (f == 1 ? N - 1 : k);
-      const int j = f == 2 ? 0 : (f == 3 ? N - 1 : k);
-      const int qn = i + N * j;
-      const double ul[NV] = {s_n[fe][0][qn], s_n[fe][1][qn], s_n[fe][2][qn]};
-      // the own node's J, G, G^-1, h_s (aux rows 12-19) from LDS
-      double xa[NA] = {};
-      xa[12] = s_n[fe][5][qn];
+  }
+  if constexpr (SPEED) {
+    // per element: the maximum over its nodes of each speed (exact in any
+    // order), one lane per line of nodes and then its first lane over the
+    // lines, and the sum over the directions
+    __syncthreads();
+    if (node_role && active && tj == 0) {
+      double m1 = s_n[es][0][ti], m2 = s_n[es][1][ti];
 #pragma unroll
-      for (int c = 0; c < 6; ++c) xa[13 + c] = s_n[fe][6 + c][qn];
-      xa[19] = s_n[fe][12][qn];
-      const AuxV ax{xa, 1};
-      const size_t fnode = ((size_t)(e0 + fe) * 4 + f) * N + k;
-      const int link = L.nbr[fnode];
-      const double* ur = L.u + (size_t)link * NV;
-      // neighbour state in this element's contravariant basis (contravariant2global,
-      // then global2contravariant: covariant_shallow_water.jl:140-153)
-      const GT* M = face_maps<GT>(L) + fnode * 4;
-      const double tr[NV] = {ur[0], M[0] * ur[1] + M[1] * ur[2], M[2] * ur[1] + M[3] * ur[2]};
-      double fs[NV];
-      if constexpr (N == 4) {
-        // polydeg 3 keeps everything in registers with the orientation as a
-        // run-time value, and runs faster so (measured)
-        // the two states selected per lane and one call: the lanes of a wave
-        // hold faces of both signs, and a branch per sign runs both calls
-        const int o = f / 2;
-        const bool neg = f % 2 == 0;  // negative-side face: -(f*(u_nbr, u_own) + g/2)
-        double sl[NV], sr[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          sl[v] = neg ? tr[v] : ul[v];
-          sr[v] = neg ? ul[v] : tr[v];
-        }
-        surface_terms(L, sl, sr, ax, o, fs);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) fs[v] = neg ? -fs[v] : fs[v];
-      } else {
-        // the orientation as a compile-time constant in each branch: every
-        // index into the node arrays (u[1 + o], G^{io}) is then fixed and they
-        // stay in registers (with a run-time orientation they went to scratch);
-        // the sign's two states selected per lane, so a wave runs at most the
-        // two orientations' calls
-        const bool neg = f % 2 == 0;  // negative-side faces: -(f*(u_nbr, u_own) + g/2)
-        double sl[NV], sr[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          sl[v] = neg ? tr[v] : ul[v];
-          sr[v] = neg ? ul[v] : tr[v];
-        }
-        if (f < 2) surface_terms(L, sl, sr, ax, 0, fs);
-        else surface_terms(L, sl, sr, ax, 1, fs);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) fs[v] = neg ? -fs[v] : fs[v];
+      for (int r = 1; r < N; ++r) {
+        m1 = speed_max(m1, s_n[es][0][ti + N * r]);
+        m2 = speed_max(m2, s_n[es][1][ti + N * r]);
       }
-#pragma unroll
-      for (int v = 0; v < NV; ++v) s_sf[fe][v][r] = fs[v] * inv_w;
+      s_n[es][2][ti] = m1;
+      s_n[es][3][ti] = m2;
     }
     __syncthreads();
-    if (active) {
+    if (node_role && active && q == 0) {
+      double m1 = s_n[es][2][0], m2 = s_n[es][3][0];
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        const bool on = f == 0 ? ti == 0 : f == 1 ? ti == N - 1 : f == 2 ? tj == 0 : tj == N - 1;
-        if (!on) continue;
-        const int k = f < 2 ? tj : ti;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) du[v] += s_sf[es][v][f * N + k];
+      for (int r = 1; r < N; ++r) {
+        m1 = speed_max(m1, s_n[es][2][r]);
+        m2 = speed_max(m2, s_n[es][3][r]);
       }
-      const size_t g = (size_t)e * N2 + q;
-      const double fac = -1.0 / s_n[es][5][q];
-      const double uo[NV] = {s_n[es][0][q], s_n[es][1][q], s_n[es][2][q]};
-#pragma unroll
-      for (int v = 0; v < NV; ++v) du[v] *= fac;
-      if (L.source_terms) {
-        const GT* gg = geo_rows<GT>(L) + g;
-        const long long NN = L.n_nodes;
-        double xa[NA] = {};
-        xa[12] = s_n[es][5][q];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) xa[13 + c] = s_n[es][6 + c][q];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) xa[20 + c] = gg[(4 + c) * NN];
-        double sv[NV];
-        if (L.source_terms == 2)
-          source_standard(L.gravity, L.rotation_rate, uo, gg[10 * NN], AuxV{xa, 1}, sv);
-        else
-          source_split(L.rotation_rate, uo, gg[10 * NN], AuxV{xa, 1}, sv);
-#pragma unroll
-        for (int v = 0; v < NV; ++v) du[v] += sv[v];
-      }
-      if (L.mode == 0) {
-#pragma unroll
-        for (int v = 0; v < NV; ++v) L.out[g * NV + v] = du[v];
-      } else {
-        // the member's step size, else the launch's; selected as values (one
-        // conditional form with both reads merges them into a read through a
-        // pointer to global or argument memory, a flat load)
-        const double dt_m = L.dt_member ? L.dt_member[L.member[e]] : 0.0;
-        const double dt = L.dt_member ? dt_m : L.rk_dt;
-        double un[NV];
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          const double kn = L.rk_a * L.k[g * NV + v] + dt * du[v];
-          L.k[g * NV + v] = kn;
-          un[v] = uo[v] + L.rk_b * kn;
-          L.out[g * NV + v] = un[v];
-        }
-        if constexpr (SPEED) {
-          // the node's speeds go to its first two LDS fields, which only this
-          // lane reads after the face phase and which it has read already
-          double l[2];
-          swe_node_speeds(un, s_n[es][9][q], s_n[es][11][q], L.gravity, l);
-          s_n[es][0][q] = l[0];
-          s_n[es][1][q] = l[1];
-        }
-      }
-    }
-    if constexpr (SPEED) {
-      // per element: the maximum over its nodes of each speed (exact in any order),
-      // then the sum over the directions, by the element's first lane
-      __syncthreads();
-      if (active && q == 0) {
-        double m1 = s_n[es][0][0], m2 = s_n[es][1][0];
-        for (int r = 1; r < N2; ++r) {
-          m1 = speed_max(m1, s_n[es][0][r]);
-          m2 = speed_max(m2, s_n[es][1][r]);
-        }
-        L.speed_partial[e] = m1 + m2;
-      }
+      L.speed_partial[e] = m1 + m2;
     }
   }
 }
@@ -516,7 +538,7 @@ __global__ __launch_bounds__(64) void swe_max_speed(SweLaunch L, double* partial
     const size_t g = (size_t)e * N2 + q;
     const double* u = L.u + g * NV;
     double J, c11, c12, c22, l[2];
-    metric_from_gcov(gr[g], gr[L.n_nodes + g], gr[2 * L.n_nodes + g], J, c11, c12, c22);
+    metric_of(gr[g], gr[L.n_nodes + g], gr[2 * L.n_nodes + g], J, c11, c12, c22);
     swe_node_speeds(u, c11, c22, L.gravity, l);
     l1 = speed_max(l1, l[0]);
     l2 = speed_max(l2, l[1]);
@@ -552,32 +574,26 @@ __global__ void swe_member_max(const double* partial, const int* member_first, i
 
 namespace {
 
-template <int N, int WAVES, bool PERSIST>
+template <int N, int WAVES, bool SPLIT>
 void launch_variant(const SweLaunch& L, hipStream_t s) {
   using S = SweShape<N, WAVES>;
-  const int groups = (L.n_elements + S::EPB - 1) / S::EPB;
-  // persistent: a few workgroups per CU (256 CUs), each looping over groups
-  const int grid = PERSIST ? (groups < 256 * 8 ? groups : 256 * 8) : groups;
+  const dim3 grid((L.n_elements + S::EPB - 1) / S::EPB), block((SPLIT ? 3 : 1) * S::LANES);
   const bool speed = L.speed_partial && L.mode == 1;
   if (L.geo32) {
     if (speed)
-      hipLaunchKernelGGL((swe_stage<N, WAVES, PERSIST, true, float>), dim3(grid), dim3(S::BLOCK), 0,
-                         s, L);
+      hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, true, float>), grid, block, 0, s, L);
     else
-      hipLaunchKernelGGL((swe_stage<N, WAVES, PERSIST, false, float>), dim3(grid), dim3(S::BLOCK),
-                         0, s, L);
+      hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, false, float>), grid, block, 0, s, L);
   } else if (speed) {
-    hipLaunchKernelGGL((swe_stage<N, WAVES, PERSIST, true, double>), dim3(grid), dim3(S::BLOCK), 0,
-                       s, L);
+    hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, true, double>), grid, block, 0, s, L);
   } else {
-    hipLaunchKernelGGL((swe_stage<N, WAVES, PERSIST, false, double>), dim3(grid), dim3(S::BLOCK), 0,
-                       s, L);
+    hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, false, double>), grid, block, 0, s, L);
   }
 }
 
 template <int N>
 bool launch_n(const SweLaunch& L, int variant, hipStream_t s) {
-  // variants: 0..2 = 1, 2, 4 waves per workgroup; +3 = persistent grid
+  // variants: 0..2 = node lanes of 1, 2, 4 waves; 3..5 the same, split
   if constexpr (N * N > 64) {
     return false;
   } else {
@@ -641,6 +657,16 @@ bool swe_launch_member_max_speed(const SweLaunch& L, double* partial, const int*
 
 namespace atmo {
 
+namespace {
+// the rows of one node's 26 auxiliary variables that the integrals read
+struct AuxV {
+  const double* a;
+  __device__ __forceinline__ double J() const { return a[12]; }
+  __device__ __forceinline__ double Gcov(int i, int j) const { return a[13 + i + j]; }
+  __device__ __forceinline__ double hs() const { return a[19]; }
+};
+}  // namespace
+
 // per element: mass, total energy (entropy) and int w(u).du with the exact
 // area element (analysis_covariant.jl:53-105; covariant_shallow_water.jl:129-164)
 template <int N>
@@ -653,7 +679,7 @@ __global__ __launch_bounds__(64) void swe_integrals_kernel(SweLaunch L, const do
   for (int q = t; q < N2; q += 64) {
     const size_t g = (size_t)e * N2 + q;
     const double* u = L.u + g * NV;
-    const AuxV a{L.aux + g * NA, 1};
+    const AuxV a{L.aux + g * NA};
     const double h = u[0], v1 = u[1] / h, v2 = u[2] / h;
     const double vc1 = a.Gcov(0, 0) * v1 + a.Gcov(0, 1) * v2;
     const double vc2 = a.Gcov(1, 0) * v1 + a.Gcov(1, 1) * v2;

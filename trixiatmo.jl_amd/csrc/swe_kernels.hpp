@@ -19,7 +19,7 @@ struct SweLaunch {
   double inv_w;         // 1 / w_end
   const double* u;
   double* out;
-  double* k;
+  double* k;            // RK register, k[v * n_nodes + node]
   const double* aux;    // [26, n, n, E]
   const double* xyz;    // [3, n, n, E]
   // the stage kernel's geometry: geo[c * n_nodes + node] for c = G_11, G_12,
@@ -46,7 +46,7 @@ struct SweLaunch {
                             // directions of the maximum scaled speed of the new state
   const int* member;        // [E] member of each element
   int topography;           // 0: h_s is zero at every node and its row is not read
-  int variant;              // workgroup shape: 0..2 = 1, 2, 4 waves; +3 persistent grid
+  int variant;              // workgroup shape: node lanes of 1, 2, 4 waves (0..2), split (3..5)
 };
 constexpr int kSweVariants = 6;
 
@@ -72,9 +72,10 @@ constexpr int kSweGeo = 12;
 
 // J = sqrt(det G) and G^-1 = adj(G) / det G from the covariant metric tensor
 // G = A^T A (the identities aux rows 12 and 16-18 satisfy: J is the area
-// element |a_1 x a_2|); one sequence of operations, with an explicit fused
-// multiply-add, on the host and in every kernel, so each use gets the same bits
-__host__ __device__ inline void metric_from_gcov(double g11, double g12, double g22, double& J,
+// element |a_1 x a_2|), with an explicit fused
+// multiply-add: the host's check of the given metric (the kernels take theirs
+// from metric_of in swe_kernels.hip)
+inline void metric_from_gcov(double g11, double g12, double g22, double& J,
                                                  double& c11, double& c12, double& c22) {
   const double det = fma(g11, g22, -(g12 * g12));
   const double inv = 1.0 / det;
