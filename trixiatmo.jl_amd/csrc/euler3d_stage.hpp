@@ -946,7 +946,7 @@ void e3_stage_direct(
           acc[3].add(ds * (F * v3s + ps4 * n2s));
           acc[4].add(ds * (F * es + (T(2) * ps) * vns));
           if constexpr (NC != 0) {
-            const T ra = NC == 1 ? ln_mean_logs_branch(l.rho, r.rho, l.lrho, r.lrho) : T(0.5) * rs;
+            const T ra = NC == 1 ? ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho) : T(0.5) * rs;
             const T sj = ra * dphi;
             T sm = sj;  // momentum part: (rho_avg - rho_avg of the background) [phi]
             if constexpr (MIXED) {
