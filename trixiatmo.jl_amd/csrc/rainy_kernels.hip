@@ -28,21 +28,20 @@ constexpr int NV = 9;
 
 // cons2nonlinearsystemsol (:219-260)
 __device__ __forceinline__ void nonlinear_sol(const double* u, double& rv, double& rc, double& T) {
-  const double rho = u[0] + u[1] + u[2];
-  const double inv = 1.0 / rho;
-  if (u[1] == 0.0 && u[2] == 0.0) {
-    const double v1 = u[3] * inv, v2 = u[4] * inv;
-    const double ek = 0.5 * (v1 * v1 + v2 * v2) * rho;
-    rv = 0.0;
-    rc = 0.0;
-    T = (u[5] - ek) / (c_vd * rho);
-    return;
-  }
   rv = u[6];
   rc = u[7];
   if (rv < 0.0 && rv >= -1e-15) rv = 0.0;
   if (rc < 0.0 && rc >= -1e-15) rc = 0.0;
   T = u[8];
+  if (u[1] == 0.0 && u[2] == 0.0) {
+    const double rho = u[0] + u[1] + u[2];
+    const double inv = 1.0 / rho;
+    const double v1 = u[3] * inv, v2 = u[4] * inv;
+    const double ek = 0.5 * (v1 * v1 + v2 * v2) * rho;
+    rv = 0.0;
+    rc = 0.0;
+    T = (u[5] - ek) / (c_vd * rho);
+  }
 }
 
 // x^(1/8) by three square roots (pow(x, 0.125) of the reference to a few
@@ -61,13 +60,14 @@ __device__ __forceinline__ double terminal_velocity(double rho_moist, double rho
 constexpr double kSvp1 = (c_pv - c_l) / R_v;
 constexpr double kSvp2 = (L_ref - (c_pv - c_l) * ref_T) / R_v;
 __device__ __forceinline__ double svp(double T) {
-  return ref_sp * exp(kSvp1 * log(T / ref_T) + kSvp2 * (1 / ref_T - 1 / T));
+  return ref_sp * exp(kSvp1 * log_(T * (1 / ref_T)) + kSvp2 * (1 / ref_T - div_nr(1.0, T)));
 }
 
 // its derivative (:377-398), ref_sp / ref_T^k1 (k1 T^(k1-1) + k2 T^(k1-2))
 // exp(...), which equals svp(T) (k1 + k2 / T) / T
 __device__ __forceinline__ double svp_deriv_from(double sv, double T) {
-  return sv * (kSvp1 + kSvp2 / T) / T;
+  const double it = div_nr(1.0, T);
+  return sv * (kSvp1 + kSvp2 * it) * it;
 }
 
 // quantities of one node used by the two-point and surface fluxes
@@ -86,28 +86,15 @@ __device__ __forceinline__ RNode rnode(const double* u) {
   a.v2 = u[4] * a.inv;
   a.E = u[5];
   nonlinear_sol(u, a.rv, a.rc, a.T);
-  a.p = (R_d * a.rd + R_v * a.rv) * a.T;
-  // speed_of_sound (:299-334)
-  const double q_v = div_nr(a.rv, a.rd);
-  const double q_l = div_nr(a.rc + a.rr, a.rd);
-  const double gm = 1 + div_nr(R_d + R_v * q_v, c_vd + c_vv * q_v + c_l * q_l);
+  // speed_of_sound (:299-334), its ratio of heat capacities 1 + (R_d + R_v q_v)
+  // / (c_vd + c_vv q_v + c_l q_l) with both parts times rho_dry
+  const double R = R_d * a.rd + R_v * a.rv;
+  a.p = R * a.T;
+  const double gm = 1 + div_nr(R, c_vd * a.rd + c_vv * a.rv + c_l * (a.rc + a.rr));
   a.c = sqrt_(gm * a.p * a.inv);
   a.vr_m = terminal_velocity(a.rm, a.rr);
   a.vr_sol = terminal_velocity(a.rv + a.rc, a.rr);
   return a;
-}
-
-// flux in normal direction (:502-545)
-__device__ __forceinline__ void flux_n(const RNode& a, double n1, double n2, double* f) {
-  const double vn = a.v1 * n1 + a.v2 * n2;
-  const double vrn = a.vr_m * n2;
-  f[0] = a.rd * vn;
-  f[1] = a.rm * vn;
-  f[2] = a.rr * (vn - vrn);
-  f[3] = a.rho * vn * a.v1 + a.p * n1 - a.rr * vrn * a.v1;
-  f[4] = a.rho * vn * a.v2 + a.p * n2 - a.rr * vrn * a.v2;
-  f[5] = (a.E + a.p) * vn - (c_l * a.T + 0.5 * (a.v1 * a.v1 + a.v2 * a.v2)) * a.rr * vrn;
-  f[6] = f[7] = f[8] = 0.0;
 }
 
 // flux in orientation form (:448-500): orientation 1 has no rain terms
@@ -186,26 +173,45 @@ __device__ __forceinline__ ECNode ecnode(const double* u) {
   return a;
 }
 
-// flux_lax_friedrichs with max_abs_speed_naive (:607-624) on all nine entries
-__device__ __forceinline__ void flux_llf(const RNode& l, const RNode& r, const double* ul,
-                                         const double* ur, double n1, double n2, double* f) {
-  double fl[NV], fr[NV];
-  flux_n(l, n1, n2, fl);
-  flux_n(r, n1, n2, fr);
-  double vl = fabs(l.v1 * n1 + l.v2 * n2);
-  vl += fabs(l.vr_m * n2);
-  double vr = fabs(r.v1 * n1 + r.v2 * n2);
-  vr += fabs(r.vr_m * n2);
-  const double lam = fmax(vl, vr) + fmax(l.c, r.c) * sqrt_(n1 * n1 + n2 * n2);
-#pragma unroll
-  for (int v = 0; v < NV; ++v) f[v] = 0.5 * (fl[v] + fr[v]) - 0.5 * lam * (ur[v] - ul[v]);
+// flux in normal direction (:502-545), its first six entries (the others are
+// zero), and the normal speeds of max_abs_speed_naive (:607-624)
+__device__ __forceinline__ double flux_n(const RNode& a, double n1, double n2, double* f) {
+  const double vn = a.v1 * n1 + a.v2 * n2;
+  const double vrn = a.vr_m * n2;
+  const double m = a.rho * vn - a.rr * vrn;
+  f[0] = a.rd * vn;
+  f[1] = a.rm * vn;
+  f[2] = a.rr * (vn - vrn);
+  f[3] = m * a.v1 + a.p * n1;
+  f[4] = m * a.v2 + a.p * n2;
+  f[5] = (a.E + a.p) * vn - (c_l * a.T + 0.5 * (a.v1 * a.v1 + a.v2 * a.v2)) * a.rr * vrn;
+  return fabs(vn) + fabs(vrn);
 }
 
-__device__ __forceinline__ void surface_flux(const RainyLaunch& L, const double* ul,
-                                             const double* ur, double n1, double n2, double* f) {
-  const RNode l = rnode(ul), r = rnode(ur);
-  if (L.surface_flux == 1) flux_ec_rain(l, r, n1, n2, f);
-  else flux_llf(l, r, ul, ur, n1, n2, f);
+// The flux of one face node along the positive axis of its direction (n1 or
+// n2 is zero), lifted: sgn w f#(own, nbr) with sgn = -1 on a face whose outward
+// normal points along the negative axis.  The averages are symmetric in the
+// two states; only flux_lax_friedrichs' dissipation (all nine entries) knows
+// the order, and its sign turns with sgn.
+__device__ __forceinline__ void surface_flux(const RainyLaunch& L, const double* uo,
+                                             const double* un, double n1, double n2, double sgn,
+                                             double w, double* f) {
+  const RNode l = rnode(uo), r = rnode(un);
+  if (L.surface_flux == 1) {
+    flux_ec_rain(l, r, n1, n2, f);
+#pragma unroll
+    for (int v = 0; v < 6; ++v) f[v] *= sgn * w;
+    f[6] = f[7] = f[8] = 0.0;
+    return;
+  }
+  double fl[6], fr[6];
+  const double sl = flux_n(l, n1, n2, fl), sr = flux_n(r, n1, n2, fr);
+  const double lam = fmax(sl, sr) + fmax(l.c, r.c) * (n1 + n2);
+  const double c = 0.5 * sgn * w, d = -0.5 * lam * w;
+#pragma unroll
+  for (int v = 0; v < 6; ++v) f[v] = c * (fl[v] + fr[v]) + d * (un[v] - uo[v]);
+#pragma unroll
+  for (int v = 6; v < NV; ++v) f[v] = d * (un[v] - uo[v]);
 }
 
 // source_terms_rainy (:547-577)
@@ -213,7 +219,7 @@ __device__ __forceinline__ void source_rainy(const double* u, double* s) {
   const double rho = u[0] + u[1] + u[2];
   double rv, rc, T;
   nonlinear_sol(u, rv, rc, T);
-  const double rho_vs = svp(T) / (R_v * T);
+  const double rho_vs = div_nr(svp(T), R_v * T);
   const double rr = u[2];
   // rr^(3/16), rr^(1/2), rr^(7/8) from the chain of square roots
   const double r2 = sqrt_(rr), r4 = sqrt_(r2), r8 = sqrt_(r4), r16 = sqrt_(r8);
@@ -283,7 +289,7 @@ __device__ __forceinline__ void residual(const double* u, const double* x, doubl
   double r1 = (c_vd * u[0] + c_vv * x[0] + c_l * (x[1] + u[2])) * x[2];
   r1 += x[0] * L_ref;
   r1 -= (u[5] - rho * 0.5 * (v1 * v1 + v2 * v2));
-  double r2 = fmin(sv / (R_v * x[2]), u[1]);
+  double r2 = fmin(div_nr(sv, R_v * x[2]), u[1]);
   r2 -= x[0];
   r2 *= 1.0e7;
   double r3 = u[1];
@@ -301,7 +307,7 @@ __device__ __forceinline__ void jacobian(const double* u, const double* x, doubl
   J[6] = c_vd * u[0] + c_vv * x[0] + c_l * (x[1] + u[2]);
   J[1] = -10000000.0;
   J[4] = 0.0;
-  J[7] = (sv / (R_v * x[2]) < u[1]) ? (svt * x[2] - sv) / (R_v * x[2] * x[2]) * 1.0e7 : 0.0;
+  J[7] = (div_nr(sv, R_v * x[2]) < u[1]) ? div_nr(svt * x[2] - sv, R_v * x[2] * x[2]) * 1.0e7 : 0.0;
   J[2] = -10000000.0;
   J[5] = -10000000.0;
   J[8] = 0.0;
@@ -349,7 +355,7 @@ __device__ __forceinline__ void solve3(const double* J, const double* r, double*
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       if (i <= c) continue;
-      const double f = a[i][c] / a[c][c];
+      const double f = div_nr(a[i][c], a[c][c]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (j >= c) a[i][j] -= f * a[c][j];
@@ -361,7 +367,7 @@ __device__ __forceinline__ void solve3(const double* J, const double* r, double*
 #pragma unroll
     for (int j = 0; j < 3; ++j)
       if (j > i) sacc -= a[i][j] * dx[j];
-    dx[i] = sacc / a[i][i];
+    dx[i] = div_nr(sacc, a[i][i]);
   }
 }
 
@@ -529,13 +535,49 @@ __device__ __forceinline__ void rainy_node_speeds(const RainyLaunch& L, const do
   l[1] = fabs(0.0 * lam1 + L.Ja22 * lam2) * L.inv_J;
 }
 
+// a face node of the workgroup's elements: the neighbour's state, requested
+// at the start of the stage
+struct RFace {
+  double u[NV];
+  bool wall;  // boundary_condition_simple_slip_wall: the own state mirrored
+};
+
+template <int N>
+__device__ __forceinline__ bool face_load(const RainyLaunch& L, int e0, int fid, RFace& x) {
+  using S = RShape<N>;
+  constexpr int N2 = S::N2;
+  const int fe = fid / S::NF, r = fid - fe * S::NF;
+  const int f = r / N, l = r - f * N, ee = e0 + fe;
+  if (fid >= S::EPB * S::NF || ee >= L.n_elements) return false;
+  const int ey = ee / L.nx, ex = ee - L.nx * ey;
+  int en, qn;
+  if (f < 2) {
+    const int x1 = f == 0 ? (ex == 0 ? L.nx - 1 : ex - 1) : (ex + 1 == L.nx ? 0 : ex + 1);
+    en = x1 + L.nx * ey;
+    qn = f == 0 ? (N - 1) + N * l : N * l;
+  } else {
+    const int y1 = f == 2 ? (ey == 0 ? L.ny - 1 : ey - 1) : (ey + 1 == L.ny ? 0 : ey + 1);
+    en = ex + L.nx * y1;
+    qn = f == 2 ? l + N * (N - 1) : l;
+  }
+  x.wall = !L.periodic_y && ((f == 2 && ey == 0) || (f == 3 && ey == L.ny - 1));
+  const double* un = L.u + ((size_t)en * N2 + qn) * NV;
+#pragma unroll
+  for (int v = 0; v < NV; ++v) x.u[v] = un[v];
+  return true;
+}
+
+// What bounds the stage: a wave's chain of dependent operations and memory
+// round trips, at four waves per SIMD (neither the FP64 rate nor HBM: 256 x 128
+// cells at polydeg 3, 151 MB and about 0.9 GFLOP, take 41 us).  So every
+// input is requested at the start (the state came in nine waited-for rounds,
+// the neighbours' after the volume terms, Dsplit from the argument block in
+// every step of the volume loop), the register is read and written in rows,
+// each pair's flux is evaluated once where both of its nodes can have it, and
+// quotients by one denominator share its reciprocal: 60 -> 41 us per stage.
 // SPEED: the RK stage also writes L.speed_partial (the last stage of a
 // resident step); a variant of its own, so the other stages keep their
 // register budget
-// polydeg 3 without the network: a four-wave register budget (128 VGPRs,
-// 64 B of scratch per lane) measured 67.0 against 68.2 us per stage at 136
-// VGPRs and three waves; the network-seeded variant, whose inference holds
-// more values, keeps the compiler's choice
 template <int N, bool SEEDED, bool SPEED>
 __global__ __launch_bounds__(RShape<N>::BLOCK)
 __attribute__((amdgpu_waves_per_eu(N == 4 && !SEEDED ? 4 : 1)))
@@ -543,49 +585,66 @@ void rainy_stage(RainyLaunch L) {
   using S = RShape<N>;
   constexpr int N2 = S::N2, EPB = S::EPB, B = S::BLOCK;
   // one buffer per element, used in turn for the volume terms (flux
-  // differencing: the per-node quantities of flux_ec_rain [11][N2]; weak form:
-  // the contravariant fluxes of the 6 flux rows, [2][6][N2] where they fit,
-  // else one direction [6][N2] at a time) and for the face fluxes [9][4 n].
-  // Sized by flux differencing and the faces: at polydeg 3 the workgroup then
-  // takes 10,240 B of LDS and sixteen fit on a CU (160 KiB) where 10,752 B
-  // let fifteen, which put the 8,192 workgroups of a 256 x 128 mesh in three
-  // rounds instead of two
-  constexpr int VOLW = 11 * N2 > NV * S::NF ? 11 * N2 : NV * S::NF;
+  // differencing: nine of the per-node quantities of flux_ec_rain [9][N2],
+  // the two densities are the state's own; weak form: the contravariant
+  // fluxes of the 6 flux rows, [2][6][N2] where they fit, else one direction
+  // [6][N2] at a time) and for the face fluxes [9][4 n].  At polydeg 3 the
+  // workgroup takes 9,344 B of LDS, so that sixteen fit on a CU (160 KiB)
+  constexpr int VOLW = 9 * N2 > NV * S::NF ? 9 * N2 : NV * S::NF;
   constexpr bool WEAK_SPLIT = 12 * N2 > VOLW;
   __shared__ double s_u[EPB][NV][N2];
   __shared__ double s_buf[EPB][VOLW];
+  __shared__ double s_ds[N2];  // Dsplit, or derivative_hat in the weak form
   auto s_f = [&](int es, int o, int v, int q) -> double& { return s_buf[es][(o * 6 + v) * N2 + q]; };
   auto s_ec = [&](int es, int k, int q) -> double& { return s_buf[es][k * N2 + q]; };
   auto s_sf = [&](int es, int v, int r) -> double& { return s_buf[es][v * S::NF + r]; };
 
   const int t = threadIdx.x;
   const int e0 = blockIdx.x * EPB;
+  const int es = t / N2, q = t - es * N2;
+  const int e = e0 + es;
+  const bool active = es < EPB && e < L.n_elements;
+  const int ti = q % N, tj = q / N;
+  const size_t g = (size_t)e * N2 + q;  // the lane's node
   double rk_dt = L.rk_dt, t_src = L.t;
   if (L.clock) {
     rk_dt = L.clock[1];
     t_src = stage_time(L.clock[0], L.c_stage, rk_dt);
     if (L.mode == 1 && rk_dt == 0.0) {  // finished: the state is carried over as it is
-      for (int idx = t; idx < EPB * N2 * NV; idx += B) {
-        const size_t g = (size_t)e0 * N2 * NV + idx;
-        if (e0 + idx / (N2 * NV) < L.n_elements) L.out[g] = L.u[g];
+      if (active) {
+#pragma unroll
+        for (int v = 0; v < NV; ++v) L.out[g * NV + v] = L.u[g * NV + v];
       }
       return;
     }
   }
-  for (int idx = t; idx < EPB * N2 * NV; idx += B) {
-    const int es = idx / (N2 * NV), r = idx - es * N2 * NV;
-    if (e0 + es < L.n_elements) s_u[es][r % NV][r / NV] = L.u[(size_t)(e0 + es) * N2 * NV + r];
+  // every input of the first phases is requested before any is waited for: the
+  // first pass's neighbour states, the own states, the matrix
+  RFace fin;
+  bool has_face = face_load<N>(L, e0, t, fin);
+  double du[NV];
+  {
+    double uo[NV];
+    if (active) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) uo[v] = L.u[g * NV + v];
+    }
+    if (t < N2) s_ds[t] = L.volume_integral == 0 ? L.dhat[t] : L.dsplit[t];
+    if (active) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) s_u[es][v][q] = uo[v];
+      if (L.volume_integral != 0) {
+        const ECNode a = ecnode(uo);
+        s_ec(es, 0, q) = a.rv; s_ec(es, 1, q) = a.rc; s_ec(es, 2, q) = a.v1;
+        s_ec(es, 3, q) = a.v2; s_ec(es, 4, q) = a.it; s_ec(es, 5, q) = a.vr;
+        s_ec(es, 6, q) = a.lrd; s_ec(es, 7, q) = a.lrv; s_ec(es, 8, q) = a.lit;
+      }
+    }
   }
   // the network's parameters are read from memory where used: the reads are
   // uniform over the wave (cached), cheaper than staging them per workgroup
   const bool seeded = SEEDED && L.mode == 1 && L.newton_max_iter > 0;
   __syncthreads();
-
-  const int es = t / N2, q = t - es * N2;
-  const int e = e0 + es;
-  const bool active = es < EPB && e < L.n_elements;
-  const int ti = q % N, tj = q / N;
-  double du[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) du[v] = 0.0;
 
@@ -612,7 +671,7 @@ void rainy_stage(RainyLaunch L) {
       if (active) {
 #pragma unroll
         for (int m = 0; m < N; ++m) {
-          const double d1 = L.dhat[ti * N + m], d2 = L.dhat[tj * N + m];
+          const double d1 = s_ds[ti * N + m], d2 = s_ds[tj * N + m];
 #pragma unroll
           for (int v = 0; v < 6; ++v)
             du[v] += d1 * s_f(es, 0, v, m + N * tj) + d2 * s_f(es, 1, v, ti + N * m);
@@ -623,7 +682,7 @@ void rainy_stage(RainyLaunch L) {
       if (active) {
 #pragma unroll
         for (int m = 0; m < N; ++m) {
-          const double d1 = L.dhat[ti * N + m];
+          const double d1 = s_ds[ti * N + m];
 #pragma unroll
           for (int v = 0; v < 6; ++v) du[v] += d1 * s_f(es, 0, v, m + N * tj);
         }
@@ -637,55 +696,49 @@ void rainy_stage(RainyLaunch L) {
       if (active) {
 #pragma unroll
         for (int m = 0; m < N; ++m) {
-          const double d2 = L.dhat[tj * N + m];
+          const double d2 = s_ds[tj * N + m];
 #pragma unroll
           for (int v = 0; v < 6; ++v) du[v] += d2 * s_f(es, 0, v, ti + N * m);
         }
       }
     }
-  } else {
-    // flux differencing with flux_ec_rain, gathered per node.  flux_ec_rain
-    // gives the same bits with its two states exchanged (every operation is
-    // commutative, negates both operands of a quotient, or is kept from
-    // contraction where the order of a contracted sum would show), so each
-    // lane takes its partners in rotated order own + 1, ..., own + n - 1
-    // (mod n) with its own node on the left: every lane has a partner in each
-    // of the n - 1 steps and the wave evaluates one flux per step (a loop over
-    // the line's n nodes that skips the own one and orders the pair by index
-    // runs both orders of the call under divergent lanes in every step)
-    if (active) {
-      double uo[NV];
+  } else if (active) {
+    // flux differencing with flux_ec_rain.  The flux has the same bits with
+    // its two states exchanged, and all nodes of a line belong to one wave: a
+    // lane evaluates the pairs with its next floor(n / 2) nodes (cyclic) and
+    // receives the flux of the pair with the node as far behind it from that
+    // node's lane, which has just evaluated it (with n even the last step pairs
+    // opposite nodes: each of the two evaluates it).  At polydeg 3 that is four
+    // fluxes of about 100 operations instead of six of about 150
+    ECNode a;
+    a.rd = s_u[es][0][q]; a.rr = s_u[es][2][q];
+    a.rv = s_ec(es, 0, q); a.rc = s_ec(es, 1, q); a.v1 = s_ec(es, 2, q); a.v2 = s_ec(es, 3, q);
+    a.it = s_ec(es, 4, q); a.vr = s_ec(es, 5, q);
+    a.lrd = s_ec(es, 6, q); a.lrv = s_ec(es, 7, q); a.lit = s_ec(es, 8, q);
 #pragma unroll
-      for (int v = 0; v < NV; ++v) uo[v] = s_u[es][v][q];
-      const ECNode a = ecnode(uo);
-      s_ec(es, 0, q) = a.rd; s_ec(es, 1, q) = a.rv; s_ec(es, 2, q) = a.rc; s_ec(es, 3, q) = a.rr;
-      s_ec(es, 4, q) = a.v1; s_ec(es, 5, q) = a.v2; s_ec(es, 6, q) = a.it; s_ec(es, 7, q) = a.vr;
-      s_ec(es, 8, q) = a.lrd; s_ec(es, 9, q) = a.lrv; s_ec(es, 10, q) = a.lit;
-    }
-    __syncthreads();
-    if (active) {
-      ECNode a;
-      a.rd = s_ec(es, 0, q); a.rv = s_ec(es, 1, q); a.rc = s_ec(es, 2, q); a.rr = s_ec(es, 3, q);
-      a.v1 = s_ec(es, 4, q); a.v2 = s_ec(es, 5, q); a.it = s_ec(es, 6, q); a.vr = s_ec(es, 7, q);
-      a.lrd = s_ec(es, 8, q); a.lrv = s_ec(es, 9, q); a.lit = s_ec(es, 10, q);
-#pragma unroll
-      for (int o = 0; o < 2; ++o) {
-        const int own = o == 0 ? ti : tj;
-        const double n1 = o == 0 ? L.Ja11 : 0.0, n2 = o == 0 ? 0.0 : L.Ja22;
+    for (int o = 0; o < 2; ++o) {
+      const int own = o == 0 ? ti : tj, stride = o == 0 ? 1 : N;
+      const double n1 = o == 0 ? L.Ja11 : 0.0, n2 = o == 0 ? 0.0 : L.Ja22;
+      const double* ds_row = s_ds + own * (N + 1);
 #pragma unroll 1
-        for (int j = 1; j < N; ++j) {
-          const int m = own + j >= N ? own + j - N : own + j;
-          const int pq = o == 0 ? m + N * tj : ti + N * m;
-          ECNode b;
-          b.rd = s_ec(es, 0, pq); b.rv = s_ec(es, 1, pq); b.rc = s_ec(es, 2, pq);
-          b.rr = s_ec(es, 3, pq); b.v1 = s_ec(es, 4, pq); b.v2 = s_ec(es, 5, pq);
-          b.it = s_ec(es, 6, pq); b.vr = s_ec(es, 7, pq);
-          b.lrd = s_ec(es, 8, pq); b.lrv = s_ec(es, 9, pq); b.lit = s_ec(es, 10, pq);
-          double f[6];
-          flux_ec_rain(a, b, n1, n2, f);
-          const double ds = L.dsplit[own * N + m];
+      for (int j = 1; j <= N / 2; ++j) {
+        const int step = own + j >= N ? j - N : j;
+        const int pq = q + step * stride;
+        ECNode b;
+        b.rd = s_u[es][0][pq]; b.rr = s_u[es][2][pq];
+        b.rv = s_ec(es, 0, pq); b.rc = s_ec(es, 1, pq); b.v1 = s_ec(es, 2, pq);
+        b.v2 = s_ec(es, 3, pq); b.it = s_ec(es, 4, pq); b.vr = s_ec(es, 5, pq);
+        b.lrd = s_ec(es, 6, pq); b.lrv = s_ec(es, 7, pq); b.lit = s_ec(es, 8, pq);
+        double f[6];
+        flux_ec_rain(a, b, n1, n2, f);
+        const double ds = ds_row[step];
 #pragma unroll
-          for (int v = 0; v < 6; ++v) du[v] += ds * f[v];
+        for (int v = 0; v < 6; ++v) du[v] += ds * f[v];
+        if (2 * j < N) {
+          const int back = own < j ? N - j : -j;
+          const double db = ds_row[back];
+#pragma unroll
+          for (int v = 0; v < 6; ++v) du[v] += db * __shfl(f[v], t + back * stride, 64);
         }
       }
     }
@@ -694,55 +747,25 @@ void rainy_stage(RainyLaunch L) {
   // surface fluxes, one lane per face node of the workgroup's elements; the
   // buffer of the volume terms is free once every lane has gathered
   __syncthreads();
-  for (int fid = t; fid < EPB * S::NF; fid += B) {
+  constexpr int PASSES = (EPB * S::NF + B - 1) / B;
+#pragma unroll
+  for (int ps = 0; ps < PASSES; ++ps) {
+    const int fid = t + ps * B;
+    if (ps > 0) has_face = face_load<N>(L, e0, fid, fin);
+    if (!has_face) continue;
     const int fe = fid / S::NF, r = fid - fe * S::NF;
     const int f = r / N, l = r - f * N;
-    const int ee = e0 + fe;
-    if (ee >= L.n_elements) continue;
-    const int ex = ee % L.nx, ey = ee / L.nx;
-    double ul[NV], ur[NV], fl[NV];
-    double n1 = 0.0, n2 = 0.0;
-    if (f < 2) {
-      n1 = L.Ja11;
-      const int en = f == 0 ? ((ex + L.nx - 1) % L.nx) + L.nx * ey : ((ex + 1) % L.nx) + L.nx * ey;
-      const int qo = f == 0 ? N * l : (N - 1) + N * l;          // own node
-      const int qn = f == 0 ? (N - 1) + N * l : N * l;          // neighbour node
-      const double* un = L.u + ((size_t)en * N2 + qn) * NV;
+    const int qo = f == 0 ? N * l : f == 1 ? (N - 1) + N * l : f == 2 ? l : l + N * (N - 1);
+    double uo[NV], fl[NV];
 #pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        const double own = s_u[fe][v][qo];
-        ul[v] = f == 0 ? un[v] : own;
-        ur[v] = f == 0 ? own : un[v];
-      }
-    } else {
-      n2 = L.Ja22;
-      const bool bottom = f == 2;
-      const int qo = bottom ? l : l + N * (N - 1);
-      const bool wall = !L.periodic_y && (bottom ? ey == 0 : ey == L.ny - 1);
-      double nb[NV];
-      if (wall) {
-        // boundary_condition_simple_slip_wall (:963-983): mirrored state
-#pragma unroll
-        for (int v = 0; v < NV; ++v) nb[v] = s_u[fe][v][qo];
-        nb[4] = -nb[4];
-      } else {
-        const int en = bottom ? ex + L.nx * ((ey + L.ny - 1) % L.ny) : ex + L.nx * ((ey + 1) % L.ny);
-        const int qn = bottom ? l + N * (N - 1) : l;
-        const double* un = L.u + ((size_t)en * N2 + qn) * NV;
-#pragma unroll
-        for (int v = 0; v < NV; ++v) nb[v] = un[v];
-      }
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        const double own = s_u[fe][v][qo];
-        ul[v] = bottom ? nb[v] : own;
-        ur[v] = bottom ? own : nb[v];
-      }
+    for (int v = 0; v < NV; ++v) {
+      uo[v] = s_u[fe][v][qo];
+      if (fin.wall) fin.u[v] = v == 4 ? -uo[v] : uo[v];  // (:963-983)
     }
-    surface_flux(L, ul, ur, n1, n2, fl);
-    const double sgn = (f % 2 == 0) ? -L.inv_w0 : L.inv_wn;
+    surface_flux(L, uo, fin.u, f < 2 ? L.Ja11 : 0.0, f < 2 ? 0.0 : L.Ja22, (f & 1) ? 1.0 : -1.0,
+                 (f & 1) ? L.inv_wn : L.inv_w0, fl);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) s_sf(fe, v, r) = sgn * fl[v];
+    for (int v = 0; v < NV; ++v) s_sf(fe, v, r) = fl[v];
   }
   __syncthreads();
   int it_stat = 0, fallback_stat = 0;
@@ -783,17 +806,20 @@ void rainy_stage(RainyLaunch L) {
       for (int v = 0; v < NV; ++v) du[v] += sv[v];
     }
     if (L.mode == 0) {
-      const size_t g = ((size_t)e * N2 + q) * NV;
 #pragma unroll
-      for (int v = 0; v < NV; ++v) L.out[g + v] = du[v];
+      for (int v = 0; v < NV; ++v) L.out[g * NV + v] = du[v];
     } else {
-      const size_t g = ((size_t)e * N2 + q) * NV;
+      const size_t NN = (size_t)L.n_elements * N2;
+      double kn[NV];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) kn[v] = L.k[v * NN + g];
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        const double kn = L.rk_a * L.k[g + v] + rk_dt * du[v];
-        L.k[g + v] = kn;
-        un[v] = uo[v] + L.rk_b * kn;
+        kn[v] = L.rk_a * kn[v] + rk_dt * du[v];
+        un[v] = uo[v] + L.rk_b * kn[v];
       }
+#pragma unroll
+      for (int v = 0; v < NV; ++v) L.k[v * NN + g] = kn[v];
     }
   }
   // the network's prediction for the updated states: every lane of the wave
@@ -806,7 +832,6 @@ void rainy_stage(RainyLaunch L) {
     }
   }
   if (active && L.mode != 0) {
-    const size_t g = ((size_t)e * N2 + q) * NV;
     // the stage limiter: NonlinearSolveDG on the updated state
     {
       if (L.newton_max_iter > 0) {
@@ -836,7 +861,7 @@ void rainy_stage(RainyLaunch L) {
         un[8] = x[2];
       }
 #pragma unroll
-      for (int v = 0; v < NV; ++v) L.out[g + v] = un[v];
+      for (int v = 0; v < NV; ++v) L.out[g * NV + v] = un[v];
       if constexpr (SPEED) {
         // the node's speeds go to its first two state fields in LDS, which
         // only this lane reads after the face phase and which it has read
@@ -849,13 +874,26 @@ void rainy_stage(RainyLaunch L) {
   }
   if constexpr (SPEED) {
     // per element: the maximum over its nodes of each speed (exact in any
-    // order, NaN-propagating), then the sum over the directions
+    // order, NaN-propagating), one lane per line of nodes and then its first
+    // lane over the lines, and the sum over the directions
+    __syncthreads();
+    if (active && tj == 0) {
+      double m1 = s_u[es][0][ti], m2 = s_u[es][1][ti];
+#pragma unroll
+      for (int r = 1; r < N; ++r) {
+        m1 = speed_max(m1, s_u[es][0][ti + N * r]);
+        m2 = speed_max(m2, s_u[es][1][ti + N * r]);
+      }
+      s_u[es][2][ti] = m1;
+      s_u[es][3][ti] = m2;
+    }
     __syncthreads();
     if (active && q == 0) {
-      double m1 = s_u[es][0][0], m2 = s_u[es][1][0];
-      for (int r = 1; r < N2; ++r) {
-        m1 = speed_max(m1, s_u[es][0][r]);
-        m2 = speed_max(m2, s_u[es][1][r]);
+      double m1 = s_u[es][2][0], m2 = s_u[es][3][0];
+#pragma unroll
+      for (int r = 1; r < N; ++r) {
+        m1 = speed_max(m1, s_u[es][2][r]);
+        m2 = speed_max(m2, s_u[es][3][r]);
       }
       L.speed_partial[e] = m1 + m2;
     }

@@ -97,7 +97,7 @@ struct RainyLaunch {
   double dhat[64];            // Trixi derivative_dhat[i * n + m]
   const double* u;
   double* out;
-  double* k;
+  double* k;                  // RK register, k[v * nodes + node]
   int mode;                   // 0 rhs, 1 RK stage (+ Newton on the new state)
   double t;                   // time of the rhs evaluation (time-dependent sources)
   double rk_a, rk_dt, rk_b;
