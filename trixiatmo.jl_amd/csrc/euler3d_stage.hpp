@@ -31,6 +31,18 @@
 // per entry instead of a stride of 72 or 40 bytes: shell 6 x 16^2 x 8 at
 // polydeg 4, 150 resident steps 101.9 against 103.0 ms (two alternating
 // runs); the other sizes within noise.
+//
+// The direct form is bound by the waits of a workgroup's own chain (loads,
+// volume, faces, update) at four waves per SIMD, not by HBM or the vector rate
+// alone.  So the inputs are requested together at the start (state, vectors and
+// links came one after the other, with Dsplit's read waited for first), the
+// volume sums are folded before the face phase, and the update's inputs are
+// requested during it: resident runs, ms, shell polydeg 4 101.6 -> 95.0, brick
+// polydeg 3 (a right-hand side, us) 14.95 -> 12.8, shell polydeg 5 13.0 ->
+// 12.2, polydeg 7 49.5 -> 47.2 (with the logarithmic means).  The register
+// budget decides what can be asked for early: 28 B of scratch per lane cost
+// 10 % (106 against 96 ms), so polydeg 3 and 4, whose faces take two passes,
+// ask for the register after the faces.
 #ifndef ATMO_EULER3D_STAGE_HPP
 #define ATMO_EULER3D_STAGE_HPP
 
@@ -289,10 +301,10 @@ __device__ __forceinline__ void surface_momentum_split(const E3Params& q, int su
 
 // face-node passes of one workgroup and the neighbour states they need,
 // loaded at the start of the kernel so that the dependent loads (link, then
-// the neighbour's state) overlap the volume phase; from polydeg 4 on only the
-// first pass (every lane of the workgroup) is: polydeg 4's partial second
-// pass then loads in place, which keeps 14 registers free during the volume
-// phase (5 % faster there; polydeg 3, one wave per element, prefetches both).
+// the neighbour's state) overlap the volume phase; from polydeg 3 on only the
+// first pass (every lane of the workgroup) is: the partial second pass of
+// polydeg 3 and 4 then loads in place, which keeps 14 registers free during
+// the volume phase.
 // A workgroup holds EPB elements (slots es = 0..EPB-1 of Shape<N>::BLOCK
 // lanes each); its EPB * 6 n^2 face nodes are spread over all its lanes,
 // face node fg = t + ps * EPB * BLOCK of pass ps being node fg mod 6 n^2 of
@@ -302,64 +314,42 @@ struct FacePrefetch {
   static constexpr int GB = EPB * Shape<N>::BLOCK;
   static constexpr int NF = 6 * Shape<N>::N2;
   static constexpr int PASSES = (EPB * NF + GB - 1) / GB;
-  static constexpr int PF = N >= 5 ? 1 : PASSES;
-  int link[PF], info[PF];
+  static constexpr int PF = N >= 4 ? 1 : PASSES;
+  int link[PASSES], info[PASSES];
   double ur[PF][6];
 };
 
-// link (neighbour's global node, < 0 on a boundary) and face_info of pass ps;
-// elements e0 .. e0 + n_valid - 1 are the workgroup's
-template <int N, int EPB = 1>
-__device__ __forceinline__ void face_link(const FacePrefetch<N, EPB>& pf, int e0, int n_valid,
-                                          int t, int ps, const int* __restrict__ nbr,
-                                          const int* __restrict__ face_info, int& link,
-                                          int& info) {
+// The links are requested first and the states once they are here; a lane
+// without a face node (or on a boundary) reads a valid address and ignores it,
+// so the loads stand in straight-line code with the kernel's other inputs
+// between them in flight.
+template <int N, int EPB, int FROM, int TO>
+__device__ __forceinline__ void face_links(FacePrefetch<N, EPB>& pf, int e0, int n_valid,
+                                           int t, const int* __restrict__ nbr,
+                                           const int* __restrict__ face_info) {
   using F = FacePrefetch<N, EPB>;
   constexpr int N2 = Shape<N>::N2, NF = F::NF;
-  if (ps < F::PF) {
-    link = pf.link[ps < F::PF ? ps : 0];
-    info = pf.info[ps < F::PF ? ps : 0];
-    return;
-  }
-  const int fg = t + ps * F::GB;
-  link = -1;
-  info = 0;
-  const int es = EPB == 1 ? 0 : fg / NF;
-  if (fg < EPB * NF && es < n_valid) {
-    const int fid = fg - es * NF;
-    const int f = fid / N2, ab = fid - f * N2;
-    const size_t e = (size_t)(e0 + es);
-    link = nbr[(e * 6 + f) * N2 + ab];
-    info = face_info[e * 6 + f];
+#pragma unroll
+  for (int ps = FROM; ps < TO; ++ps) {
+    const int fg = t + ps * F::GB;
+    const int es = EPB == 1 ? 0 : fg / NF;
+    const bool valid = fg < EPB * NF && es < n_valid;
+    const int fid = valid ? fg - es * NF : 0;
+    const size_t e = (size_t)(e0 + (valid ? es : 0));
+    pf.link[ps] = nbr[e * NF + fid];
+    pf.info[ps] = face_info[e * 6 + fid / N2];
+    if (!valid) pf.link[ps] = -1;
   }
 }
 
 template <int N, int EPB = 1>
-__device__ __forceinline__ void face_prefetch(FacePrefetch<N, EPB>& pf, int e0, int n_valid, int t,
-                                              const double* __restrict__ u,
-                                              const int* __restrict__ nbr,
-                                              const int* __restrict__ face_info) {
-  using F = FacePrefetch<N, EPB>;
-  constexpr int N2 = Shape<N>::N2, NF = F::NF;
+__device__ __forceinline__ void face_prefetch_states(FacePrefetch<N, EPB>& pf,
+                                                     const double* __restrict__ u) {
 #pragma unroll
-  for (int ps = 0; ps < F::PF; ++ps) {
-    const int fg = t + ps * F::GB;
-    const int es = EPB == 1 ? 0 : fg / NF;
-    pf.link[ps] = -1;
-    pf.info[ps] = 0;
-    if (fg < EPB * NF && es < n_valid) {
-      const int fid = fg - es * NF;
-      const int f = fid / N2, ab = fid - f * N2;
-      const size_t e = (size_t)(e0 + es);
-      pf.link[ps] = nbr[(e * 6 + f) * N2 + ab];
-      pf.info[ps] = face_info[e * 6 + f];
-    }
-  }
+  for (int ps = 0; ps < FacePrefetch<N, EPB>::PF; ++ps) {
+    const double* ur = u + (size_t)(pf.link[ps] >= 0 ? pf.link[ps] : 0) * 6;
 #pragma unroll
-  for (int ps = 0; ps < F::PF; ++ps) {
-    const int link = pf.link[ps];
-#pragma unroll
-    for (int v = 0; v < 6; ++v) pf.ur[ps][v] = link >= 0 ? u[(size_t)link * 6 + v] : 0.0;
+    for (int v = 0; v < 6; ++v) pf.ur[ps][v] = ur[v];
   }
 }
 
@@ -399,33 +389,46 @@ struct FaceNormals {
 template <int N, typename T, int EPB = 1, typename G = T, bool LDS_CV = true>
 __device__ __forceinline__ void face_normals(FaceNormals<N, T, EPB>& fn, int e0, int n_valid, int t,
                                              const G* __restrict__ cv, const T* s_cv,
-                                             int cv_stride, const FacePrefetch<N, EPB>& pf,
-                                             const int* __restrict__ nbr,
-                                             const int* __restrict__ face_info) {
-  constexpr int N3 = Shape<N>::N3;
+                                             int cv_stride, const FacePrefetch<N, EPB>& pf) {
+  constexpr int N3 = Shape<N>::N3, PASSES = FacePrefetch<N, EPB>::PASSES;
+  // the vectors in memory of every pass are requested before any is waited
+  // for: the primary's on a secondary face (face_info: 8 | dp), else the own
+  // one, or with an LDS copy of it one fixed address whose value is not used
+  G m[PASSES][3];
 #pragma unroll
-  for (int ps = 0; ps < FacePrefetch<N, EPB>::PASSES; ++ps) {
-    int es, fid, f, d, node;
-    fn.n[ps][0] = fn.n[ps][1] = fn.n[ps][2] = T(0);
-    if (!face_node_of<N, EPB>(t, ps, n_valid, es, fid, f, d, node)) continue;
-    // face_info: 0 = primary side or boundary; 8 | dp = secondary side of an
-    // interface whose primary face direction is dp
-    int link, info;
-    face_link<N, EPB>(pf, e0, n_valid, t, ps, nbr, face_info, link, info);
-    if (info == 0) {
-      const T sgn = (f % 2 == 0) ? T(-1) : T(1);
-      const size_t e = (size_t)(e0 + es);
+  for (int ps = 0; ps < PASSES; ++ps) {
+    int es = 0, fid = 0, f = 0, d = 0, node = 0;
+    const bool valid = face_node_of<N, EPB>(t, ps, n_valid, es, fid, f, d, node);
+    const int info = pf.info[ps], link = pf.link[ps];
+    size_t at = (size_t)e0 * (9 * N3);
+    if (valid && info != 0) {
+      const int le = link / N3;
+      at = ((size_t)le * 9 + 3 * ((info & 7) >> 1)) * N3 + (link - le * N3);
+    } else if (valid && !LDS_CV) {
+      at = ((size_t)(e0 + es) * 9 + 3 * d) * N3 + node;
+    }
+    const G* jp = cv + at;
 #pragma unroll
-      for (int c = 0; c < 3; ++c)
-        if constexpr (LDS_CV) fn.n[ps][c] = sgn * s_cv[es * cv_stride + (3 * d + c) * N3 + node];
-        else fn.n[ps][c] = sgn * T(cv[(e * 9 + 3 * d + c) * N3 + node]);
-    } else {
-      const int dp = info & 7;
-      const T sgn = (dp % 2 == 0) ? T(1) : T(-1);  // minus the primary's outward normal
-      const int le = link / N3, ln = link - le * N3;
-      const G* jp = cv + ((size_t)le * 9 + 3 * (dp / 2)) * N3 + ln;
+    for (int c = 0; c < 3; ++c) m[ps][c] = jp[c * N3];
+  }
 #pragma unroll
-      for (int c = 0; c < 3; ++c) fn.n[ps][c] = sgn * T(jp[c * N3]);
+  for (int ps = 0; ps < PASSES; ++ps) {
+    int es = 0, fid = 0, f = 0, d = 0, node = 0;
+    face_node_of<N, EPB>(t, ps, n_valid, es, fid, f, d, node);
+    const int info = pf.info[ps];
+    const bool own = info == 0;
+    // outward of the own element: minus the primary's outward normal on a
+    // secondary face
+    const int side = own ? f : (info & 7) ^ 1;
+    const T sgn = (side % 2 == 0) ? T(-1) : T(1);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      T v = T(m[ps][c]);
+      if constexpr (LDS_CV) {
+        const T o = s_cv[es * cv_stride + (3 * d + c) * N3 + node];  // read on every lane
+        v = own ? o : v;
+      }
+      fn.n[ps][c] = sgn * v;
     }
   }
 }
@@ -436,8 +439,7 @@ __device__ __forceinline__ void face_normals(FaceNormals<N, T, EPB>& fn, int e0,
 template <int N, typename T, int EPB = 1>
 __device__ __forceinline__ void face_fluxes_to_lds(
     const E3Params& q, int e0, int n_valid, int t, double inv_w, const double* __restrict__ u,
-    const FacePrefetch<N, EPB>& pf, const FaceNormals<N, T, EPB>& fn,
-    const int* __restrict__ nbr, const int* __restrict__ face_info, int surf, int snc,
+    const FacePrefetch<N, EPB>& pf, const FaceNormals<N, T, EPB>& fn, int surf, int snc,
     const Background& bg, const T* s_w_all, int w_stride, const double* s_pb_all,
     T* s_sf_all, int sf_stride) {
   constexpr int N2 = Shape<N>::N2, N3 = Shape<N>::N3, NF = 6 * N2;
@@ -466,8 +468,7 @@ __device__ __forceinline__ void face_fluxes_to_lds(
 #pragma unroll
       for (int v = 0; v < 6; ++v) uo[v] = u[gn * 6 + v];
     }
-    int link, info;
-    face_link<N, EPB>(pf, e0, n_valid, t, ps, nbr, face_info, link, info);
+    const int link = pf.link[ps];
     const T n0 = fn.n[ps][0], n1 = fn.n[ps][1], n2 = fn.n[ps][2];
     double ur[6];
     if (link >= 0) {
@@ -562,14 +563,11 @@ struct NodeFields {
 };
 
 template <int N, int VOL, int NC, typename T>
-__device__ __forceinline__ void node_fields_to_lds(const E3Params& q, const double* __restrict__ u,
-                                                   size_t gnode, int t, T* s_w, double* s_phi,
-                                                   double* s_pb, const Background& bg) {
+__device__ __forceinline__ void node_fields_to_lds(const E3Params& q, const double* uo, int t,
+                                                   T* s_w, double* s_phi, double* s_pb,
+                                                   const Background& bg) {
   constexpr int N3 = Shape<N>::N3;
   constexpr bool MIXED = NodeFields<VOL, NC, T>::MIXED;
-  double uo[6];
-#pragma unroll
-  for (int v = 0; v < 6; ++v) uo[v] = u[gnode * 6 + v];
   // primitives (pressure from total minus kinetic energy) in FP64
   const Prim<double> w = cons2prim(q, uo);
   s_w[0 * N3 + t] = T(w.rho); s_w[1 * N3 + t] = T(w.v1); s_w[2 * N3 + t] = T(w.v2);
@@ -610,20 +608,46 @@ __device__ __forceinline__ FastPrim<T> load_fast_prim(const T* s_w, int node, co
   return l;
 }
 
-// after the volume terms (acc, acc_nc) and the lifted face fluxes (s_sf) are
-// complete: surface integral, -1/J, sources, then du or the RK update
-template <int N, typename T, bool KAHAN>
-__device__ __forceinline__ void stage_epilogue(
-    const Acc<T, KAHAN>* acc, const Acc<T, KAHAN>* acc_nc, const T* s_sf, int ti, int tj, int tk,
-    int e, size_t gnode, const double* __restrict__ u, double* __restrict__ out,
-    double* __restrict__ kreg, const double* __restrict__ invJ, int mode, double rk_a,
-    double rk_dt, double rk_b, double coriolis, const Background& bg, double* un) {
-  constexpr int NV = 6, N2 = Shape<N>::N2, N3 = Shape<N>::N3;
-  double du[NV];
+// the volume terms of one node: f# plus half the gravity term
+template <typename T, bool KAHAN>
+__device__ __forceinline__ void volume_sum(const Acc<T, KAHAN>* acc, const Acc<T, KAHAN>* acc_nc,
+                                           double* du) {
   du[0] = double(acc[0].value());
 #pragma unroll
   for (int v = 1; v < 5; ++v)
     du[v] = double(acc[v].value()) + 0.5 * double(acc_nc[v - 1].value());
+}
+
+// what the node's update reads from memory besides its state: 1/J and, in an
+// RK stage, the register
+struct NodeRest {
+  double invJ, k[5];
+};
+template <int N>
+__device__ __forceinline__ NodeRest load_rest(int e, int tl, const double* __restrict__ invJ,
+                                              const double* __restrict__ kreg, int mode) {
+  constexpr int N3 = Shape<N>::N3;
+  NodeRest r;
+  r.invJ = invJ[(size_t)e * N3 + tl];
+  if (mode != 0) {
+#pragma unroll
+    for (int v = 0; v < 5; ++v) r.k[v] = kreg[((size_t)e * 5 + v) * N3 + tl];
+  }
+  return r;
+}
+
+// after the volume terms (vol[5]) and the lifted face fluxes (s_sf) are
+// complete: surface integral, -1/J, sources, then du or the RK update
+template <int N, typename T>
+__device__ __forceinline__ void stage_epilogue(
+    const double* vol, const T* s_sf, int ti, int tj, int tk, int e, size_t gnode,
+    const double* uo, double* __restrict__ out, double* __restrict__ kreg,
+    const NodeRest& rest, int mode, double rk_a, double rk_dt, double rk_b, double coriolis,
+    const Background& bg, double* un) {
+  constexpr int NV = 6, N2 = Shape<N>::N2, N3 = Shape<N>::N3;
+  double du[NV];
+#pragma unroll
+  for (int v = 0; v < 5; ++v) du[v] = vol[v];
   du[5] = 0.0;
   constexpr int NF = 6 * N2;
 #pragma unroll
@@ -638,12 +662,9 @@ __device__ __forceinline__ void stage_epilogue(
 #pragma unroll
     for (int v = 0; v < NV; ++v) du[v] += double(s_sf[v * NF + fid]);
   }
-  const double fac = -invJ[gnode];
+  const double fac = -rest.invJ;
 #pragma unroll
   for (int v = 0; v < NV; ++v) du[v] *= fac;
-  double uo[NV];  // read again rather than kept live through the volume phase
-#pragma unroll
-  for (int v = 0; v < NV; ++v) uo[v] = u[gnode * NV + v];
   if (bg.on) {  // tendency of the hydrostatic background, computed in FP64
     du[1] += double(bg.B[gnode * 3 + 0]);
     du[2] += double(bg.B[gnode * 3 + 1]);
@@ -664,7 +685,7 @@ __device__ __forceinline__ void stage_epilogue(
     double* kn_ = kreg + (size_t)e * ((NV - 1) * N3) + (gnode - (size_t)e * N3);
 #pragma unroll
     for (int v = 0; v < NV - 1; ++v) {
-      const double kn = rk_a * kn_[v * N3] + rk_dt * du[v];
+      const double kn = rk_a * rest.k[v] + rk_dt * du[v];
       kn_[v * N3] = kn;
       un[v] = uo[v] + rk_b * kn;
       out[gnode * NV + v] = un[v];
@@ -738,6 +759,8 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
   const bool active = t < N3;
   const int ti = t % N, tj = (t / N) % N, tk = t / N2;
   const size_t gnode = (size_t)e * N3 + t;
+  FacePrefetch<N> pf;
+  face_links<N, 1, 0, FacePrefetch<N>::PASSES>(pf, e, 1, t, nbr, face_info);
   if (t < N * N) s_ds[t] = T(dst.ds[t]);
   if (t < P) {
     int qq = t, a = 0;
@@ -745,10 +768,13 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
     s_pa[t] = (unsigned char)a;
     s_pm[t] = (unsigned char)(a + 1 + qq);
   }
-  if (active) node_fields_to_lds<N, VOL, NC, T>(q, u, gnode, t, s_w, s_phi, s_pb, bg);
-
-  FacePrefetch<N> pf;
-  face_prefetch<N>(pf, e, 1, t, u, nbr, face_info);
+  face_prefetch_states<N>(pf, u);
+  if (active) {
+    double uo[6];
+#pragma unroll
+    for (int v = 0; v < 6; ++v) uo[v] = u[gnode * 6 + v];
+    node_fields_to_lds<N, VOL, NC, T>(q, uo, t, s_w, s_phi, s_pb, bg);
+  }
 
   Acc<T, KAHAN> acc[5], acc_nc[4];
   for (int d = 0; d < 3; ++d) {
@@ -820,15 +846,22 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
     }
   }
   FaceNormals<N, T> fn;
-  face_normals<N, T, 1, T, false>(fn, e, 1, t, cv, nullptr, 0, pf, nbr, face_info);
+  face_normals<N, T, 1, T, false>(fn, e, 1, t, cv, nullptr, 0, pf);
   __syncthreads();  // pair terms consumed; the buffer now takes the face fluxes
-  face_fluxes_to_lds<N, T>(q, e, 1, t, inv_w, u, pf, fn, nbr, face_info, surf, snc, bg, s_w, 0,
+  face_fluxes_to_lds<N, T>(q, e, 1, t, inv_w, u, pf, fn, surf, snc, bg, s_w, 0,
                            s_pb, s_fl, 0);
   __syncthreads();
   double un[6];
-  if (active)
-    stage_epilogue<N, T, KAHAN>(acc, acc_nc, s_fl, ti, tj, tk, e, gnode, u, out, kreg, invJ, mode,
-                                rk_a, res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
+  if (active) {
+    double vol[5];
+    volume_sum(acc, acc_nc, vol);
+    double uo[6];
+#pragma unroll
+    for (int v = 0; v < 6; ++v) uo[v] = u[gnode * 6 + v];
+    stage_epilogue<N, T>(vol, s_fl, ti, tj, tk, e, gnode, uo, out, kreg,
+                         load_rest<N>(e, t, invJ, kreg, mode), mode, rk_a,
+                         res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
+  }
   if (res.speed_partial) {
     __shared__ double s_red[B / 64][3];
     element_speed<N>(q, active, un, res.cv64, invJ, gnode, t, e, 1, s_red, res.speed_partial);
@@ -867,7 +900,7 @@ void e3_stage_direct(
   __shared__ double s_phi_all[EPB][MIXED ? N3 : 1];
   __shared__ double s_pb_all[EPB][MIXED ? N3 : 1];
   __shared__ T s_buf_all[EPB][BUF];  // contravariant vectors [9][n^3], later face fluxes [6][6 n^2]
-  __shared__ T s_ds[N * N];
+  __shared__ T s_ds[N * N + 1];  // and a slot for the lanes past the table
 
   if constexpr (!MIXED) bg.on = 0;
   const int n_groups = (n_elements + EPB - 1) / EPB;
@@ -886,14 +919,29 @@ void e3_stage_direct(
   double* s_phi = s_phi_all[es];
   double* s_pb = s_pb_all[es];
   T* s_buf = s_buf_all[es];
-  if (t < N * N) s_ds[t] = T(dst.ds[t]);
-  if (active) {
-    node_fields_to_lds<N, VOL, NC, T>(q, u, gnode, tl, s_w, s_phi, s_pb, bg);
-#pragma unroll
-    for (int c = 0; c < 9; ++c) s_buf[c * N3 + tl] = T(cv[((size_t)e * 9 + c) * N3 + tl]);
-  }
+  // every input is requested before any is waited for (a lane without a node
+  // reads the group's first one): the links, the own state, the vectors and
+  // Dsplit, then, when the links are here, the neighbours' states
   FacePrefetch<N, EPB> pf;
-  face_prefetch<N, EPB>(pf, e0, n_valid, t, u, nbr, face_info);
+  face_links<N, EPB, 0, FacePrefetch<N, EPB>::PF>(pf, e0, n_valid, t, nbr, face_info);
+  {
+    const size_t ge = active ? (size_t)e : (size_t)e0;
+    const int gl = active ? tl : 0;
+    double uo[6];
+    G ja[9];
+#pragma unroll
+    for (int v = 0; v < 6; ++v) uo[v] = u[(ge * N3 + gl) * 6 + v];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) ja[c] = cv[(ge * 9 + c) * N3 + gl];
+    const double ds = dst.ds[t < N * N ? t : 0];
+    face_prefetch_states<N, EPB>(pf, u);
+    s_ds[t < N * N ? t : N * N] = T(ds);
+    // lanes without a node form the first node's fields once more and store
+    // the same values: no branch, below which the compiler would sink the loads
+    node_fields_to_lds<N, VOL, NC, T>(q, uo, gl, s_w, s_phi, s_pb, bg);
+#pragma unroll
+    for (int c = 0; c < 9; ++c) s_buf[c * N3 + gl] = T(ja[c]);
+  }
   __syncthreads();
 
   Acc<T, KAHAN> acc[5], acc_nc[4];
@@ -1025,16 +1073,33 @@ void e3_stage_direct(
       for (int v = 0; v < 4; ++v) acc_nc[v].scale(scn[v]);
     }
   }
+  // the links of the other passes, then the update's inputs, which arrive
+  // during the face phase
+  face_links<N, EPB, FacePrefetch<N, EPB>::PF, FacePrefetch<N, EPB>::PASSES>(pf, e0, n_valid, t,
+                                                                             nbr, face_info);
+  constexpr bool LATE = FacePrefetch<N, EPB>::PASSES > 1;
+  double vol[5];
+  NodeRest rest;
+  if (active) {
+    volume_sum(acc, acc_nc, vol);
+    if (!LATE) rest = load_rest<N>(e, tl, invJ, kreg, mode);
+  }
   FaceNormals<N, T, EPB> fn;
-  face_normals<N, T, EPB, G>(fn, e0, n_valid, t, cv, s_buf_all[0], BUF, pf, nbr, face_info);
+  face_normals<N, T, EPB, G>(fn, e0, n_valid, t, cv, s_buf_all[0], BUF, pf);
   __syncthreads();  // contravariant vectors consumed; the buffer takes the face fluxes
-  face_fluxes_to_lds<N, T, EPB>(q, e0, n_valid, t, inv_w, u, pf, fn, nbr, face_info, surf, snc, bg,
+  face_fluxes_to_lds<N, T, EPB>(q, e0, n_valid, t, inv_w, u, pf, fn, surf, snc, bg,
                                 s_w_all[0], NW * N3, s_pb_all[0], s_buf_all[0], BUF);
+  double uo[6];  // read again rather than kept live through the phases before
+  if (active) {
+    if (LATE) rest = load_rest<N>(e, tl, invJ, kreg, mode);
+#pragma unroll
+    for (int v = 0; v < 6; ++v) uo[v] = u[gnode * 6 + v];
+  }
   __syncthreads();
   double un[6];
   if (active)
-    stage_epilogue<N, T, KAHAN>(acc, acc_nc, s_buf, ti, tj, tk, e, gnode, u, out, kreg, invJ, mode,
-                                rk_a, res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
+    stage_epilogue<N, T>(vol, s_buf, ti, tj, tk, e, gnode, uo, out, kreg, rest, mode, rk_a,
+                         res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
   if (res.speed_partial) {
     __shared__ double s_red[EPB * BE / 64][3];
     element_speed<N, EPB>(q, active, un, res.cv64, invJ, gnode, t, e0, n_valid, s_red,
