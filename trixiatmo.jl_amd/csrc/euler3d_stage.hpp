@@ -920,13 +920,13 @@ void e3_stage_direct(
   double* s_pb = s_pb_all[es];
   T* s_buf = s_buf_all[es];
   // every input is requested before any is waited for (a lane without a node
-  // reads the group's first one): the links, the own state, the vectors and
+  // reads its element's first one): the links, the own state, the vectors and
   // Dsplit, then, when the links are here, the neighbours' states
   FacePrefetch<N, EPB> pf;
   face_links<N, EPB, 0, FacePrefetch<N, EPB>::PF>(pf, e0, n_valid, t, nbr, face_info);
   {
-    const size_t ge = active ? (size_t)e : (size_t)e0;
-    const int gl = active ? tl : 0;
+    const size_t ge = es < n_valid ? (size_t)e : (size_t)e0;
+    const int gl = tl < N3 ? tl : 0;
     double uo[6];
     G ja[9];
 #pragma unroll
@@ -936,8 +936,9 @@ void e3_stage_direct(
     const double ds = dst.ds[t < N * N ? t : 0];
     face_prefetch_states<N, EPB>(pf, u);
     s_ds[t < N * N ? t : N * N] = T(ds);
-    // lanes without a node form the first node's fields once more and store
-    // the same values: no branch, below which the compiler would sink the loads
+    // lanes without a node form their slot's first node's fields once more and
+    // store the same values: no branch, below which the compiler would sink the
+    // loads
     node_fields_to_lds<N, VOL, NC, T>(q, uo, gl, s_w, s_phi, s_pb, bg);
 #pragma unroll
     for (int c = 0; c < 9; ++c) s_buf[c * N3 + gl] = T(ja[c]);
