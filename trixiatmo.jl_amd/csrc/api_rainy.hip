@@ -453,9 +453,9 @@ int atmo_mlp_get_params(atmo_mlp* m, float* params) {
 int atmo_mlp_loss_grad(atmo_mlp* m, const float* x, const float* y, int64_t n, float* loss,
                        float* grad) {
   if (!m || !x || !y || n < 1) return fail(m ? &m->err : nullptr, ATMO_ERR_INVALID, "bad arguments");
-  const int64_t blocks = (n + 63) / 64;
-  if (blocks > (int64_t)1 << 24) return fail(&m->err, ATMO_ERR_INVALID, "too many samples");
-  int rc = mlp_ensure_partials(m, blocks);
+  if ((n + 63) / 64 > (int64_t)1 << 24)
+    return fail(&m->err, ATMO_ERR_INVALID, "too many samples");
+  int rc = mlp_ensure_partials(m, mlp_grad_blocks(n));
   if (rc != ATMO_OK) return rc;
   const int nb = mlp_launch_loss_grad(m->d_params, m->d_norm, x, y, nullptr, 0, n, m->d_partial,
                                       m->stream);
@@ -476,14 +476,13 @@ int atmo_mlp_train(atmo_mlp* m, const float* x, const float* y, const int32_t* p
     return fail(m ? &m->err : nullptr, ATMO_ERR_INVALID, "bad arguments");
   if ((int64_t)batch * n_batches > n)
     return fail(&m->err, ATMO_ERR_INVALID, "batches exceed the samples");
-  int rc = mlp_ensure_partials(m, (batch + 63) / 64);
+  int rc = mlp_ensure_partials(m, mlp_grad_blocks(batch));
   if (rc != ATMO_OK) return rc;
   for (int b = 0; b < n_batches; ++b) {
     const int nb = mlp_launch_loss_grad(m->d_params, m->d_norm, x, y, perm, (int64_t)b * batch,
                                         batch, m->d_partial, m->stream);
-    mlp_launch_reduce(m->d_partial, nb, m->d_grad, m->stream);
-    mlp_launch_adam(m->d_params, m->d_m, m->d_v, m->d_grad, lr, 0.9f, 0.999f, 1e-8f, ++m->step,
-                    m->stream);
+    mlp_launch_reduce_adam(m->d_partial, nb, m->d_grad, m->d_params, m->d_m, m->d_v, lr, 0.9f,
+                           0.999f, 1e-8f, ++m->step, m->stream);
   }
   MLP_TRY(m, hipGetLastError());
   float g = 0.0f;

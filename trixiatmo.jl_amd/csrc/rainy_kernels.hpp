@@ -136,15 +136,18 @@ bool rainy_launch_integrals(const RainyLaunch& L, const double* w, double* parti
 void rainy_launch_newton(const RainyLaunch& L, double* u, const MlpView* mlp, int* iterations,
                          hipStream_t s);
 
-// MLP training: per-wave loss and gradient partials of samples
-// [offset, offset + count) (through `perm` when given), returning the number
-// of partials; their sum in a fixed order; Adam; forward in physical units
+// MLP training: loss and gradient partials of samples [offset, offset + count)
+// (through `perm` when given), one per workgroup, returning their number
+// (mlp_grad_blocks(count)); their sum in a fixed order, with or without the
+// Adam update from it; forward in physical units
+int mlp_grad_blocks(int64_t count);
 int mlp_launch_loss_grad(const float* params, const float* norm, const float* x, const float* y,
                          const int* perm, int64_t offset, int64_t count, float* partial,
                          hipStream_t s);
 void mlp_launch_reduce(const float* partial, int blocks, float* grad_loss, hipStream_t s);
-void mlp_launch_adam(float* params, float* m, float* v, const float* grad, float lr, float beta1,
-                     float beta2, float eps, int step, hipStream_t s);
+void mlp_launch_reduce_adam(const float* partial, int blocks, float* grad_loss, float* params,
+                            float* m, float* v, float lr, float beta1, float beta2, float eps,
+                            int step, hipStream_t s);
 void mlp_launch_forward(const float* params, const float* norm, const float* x, float* y,
                         int64_t n, hipStream_t s);
 // features of a rainy state: x = (rho, internal energy, total water), y = (T, q_v)
