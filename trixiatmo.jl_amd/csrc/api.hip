@@ -71,6 +71,16 @@ inline void face_ab(int dir, int i, int j, int k, int* a, int* b) {
 }  // namespace
 
 namespace atmo {
+bool alloc_result(atmo_handle* h, size_t n) {
+  void* p = nullptr;
+  if (hipHostMalloc(reinterpret_cast<void**>(&h->h_result), sizeof(double) * n,
+                    hipHostMallocDefault) != hipSuccess ||
+      hipHostGetDevicePointer(&p, h->h_result, 0) != hipSuccess)
+    return false;
+  h->d_result = static_cast<double*>(p);
+  return true;
+}
+
 void timer_begin(atmo_handle* h, int cls, TimerPair* tp) {
   tp->cls = cls;
   hipEventCreate(&tp->a);
@@ -607,7 +617,7 @@ int atmo_create(const atmo_config* cfg, const atmo_geometry3d* g, atmo_handle** 
       hipMalloc(&h->d_nbr, sizeof(int32_t) * nbr.size()) != hipSuccess ||
       hipMalloc(&h->d_face_info, sizeof(int32_t) * face_info.size()) != hipSuccess ||
       hipMalloc(&h->d_partial, sizeof(double) * 9 * (size_t)E) != hipSuccess ||
-      hipMalloc(&h->d_result, sizeof(double) * 16) != hipSuccess ||
+      !alloc_result(h, 16) ||
       (cfg->precision != ATMO_PREC_FP64 &&
        hipMalloc(&h->d_cv32, sizeof(float) * 9 * n3 * (size_t)E) != hipSuccess) ||
       (h->bg_on && (hipMalloc(&h->d_ubg, sb) != hipSuccess || hipMalloc(&h->d_dubg, sb) != hipSuccess ||
@@ -664,9 +674,10 @@ void atmo_destroy(atmo_handle* h) {
     hipEventDestroy(tp.b);
   }
   double* bufs[] = {h->d_u, h->d_u2, h->d_k, h->d_du, h->d_uio, h->d_duio,
-                    h->d_cv, h->d_invJ, h->d_partial, h->d_result};
+                    h->d_cv, h->d_invJ, h->d_partial};
   for (double* p : bufs)
     if (p) hipFree(p);
+  if (h->h_result) hipHostFree(h->h_result);
   if (h->d_nbr) hipFree(h->d_nbr);
   if (h->d_cv32) hipFree(h->d_cv32);
   if (h->d_ubg) hipFree(h->d_ubg);
@@ -766,7 +777,7 @@ int atmo_step(atmo_handle* h, double dt, int32_t n_steps) {
     // pairs of steps from a captured graph whose stages read dt from memory
     const int rc = ensure_e3_graph(h);
     if (rc != ATMO_OK) return rc;
-    launch_set_scalar(h->d_step_dt, dt, h->stream);
+    launch_fill(h->d_step_dt, dt, 1, h->stream);
     HIP_TRY(h, hipGetLastError());
     for (; done + 2 <= n_steps; done += 2) {
       HIP_TRY(h, hipGraphLaunch(h->e3_graph, h->stream));
@@ -802,9 +813,8 @@ int atmo_max_dt(atmo_handle* h, double cfl, double* dt) {
   e3_launch_reduction(L, 0, nullptr, h->d_partial, h->d_result, h->stream);
   if (h->timing) timer_end(h, &tp);
   HIP_TRY(h, hipGetLastError());
-  double mx = 0;
-  HIP_TRY(h, hipMemcpyAsync(&mx, h->d_result, sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
+  double mx = h->h_result[0];
   if (!std::isfinite(mx)) return fail(&h->err, ATMO_ERR_NONFINITE, "non-finite wave speed in state");
   if (mx < 5e-324) mx = 5e-324;
   *dt = cfl * (2.0 / (h->n * mx));  // max_dt (stepsize_dg2d.jl:43), then StepsizeCallback's cfl factor
@@ -827,8 +837,8 @@ int atmo_integrals(atmo_handle* h, int32_t fresh_rhs, double* out) {
   e3_launch_reduction(L, 1, h->du_valid ? h->d_du : nullptr, h->d_partial, h->d_result, h->stream);
   if (h->timing) timer_end(h, &tp);
   HIP_TRY(h, hipGetLastError());
-  HIP_TRY(h, hipMemcpyAsync(out, h->d_result, sizeof(double) * 9, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
+  std::memcpy(out, h->h_result, sizeof(double) * 9);
   return ATMO_OK;
 }
 

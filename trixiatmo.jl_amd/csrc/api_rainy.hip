@@ -162,9 +162,8 @@ int rainy_max_dt(atmo_handle* h, double cfl, double* dt) {
   if (h->timing) timer_end(h, &tp);
   if (!ok) return fail(&h->err, ATMO_ERR_INVALID, "no rainy kernel for this polydeg");
   HIP_TRY(h, hipGetLastError());
-  double mx = 0;
-  HIP_TRY(h, hipMemcpyAsync(&mx, h->d_result, sizeof(double), hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
+  const double mx = h->h_result[0];
   if (!std::isfinite(mx)) return fail(&h->err, ATMO_ERR_NONFINITE, "non-finite wave speed");
   *dt = cfl * (2.0 / (h->n * mx));  // max_dt (stepsize_dg2d.jl:43), then StepsizeCallback's cfl factor
   return ATMO_OK;
@@ -177,9 +176,8 @@ int rainy_integrals(atmo_handle* h, double* out) {
   if (!rainy_launch_integrals(L, h->d_dt_member, h->d_partial, h->d_result, h->stream))
     return fail(&h->err, ATMO_ERR_INVALID, "no rainy kernel for this polydeg");
   HIP_TRY(h, hipGetLastError());
-  HIP_TRY(h, hipMemcpyAsync(out, h->d_result, sizeof(double) * 9, hipMemcpyDeviceToHost,
-                            h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
+  std::memcpy(out, h->h_result, sizeof(double) * 9);
   return ATMO_OK;
 }
 
@@ -241,7 +239,7 @@ int atmo_rainy_create(const atmo_rainy_config* cfg, atmo_handle** out) {
       hipMalloc(&h->d_uio, sb) != hipSuccess || hipMalloc(&h->d_duio, sb) != hipSuccess ||
       hipMalloc(&h->d_dt_member, sizeof(double) * 16) != hipSuccess ||
       hipMalloc(&h->d_partial, sizeof(double) * 9 * (size_t)E) != hipSuccess ||
-      hipMalloc(&h->d_result, sizeof(double) * 16) != hipSuccess ||
+      !alloc_result(h, 16) ||
       hipMalloc(&h->d_stats, stat_bytes) != hipSuccess)
     return cleanup_fail(ATMO_ERR_DEVICE, "device allocation failed");
   if (hipMemcpy(h->d_dt_member, b.w.data(), sizeof(double) * n, hipMemcpyHostToDevice) !=

@@ -72,12 +72,13 @@ const double kB[5] = {1432997174477.0 / 9575080441755.0, 5161836677717.0 / 13612
                       2277821191437.0 / 14882151754819.0};
 
 // the 5 stage launches of n_steps CarpenterKennedy2N54 steps, time steps read
-// from d_dt_member
-int enqueue_steps(atmo_handle* h, int n_steps, double* speed_partial = nullptr) {
+// from d_dt_member or, with dt > 0, dt for every member
+int enqueue_steps(atmo_handle* h, int n_steps, double* speed_partial = nullptr, double dt = 0.0) {
   SweLaunch L = h->swe_base;
   L.mode = 1;
   L.k = h->d_k;
-  L.dt_member = h->d_dt_member;
+  L.dt_member = dt > 0.0 ? nullptr : h->d_dt_member;
+  L.rk_dt = dt;
   for (int s = 0; s < n_steps; ++s)
     for (int st = 0; st < 5; ++st) {
       L.u = h->d_u;
@@ -194,13 +195,9 @@ int swe_autotune(atmo_handle* h, double* ms_per_variant) {
 }
 
 int swe_step(atmo_handle* h, const double* dt_members, double dt, int n_steps) {
-  std::vector<double> dts;
-  if (!dt_members) {
-    dts.assign(h->n_members, dt);
-    dt_members = dts.data();
-  }
-  HIP_TRY(h, hipMemcpyAsync(h->d_dt_member, dt_members, sizeof(double) * h->n_members,
-                            hipMemcpyHostToDevice, h->stream));
+  if (dt_members)
+    HIP_TRY(h, hipMemcpyAsync(h->d_dt_member, dt_members, sizeof(double) * h->n_members,
+                              hipMemcpyHostToDevice, h->stream));
   if (!h->swe_tuned) {
     const int rc = swe_autotune(h, nullptr);
     if (rc != ATMO_OK) return rc;
@@ -209,14 +206,20 @@ int swe_step(atmo_handle* h, const double* dt_members, double dt, int n_steps) {
   if (!h->timing && n_steps >= 2) {
     int rc = ensure_graph(h);
     if (rc != ATMO_OK) return rc;
+    // one step size for all members goes by a kernel argument, here to the
+    // array that the graph's stages read
+    if (!dt_members) {
+      launch_fill(h->d_dt_member, dt, h->n_members, h->stream);
+      HIP_TRY(h, hipGetLastError());
+    }
     for (; done + 2 <= n_steps; done += 2) HIP_TRY(h, hipGraphLaunch(h->swe_graph, h->stream));
   }
   if (done < n_steps) {
-    const int rc = enqueue_steps(h, n_steps - done);
+    const int rc = enqueue_steps(h, n_steps - done, nullptr, dt_members ? 0.0 : dt);
     if (rc != ATMO_OK) return rc;
   }
   // the host copy of the time steps may go out of scope: finish the upload
-  HIP_TRY(h, hipStreamSynchronize(h->stream));
+  if (dt_members) HIP_TRY(h, hipStreamSynchronize(h->stream));
   h->du_valid = false;
   return ATMO_OK;
 }
@@ -231,10 +234,8 @@ int swe_max_dt(atmo_handle* h, double cfl, double* dt_members) {
   if (h->timing) timer_end(h, &tp);
   if (!ok) return fail(&h->err, ATMO_ERR_INVALID, "no covariant kernel for this polydeg");
   HIP_TRY(h, hipGetLastError());
-  std::vector<double> mx(h->n_members);
-  HIP_TRY(h, hipMemcpyAsync(mx.data(), h->d_result, sizeof(double) * h->n_members,
-                            hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
+  const double* mx = h->h_result;
   for (int m = 0; m < h->n_members; ++m) {
     if (!std::isfinite(mx[m])) return fail(&h->err, ATMO_ERR_NONFINITE, "non-finite wave speed");
     dt_members[m] = cfl * (2.0 / (h->n * mx[m]));  // max_dt (stepsize_dg2d.jl:70), then the cfl factor
@@ -256,8 +257,8 @@ int swe_integrals(atmo_handle* h, int fresh_rhs, double* out) {
                             h->stream))
     return fail(&h->err, ATMO_ERR_INVALID, "no covariant kernel for this polydeg");
   HIP_TRY(h, hipGetLastError());
-  HIP_TRY(h, hipMemcpyAsync(out, h->d_result, sizeof(double) * 3, hipMemcpyDeviceToHost, h->stream));
   HIP_TRY(h, hipStreamSynchronize(h->stream));
+  std::memcpy(out, h->h_result, sizeof(double) * 3);
   return ATMO_OK;
 }
 
@@ -547,7 +548,7 @@ int atmo_swe_create(const atmo_swe_config* cfg, const atmo_geometry2d* g, atmo_h
       hipMalloc(&h->d_member_first, sizeof(int32_t) * (M + 1)) != hipSuccess ||
       hipMalloc(&h->d_dt_member, sizeof(double) * (M + n)) != hipSuccess ||
       hipMalloc(&h->d_partial, sizeof(double) * 3 * (size_t)E) != hipSuccess ||
-      hipMalloc(&h->d_result, sizeof(double) * (M > 16 ? M : 16)) != hipSuccess)
+      !alloc_result(h, M > 16 ? M : 16))
     return cleanup_fail(ATMO_ERR_DEVICE, "device allocation failed");
   if ((!aux_on_device && hipMemcpy(h->d_aux, g->aux_node_vars, sizeof(double) * 26 * n2 * (size_t)E,
                                    hipMemcpyHostToDevice) != hipSuccess) ||

@@ -5,6 +5,7 @@
 
 #include "euler3d_kernels.hpp"
 #include "euler3d_physics.hpp"
+#include "handle.hpp"
 #include "speed_max.hpp"
 
 namespace atmo {
@@ -59,6 +60,7 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_max_speed(E3Params q, cons
 }
 
 // per element: integrals of mass, entropy, w(u).du and every conserved variable
+// (partial [9][elements])
 template <int N>
 __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_integrals(E3Params q, WeightTable wt,
                                                                const double* __restrict__ u,
@@ -99,30 +101,7 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_integrals(E3Params q, Weig
       for (int c = 0; c < K; ++c) s[c][t] += s[c][t + w];
     __syncthreads();
   }
-  if (t < K) partial[(size_t)e * K + t] = s[t][0];
-}
-
-// single-block reduction of partial[n_items * width] (op 0: sum, 1: max)
-__global__ __launch_bounds__(256) void reduce_columns(const double* __restrict__ partial,
-                                                      int n_items, int width, int op,
-                                                      double* __restrict__ result) {
-  __shared__ double s[256];
-  const int t = threadIdx.x;
-  for (int c = 0; c < width; ++c) {
-    double acc = op == 0 ? 0.0 : -1e300;
-    for (int i = t; i < n_items; i += 256) {
-      const double x = partial[(size_t)i * width + c];
-      acc = op == 0 ? acc + x : speed_max(acc, x);
-    }
-    s[t] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if (t < w) s[t] = op == 0 ? s[t] + s[t + w] : speed_max(s[t], s[t + w]);
-      __syncthreads();
-    }
-    if (t == 0) result[c] = s[0];
-    __syncthreads();
-  }
+  if (t < K) partial[(size_t)t * gridDim.x + e] = s[t][0];
 }
 
 template <int N>
@@ -156,9 +135,8 @@ bool e3_launch_reduction(const E3Launch& L, int which, const double* du, double*
     case 8: launch_red<8>(L, which, du, partial, s); break;
     default: return false;
   }
-  const int width = which == 0 ? 1 : 9;
-  hipLaunchKernelGGL(reduce_columns, dim3(1), dim3(256), 0, s, partial, L.n_elements, width,
-                     which == 0 ? 1 : 0, result);
+  if (which == 0) launch_reduce_max(partial, L.n_elements, 0.0, result, s);
+  else launch_sum_rows(partial, L.n_elements, 9, result, s);
   return true;
 }
 

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include "euler3d_physics.hpp"
+#include "handle.hpp"
 #include "rainy_flux.hpp"
 #include "rainy_kernels.hpp"
 #include "speed_max.hpp"
@@ -929,20 +930,6 @@ __global__ __launch_bounds__(64) void rainy_max_speed(RainyLaunch L, double* par
   if (t == 0) partial[e] = s1[0] + s2[0];
 }
 
-__global__ __launch_bounds__(256) void rainy_max_reduce(const double* partial, int n, double* out) {
-  __shared__ double s[256];
-  const int t = threadIdx.x;
-  double acc = 5e-324;
-  for (int i = t; i < n; i += 256) acc = speed_max(acc, partial[i]);
-  s[t] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) s[t] = speed_max(s[t], s[t + w]);
-    __syncthreads();
-  }
-  if (t == 0) out[0] = s[0];
-}
-
 template <int N>
 __global__ __launch_bounds__(64) void rainy_integrals(RainyLaunch L, const double* w,
                                                       double* partial) {
@@ -967,25 +954,7 @@ __global__ __launch_bounds__(64) void rainy_integrals(RainyLaunch L, const doubl
       for (int v = 0; v < NV; ++v) s[v][t] += s[v][t + k];
     __syncthreads();
   }
-  if (t < NV) partial[(size_t)e * NV + t] = s[t][0];
-}
-
-__global__ __launch_bounds__(256) void rainy_sum_columns(const double* partial, int n_items,
-                                                         double* out) {
-  __shared__ double s[256];
-  const int t = threadIdx.x;
-  for (int c = 0; c < NV; ++c) {
-    double acc = 0.0;
-    for (int i = t; i < n_items; i += 256) acc += partial[(size_t)i * NV + c];
-    s[t] = acc;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-      if (t < k) s[t] += s[t + k];
-      __syncthreads();
-    }
-    if (t == 0) out[c] = s[0];
-    __syncthreads();
-  }
+  if (t < NV) partial[(size_t)t * gridDim.x + e] = s[t][0];
 }
 
 __global__ __launch_bounds__(256) void rainy_newton_kernel(RainyLaunch L, double* u,
@@ -1091,7 +1060,7 @@ bool rainy_launch_max_speed(const RainyLaunch& L, double* partial, double* out, 
     break;
   ATMO_RAINY_SWITCH(ATMO_CASE)
 #undef ATMO_CASE
-  hipLaunchKernelGGL(rainy_max_reduce, dim3(1), dim3(256), 0, s, partial, L.n_elements, out);
+  launch_reduce_max(partial, L.n_elements, 5e-324, out, s);
   return true;
 }
 
@@ -1103,7 +1072,7 @@ bool rainy_launch_integrals(const RainyLaunch& L, const double* w, double* parti
     break;
   ATMO_RAINY_SWITCH(ATMO_CASE)
 #undef ATMO_CASE
-  hipLaunchKernelGGL(rainy_sum_columns, dim3(1), dim3(256), 0, s, partial, L.n_elements, out);
+  launch_sum_rows(partial, L.n_elements, NV, out, s);
   return true;
 }
 

@@ -55,19 +55,20 @@ __global__ void step_control_kernel(const double* __restrict__ max_speed, int M,
   if (m < M) step_control_kernel_body(max_speed[m], m, M, n, clock, dt);
 }
 
-// the same for one member whose maximum speed is the maximum over per-element
-// partials (written by the last stage of the step just taken)
-__global__ __launch_bounds__(1024) void step_control_reduce_kernel(const double* __restrict__ partial,
-                                                                   int n_items, int n,
-                                                                   double* clock, double* dt) {
-  __shared__ double s[1024 / 64];
+// maximum over partial[from .. to) of a workgroup of B lanes, on every lane of
+// its first wave: eight independent loads in flight per lane, then their
+// maximum (one load at a time waited for each: 33 us for 32,768 partials
+// against 6)
+template <int B>
+__device__ __forceinline__ double block_max(const double* __restrict__ partial, int from, int to,
+                                            double floor) {
+  __shared__ double s[B / 64];
   const int t = threadIdx.x;
-  double m = 0.0;
-  // eight independent loads in flight per lane, then their maximum
-  for (int i0 = t; i0 < n_items; i0 += 8 * 1024) {
+  double m = floor;
+  for (int i0 = from + t; i0 < to; i0 += 8 * B) {
     double v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = i0 + k * 1024 < n_items ? partial[i0 + k * 1024] : 0.0;
+    for (int k = 0; k < 8; ++k) v[k] = i0 + k * B < to ? partial[i0 + k * B] : floor;
 #pragma unroll
     for (int k = 0; k < 8; ++k) m = speed_max(m, v[k]);
   }
@@ -75,12 +76,17 @@ __global__ __launch_bounds__(1024) void step_control_reduce_kernel(const double*
   for (int o = 32; o > 0; o >>= 1) m = speed_max(m, __shfl_xor(m, o, 64));
   if ((t & 63) == 0) s[t >> 6] = m;
   __syncthreads();
-  if (t == 0) {
-    for (int w = 1; w < 1024 / 64; ++w) m = speed_max(m, s[w]);
-    s[0] = m;
-  }
-  __syncthreads();
-  if (t == 0) step_control_kernel_body(s[0], 0, 1, n, clock, dt);
+  for (int w = 0; w < B / 64; ++w) m = speed_max(m, s[w]);
+  return m;
+}
+
+// the same for one member whose maximum speed is the maximum over per-element
+// partials (written by the last stage of the step just taken)
+__global__ __launch_bounds__(1024) void step_control_reduce_kernel(const double* __restrict__ partial,
+                                                                   int n_items, int n,
+                                                                   double* clock, double* dt) {
+  const double m = block_max<1024>(partial, 0, n_items, 0.0);
+  if (threadIdx.x == 0) step_control_kernel_body(m, 0, 1, n, clock, dt);
 }
 
 // one workgroup per ensemble member: its maximum speed is the maximum over the
@@ -88,25 +94,48 @@ __global__ __launch_bounds__(1024) void step_control_reduce_kernel(const double*
 __global__ __launch_bounds__(256) void step_control_members_reduce_kernel(
     const double* __restrict__ partial, const int* __restrict__ member_first, int M, int n,
     double* clock, double* dt) {
-  __shared__ double s[256 / 64];
-  const int m = blockIdx.x, t = threadIdx.x;
-  double mx = 0.0;
-  const int e1 = member_first[m + 1];
-  for (int e0 = member_first[m] + t; e0 < e1; e0 += 8 * 256) {
+  const int m = blockIdx.x;
+  const double mx = block_max<256>(partial, member_first[m], member_first[m + 1], 0.0);
+  if (threadIdx.x == 0) step_control_kernel_body(mx, m, M, n, clock, dt);
+}
+
+__global__ __launch_bounds__(1024) void reduce_max_kernel(const double* __restrict__ partial, int n,
+                                                          double floor, double* result) {
+  const double m = block_max<1024>(partial, 0, n, floor);
+  if (threadIdx.x == 0) result[0] = m;
+}
+
+__global__ __launch_bounds__(256) void member_max_kernel(const double* __restrict__ partial,
+                                                         const int* __restrict__ member_first,
+                                                         double* result) {
+  const int m = blockIdx.x;
+  const double mx = block_max<256>(partial, member_first[m], member_first[m + 1], 5e-324);
+  if (threadIdx.x == 0) result[m] = mx;
+}
+
+// one workgroup per row, the sum in a fixed order (one workgroup for all nine
+// rows of 5,184 partials, 256 lanes and a load at a time: 40 us; this: 4)
+__global__ __launch_bounds__(1024) void sum_rows_kernel(const double* __restrict__ partial, int n,
+                                                        double* result) {
+  __shared__ double s[1024 / 64];
+  const int t = threadIdx.x;
+  const double* p = partial + (size_t)blockIdx.x * n;
+  double a = 0.0;
+  for (int i0 = t; i0 < n; i0 += 8 * 1024) {
     double v[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) v[k] = e0 + k * 256 < e1 ? partial[e0 + k * 256] : 0.0;
+    for (int k = 0; k < 8; ++k) v[k] = i0 + k * 1024 < n ? p[i0 + k * 1024] : 0.0;
 #pragma unroll
-    for (int k = 0; k < 8; ++k) mx = speed_max(mx, v[k]);
+    for (int k = 0; k < 8; ++k) a += v[k];
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) mx = speed_max(mx, __shfl_xor(mx, o, 64));
-  if ((t & 63) == 0) s[t >> 6] = mx;
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+  if ((t & 63) == 0) s[t >> 6] = a;
   __syncthreads();
-  if (t == 0) {
-    for (int w = 1; w < 256 / 64; ++w) mx = speed_max(mx, s[w]);
-    step_control_kernel_body(mx, m, M, n, clock, dt);
-  }
+  if (t != 0) return;
+  a = s[0];
+  for (int w = 1; w < 1024 / 64; ++w) a += s[w];
+  result[blockIdx.x] = a;
 }
 
 }  // namespace
@@ -125,13 +154,28 @@ void launch_step_control(const double* max_speed, int n_members, int n, double* 
 }
 
 namespace {
-__global__ void set_scalar_kernel(double* ptr, double value) {
-  if (threadIdx.x == 0) *ptr = value;
+__global__ void fill_kernel(double* ptr, double value, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) ptr[i] = value;
 }
 }  // namespace
 
-void launch_set_scalar(double* ptr, double value, hipStream_t s) {
-  hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(64), 0, s, ptr, value);
+void launch_fill(double* ptr, double value, int n, hipStream_t s) {
+  hipLaunchKernelGGL(fill_kernel, dim3((n + 63) / 64), dim3(64), 0, s, ptr, value, n);
+}
+
+void launch_reduce_max(const double* partial, int n, double floor, double* result, hipStream_t s) {
+  hipLaunchKernelGGL(reduce_max_kernel, dim3(1), dim3(1024), 0, s, partial, n, floor, result);
+}
+
+void launch_member_max(const double* partial, const int* member_first, int n_members,
+                       double* result, hipStream_t s) {
+  hipLaunchKernelGGL(member_max_kernel, dim3(n_members), dim3(256), 0, s, partial, member_first,
+                     result);
+}
+
+void launch_sum_rows(const double* partial, int n, int width, double* result, hipStream_t s) {
+  hipLaunchKernelGGL(sum_rows_kernel, dim3(width), dim3(1024), 0, s, partial, n, result);
 }
 
 void launch_step_control_reduce(const double* partial, int n_items, int n, double* clock,

@@ -42,6 +42,7 @@
 #include <hip/hip_runtime.h>
 
 #include "euler3d_physics.hpp"
+#include "handle.hpp"
 #include "swe_kernels.hpp"
 #include "speed_max.hpp"
 
@@ -556,22 +557,6 @@ __global__ __launch_bounds__(64) void swe_max_speed(SweLaunch L, double* partial
   if (t == 0) partial[e] = s1[0] + s2[0];
 }
 
-// per-member maximum over its elements
-__global__ void swe_member_max(const double* partial, const int* member_first, int n_members,
-                               double* out) {
-  const int m = blockIdx.x, t = threadIdx.x;
-  __shared__ double s[256];
-  double acc = 5e-324;
-  for (int e = member_first[m] + t; e < member_first[m + 1]; e += 256) acc = speed_max(acc, partial[e]);
-  s[t] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) s[t] = speed_max(s[t], s[t + w]);
-    __syncthreads();
-  }
-  if (t == 0) out[m] = s[0];
-}
-
 namespace {
 
 template <int N, int WAVES, bool SPLIT>
@@ -648,8 +633,7 @@ bool swe_launch_member_max_speed(const SweLaunch& L, double* partial, const int*
       return false;
   }
 #undef ATMO_SWE_CASE
-  hipLaunchKernelGGL(swe_member_max, dim3(n_members), dim3(256), 0, s, partial, member_first,
-                     n_members, out);
+  launch_member_max(partial, member_first, n_members, out, s);
   return true;
 }
 
@@ -700,24 +684,7 @@ __global__ __launch_bounds__(64) void swe_integrals_kernel(SweLaunch L, const do
       for (int c = 0; c < 3; ++c) s[c][t] += s[c][t + k];
     __syncthreads();
   }
-  if (t < 3) partial[(size_t)e * 3 + t] = s[t][0];
-}
-
-__global__ void swe_sum_columns(const double* partial, int n_items, double* out) {
-  __shared__ double s[256];
-  const int t = threadIdx.x;
-  for (int c = 0; c < 3; ++c) {
-    double acc = 0.0;
-    for (int i = t; i < n_items; i += 256) acc += partial[(size_t)i * 3 + c];
-    s[t] = acc;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-      if (t < k) s[t] += s[t + k];
-      __syncthreads();
-    }
-    if (t == 0) out[c] = s[0];
-    __syncthreads();
-  }
+  if (t < 3) partial[(size_t)t * gridDim.x + e] = s[t][0];
 }
 
 bool swe_launch_integrals(const SweLaunch& L, const double* du, const double* w, double* partial,
@@ -739,7 +706,7 @@ bool swe_launch_integrals(const SweLaunch& L, const double* du, const double* w,
       return false;
   }
 #undef ATMO_SWE_CASE
-  hipLaunchKernelGGL(swe_sum_columns, dim3(1), dim3(256), 0, s, partial, L.n_elements, out);
+  launch_sum_rows(partial, L.n_elements, 3, out, s);
   return true;
 }
 
