@@ -196,13 +196,18 @@ __device__ __forceinline__ Prim<T> cons2prim(const E3Params& q, const T* u) {
 __device__ __forceinline__ void node_scaled_speeds(const E3Params& q, const double* uu,
                                                    const double* ja, int stride, double ij_abs,
                                                    double l[3]) {
-  const Prim<double> w = cons2prim(q, uu);
-  const double c = sqrt(q.gamma * w.p / w.rho);
-  const double a1 = fabs(w.v1) + c, a2 = fabs(w.v2) + c, a3 = fabs(w.v3) + c;
+#pragma clang fp contract(off)
+  // every fused multiply-add written out: the kernels that inline this get the
+  // same bits
+  const double inv = div_nr(1.0, uu[0]);
+  const double v1 = uu[1] * inv, v2 = uu[2] * inv, v3 = uu[3] * inv;
+  const double p = q.gm1 * fma(-0.5, fma(uu[1], v1, fma(uu[2], v2, uu[3] * v3)), uu[4]);
+  const double c = sqrt(q.gamma * p / uu[0]);
+  const double a1 = fabs(v1) + c, a2 = fabs(v2) + c, a3 = fabs(v3) + c;
 #pragma unroll
   for (int d = 0; d < 3; ++d)
-    l[d] = ij_abs * fabs(ja[(3 * d) * stride] * a1 + ja[(3 * d + 1) * stride] * a2 +
-                         ja[(3 * d + 2) * stride] * a3);
+    l[d] = ij_abs * fabs(fma(ja[(3 * d) * stride], a1,
+                             fma(ja[(3 * d + 1) * stride], a2, ja[(3 * d + 2) * stride] * a3)));
 }
 
 // flux_ranocha, :382-415

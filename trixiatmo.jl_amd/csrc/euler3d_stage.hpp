@@ -309,11 +309,13 @@ __device__ __forceinline__ void surface_momentum_split(const E3Params& q, int su
 // lanes each); its EPB * 6 n^2 face nodes are spread over all its lanes,
 // face node fg = t + ps * EPB * BLOCK of pass ps being node fg mod 6 n^2 of
 // slot fg / (6 n^2).
+// EPB = 0: the split form, one element whose face nodes have lanes of their own.
 template <int N, int EPB = 1>
 struct FacePrefetch {
-  static constexpr int GB = EPB * Shape<N>::BLOCK;
   static constexpr int NF = 6 * Shape<N>::N2;
-  static constexpr int PASSES = (EPB * NF + GB - 1) / GB;
+  static constexpr int SLOTS = EPB == 0 ? 1 : EPB;
+  static constexpr int GB = EPB == 0 ? (NF + 63) / 64 * 64 : EPB * Shape<N>::BLOCK;
+  static constexpr int PASSES = (SLOTS * NF + GB - 1) / GB;
   static constexpr int PF = N >= 4 ? 1 : PASSES;
   int link[PASSES], info[PASSES];
   double ur[PF][6];
@@ -332,8 +334,8 @@ __device__ __forceinline__ void face_links(FacePrefetch<N, EPB>& pf, int e0, int
 #pragma unroll
   for (int ps = FROM; ps < TO; ++ps) {
     const int fg = t + ps * F::GB;
-    const int es = EPB == 1 ? 0 : fg / NF;
-    const bool valid = fg < EPB * NF && es < n_valid;
+    const int es = EPB <= 1 ? 0 : fg / NF;
+    const bool valid = fg < F::SLOTS * NF && es < n_valid;
     const int fid = valid ? fg - es * NF : 0;
     const size_t e = (size_t)(e0 + (valid ? es : 0));
     pf.link[ps] = nbr[e * NF + fid];
@@ -362,8 +364,8 @@ __device__ __forceinline__ bool face_node_of(int t, int ps, int n_valid, int& es
   using F = FacePrefetch<N, EPB>;
   constexpr int N2 = Shape<N>::N2, NF = F::NF;
   const int fg = t + ps * F::GB;
-  es = EPB == 1 ? 0 : fg / NF;
-  if (fg >= EPB * NF || es >= n_valid) return false;
+  es = EPB <= 1 ? 0 : fg / NF;
+  if (fg >= F::SLOTS * NF || es >= n_valid) return false;
   fid = fg - es * NF;
   f = fid / N2;
   const int ab = fid - f * N2;
@@ -868,6 +870,155 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
   }
 }
 
+// flux_kennedy_gruber (with or without a gravity term) takes a sum form in the
+// volume terms, and so does the FP64 flux_ranocha (alone or with the Waruszewski
+// term): the averages' powers of two are applied once, by volume_scale
+template <int VOL, int NC, typename T>
+struct VolumeForm {
+  static constexpr bool MIXED = sizeof(T) == 4;
+  static constexpr bool KG_SUMS = VOL == 1;
+  static constexpr bool RANOCHA_SUMS = VOL == 0 && !MIXED && NC != 2;
+};
+
+// the volume terms of one node along direction d, added to acc and acc_nc
+template <int N, int VOL, int NC, typename T, bool KAHAN>
+__device__ __forceinline__ void volume_direction(const E3Params& q, const FastPrim<T>& l,
+                                                 const T* s_w, const double* s_phi,
+                                                 const T* s_buf, const T* s_ds, int tl, int ti,
+                                                 int tj, int tk, int d, double phi_own,
+                                                 const Background& bg, Acc<T, KAHAN>* acc,
+                                                 Acc<T, KAHAN>* acc_nc) {
+  constexpr int N2 = Shape<N>::N2, N3 = Shape<N>::N3;
+  constexpr bool MIXED = sizeof(T) == 4;
+  constexpr bool KG_SUMS = VolumeForm<VOL, NC, T>::KG_SUMS;
+  constexpr bool RANOCHA_SUMS = VolumeForm<VOL, NC, T>::RANOCHA_SUMS;
+  const int stride = d == 0 ? 1 : (d == 1 ? N : N2);
+  const int own_d = d == 0 ? ti : (d == 1 ? tj : tk);
+  const T* ja = s_buf + 3 * d * N3;
+  const T jo0 = ja[tl], jo1 = ja[N3 + tl], jo2 = ja[2 * N3 + tl];
+  // per lane: the step from which the partner index wraps, and the
+  // Dsplit row of the own node
+  const int lim = N - own_d;
+  const T* ds_row = s_ds + own_d * N + own_d;
+  // the partners in cyclic order own_d + 1, ..., own_d + n - 1 (mod n):
+  // every lane has a partner in each of the n - 1 iterations (a loop over
+  // the line's n nodes that skips the own one leaves a lane in n idle in
+  // every iteration)
+#pragma unroll 1
+  for (int j = 1; j < N; ++j) {
+    const bool wrap = j >= lim;
+    const int jw = wrap ? j - N : j;  // partner index minus own index
+    const int pn = tl + jw * stride;  // the partner node
+    const FastPrim<T> r = load_fast_prim<VOL, NC, N3, T>(s_w, pn, bg);
+    T dphi;
+    if constexpr (MIXED) dphi = T(s_phi[pn] - phi_own);
+    else dphi = r.phi - l.phi;
+    const T ds = ds_row[jw];
+    if constexpr (KG_SUMS) {
+      // flux_kennedy_gruber and the gravity term from sums of the two
+      // nodes' values: every average's factor 1/2 is a power of two, so
+      // accumulating 8 f_rho, 16 f_m, 16 f_E, 2 g_m and 4 g_E and scaling
+      // once at the end rounds exactly as the averaged form
+      const T rs = l.rho + r.rho, ps = l.p + r.p, es = l.e + r.e;
+      const T v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
+      const T n0s = jo0 + ja[pn], n1s = jo1 + ja[N3 + pn], n2s = jo2 + ja[2 * N3 + pn];
+      const T vns = v1s * n0s + v2s * n1s + v3s * n2s;
+      const T F = rs * vns;
+      // the momentum rows carry p' = p - p_bg when the background is split off
+      T pms = ps;
+      if constexpr (MIXED) {
+        if (bg.on) pms = l.pp + r.pp;
+      }
+      const T ps4 = T(4) * pms;
+      acc[0].add(ds * F);
+      acc[1].add(ds * (F * v1s + ps4 * n0s));
+      acc[2].add(ds * (F * v2s + ps4 * n1s));
+      acc[3].add(ds * (F * v3s + ps4 * n2s));
+      acc[4].add(ds * (F * es + (T(2) * ps) * vns));
+      if constexpr (NC != 0) {
+        const T ra = NC == 1 ? ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho) : T(0.5) * rs;
+        const T sj = ra * dphi;
+        T sm = sj;  // momentum part: (rho_avg - rho_avg of the background) [phi]
+        if constexpr (MIXED) {
+          if (bg.on) {
+            const T Ap = r.rp - l.rp, sp = l.rp + r.rp;
+            const T Ab = r.rb - l.rb, sb = l.rb + r.rb;
+            const T dmean = (NC == 1) ? delta_ln_mean(Ap + Ab, sp + sb, Ab, sb, Ap, sp,
+                                                      -dphi * T(bg.inv_RT0), r.lam - l.lam)
+                                      : T(0.5) * sp;
+            sm = dmean * dphi;
+          }
+        }
+        acc_nc[0].add(ds * (n0s * sm));
+        acc_nc[1].add(ds * (n1s * sm));
+        acc_nc[2].add(ds * (n2s * sm));
+        acc_nc[3].add(ds * (sj * vns));
+      }
+    } else if constexpr (RANOCHA_SUMS) {
+      // flux_ranocha and the Waruszewski term with every factor 1/2 of
+      // the averages (normals, velocities, pressure) left out and applied
+      // once at the end: 4 f_rho, 8 f_m, 8 f_E, 2 g_m and 4 g_E, each the
+      // averaged form's value times a power of two, so the sums round as
+      // the averaged form's do
+      const T n0s = jo0 + ja[pn], n1s = jo1 + ja[N3 + pn], n2s = jo2 + ja[2 * N3 + pn];
+      const T vnls = l.v1 * n0s + l.v2 * n1s + l.v3 * n2s;
+      const T vnrs = r.v1 * n0s + r.v2 * n1s + r.v3 * n2s;
+      const T rho_mean = ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho);
+      const T inv_rp = l.p * r.p * inv_ln_mean_logs(l.rho * r.p, r.rho * l.p, l.lrp - r.lrp);
+      const T v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
+      const T ps2 = T(2) * (l.p + r.p);
+      const T vvs = l.v1 * r.v1 + l.v2 * r.v2 + l.v3 * r.v3;
+      const T F = rho_mean * (vnls + vnrs);
+      acc[0].add(ds * F);
+      acc[1].add(ds * (F * v1s + ps2 * n0s));
+      acc[2].add(ds * (F * v2s + ps2 * n1s));
+      acc[3].add(ds * (F * v3s + ps2 * n2s));
+      acc[4].add(ds * (F * (vvs + inv_rp * T(2.0 * q.inv_gm1)) +
+                       T(2) * (l.p * vnrs + r.p * vnls)));
+      if constexpr (NC == 1) {
+        const T sj = rho_mean * dphi;
+        acc_nc[0].add(ds * (n0s * sj));
+        acc_nc[1].add(ds * (n1s * sj));
+        acc_nc[2].add(ds * (n2s * sj));
+        acc_nc[3].add(ds * (n0s * sj * v1s + n1s * sj * v2s + n2s * sj * v3s));
+      }
+    } else {
+      const T n0 = T(0.5) * (jo0 + ja[pn]);
+      const T n1 = T(0.5) * (jo1 + ja[N3 + pn]);
+      const T n2 = T(0.5) * (jo2 + ja[2 * N3 + pn]);
+      T f[5], g[5];
+      pair_flux<VOL, NC, T>(q, l, r, n0, n1, n2, dphi, bg, f, g);
+#pragma unroll
+      for (int v = 0; v < 5; ++v) acc[v].add(ds * f[v]);
+      if constexpr (NC != 0) {
+        acc_nc[0].add(ds * g[0]);
+        acc_nc[1].add(ds * g[1]);
+        acc_nc[2].add(ds * g[2]);
+        acc_nc[3].add(ds * g[3]);
+      }
+    }
+  }
+}
+
+template <int VOL, int NC, typename T, bool KAHAN>
+__device__ __forceinline__ void volume_scale(Acc<T, KAHAN>* acc, Acc<T, KAHAN>* acc_nc) {
+  if constexpr (VolumeForm<VOL, NC, T>::KG_SUMS) {
+    constexpr T sc[5] = {T(0.125), T(0.0625), T(0.0625), T(0.0625), T(0.0625)};
+    constexpr T scn[4] = {T(0.5), T(0.5), T(0.5), T(0.25)};
+#pragma unroll
+    for (int v = 0; v < 5; ++v) acc[v].scale(sc[v]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc_nc[v].scale(scn[v]);
+  } else if constexpr (VolumeForm<VOL, NC, T>::RANOCHA_SUMS) {
+    constexpr T sc[5] = {T(0.25), T(0.125), T(0.125), T(0.125), T(0.125)};
+    constexpr T scn[4] = {T(0.5), T(0.5), T(0.5), T(0.25)};
+#pragma unroll
+    for (int v = 0; v < 5; ++v) acc[v].scale(sc[v]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc_nc[v].scale(scn[v]);
+  }
+}
+
 // Direct form: every node evaluates the two-point flux with each of its n-1
 // partners on each line itself (each unordered pair is evaluated by both of
 // its nodes).  The fluxes are symmetric and the gravity terms antisymmetric
@@ -890,11 +1041,6 @@ void e3_stage_direct(
   constexpr bool MIXED = sizeof(T) == 4;
   constexpr int NW = NodeFields<VOL, NC, T>::NW;
   constexpr int BUF = 9 * N3 > 36 * N2 ? 9 * N3 : 36 * N2;
-  // flux_kennedy_gruber (with or without a gravity term) takes the sum form
-  // below, and so does the FP64 flux_ranocha (alone or with the Waruszewski
-  // term)
-  constexpr bool KG_SUMS = VOL == 1;
-  constexpr bool RANOCHA_SUMS = VOL == 0 && !MIXED && NC != 2;
   // EPB element slots of BE lanes each; slot es owns s_w_all[es], s_buf_all[es]
   __shared__ T s_w_all[EPB][NW * N3];
   __shared__ double s_phi_all[EPB][MIXED ? N3 : 1];
@@ -950,129 +1096,11 @@ void e3_stage_direct(
     const FastPrim<T> l = load_fast_prim<VOL, NC, N3, T>(s_w, tl, bg);
     double phi_own = 0.0;
     if constexpr (MIXED) phi_own = s_phi[tl];
-    for (int d = 0; d < 3; ++d) {
-      const int stride = d == 0 ? 1 : (d == 1 ? N : N2);
-      const int own_d = d == 0 ? ti : (d == 1 ? tj : tk);
-      const T* ja = s_buf + 3 * d * N3;
-      const T jo0 = ja[tl], jo1 = ja[N3 + tl], jo2 = ja[2 * N3 + tl];
-      // per lane: the step from which the partner index wraps, and the
-      // Dsplit row of the own node
-      const int lim = N - own_d;
-      const T* ds_row = s_ds + own_d * N + own_d;
-      // the partners in cyclic order own_d + 1, ..., own_d + n - 1 (mod n):
-      // every lane has a partner in each of the n - 1 iterations (a loop over
-      // the line's n nodes that skips the own one leaves a lane in n idle in
-      // every iteration)
-#pragma unroll 1
-      for (int j = 1; j < N; ++j) {
-        const bool wrap = j >= lim;
-        const int jw = wrap ? j - N : j;  // partner index minus own index
-        const int pn = tl + jw * stride;  // the partner node
-        const FastPrim<T> r = load_fast_prim<VOL, NC, N3, T>(s_w, pn, bg);
-        T dphi;
-        if constexpr (MIXED) dphi = T(s_phi[pn] - phi_own);
-        else dphi = r.phi - l.phi;
-        const T ds = ds_row[jw];
-        if constexpr (KG_SUMS) {
-          // flux_kennedy_gruber and the gravity term from sums of the two
-          // nodes' values: every average's factor 1/2 is a power of two, so
-          // accumulating 8 f_rho, 16 f_m, 16 f_E, 2 g_m and 4 g_E and scaling
-          // once at the end rounds exactly as the averaged form
-          const T rs = l.rho + r.rho, ps = l.p + r.p, es = l.e + r.e;
-          const T v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
-          const T n0s = jo0 + ja[pn], n1s = jo1 + ja[N3 + pn], n2s = jo2 + ja[2 * N3 + pn];
-          const T vns = v1s * n0s + v2s * n1s + v3s * n2s;
-          const T F = rs * vns;
-          // the momentum rows carry p' = p - p_bg when the background is split off
-          T pms = ps;
-          if constexpr (MIXED) {
-            if (bg.on) pms = l.pp + r.pp;
-          }
-          const T ps4 = T(4) * pms;
-          acc[0].add(ds * F);
-          acc[1].add(ds * (F * v1s + ps4 * n0s));
-          acc[2].add(ds * (F * v2s + ps4 * n1s));
-          acc[3].add(ds * (F * v3s + ps4 * n2s));
-          acc[4].add(ds * (F * es + (T(2) * ps) * vns));
-          if constexpr (NC != 0) {
-            const T ra = NC == 1 ? ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho) : T(0.5) * rs;
-            const T sj = ra * dphi;
-            T sm = sj;  // momentum part: (rho_avg - rho_avg of the background) [phi]
-            if constexpr (MIXED) {
-              if (bg.on) {
-                const T Ap = r.rp - l.rp, sp = l.rp + r.rp;
-                const T Ab = r.rb - l.rb, sb = l.rb + r.rb;
-                const T dmean = (NC == 1) ? delta_ln_mean(Ap + Ab, sp + sb, Ab, sb, Ap, sp,
-                                                          -dphi * T(bg.inv_RT0), r.lam - l.lam)
-                                          : T(0.5) * sp;
-                sm = dmean * dphi;
-              }
-            }
-            acc_nc[0].add(ds * (n0s * sm));
-            acc_nc[1].add(ds * (n1s * sm));
-            acc_nc[2].add(ds * (n2s * sm));
-            acc_nc[3].add(ds * (sj * vns));
-          }
-        } else if constexpr (RANOCHA_SUMS) {
-          // flux_ranocha and the Waruszewski term with every factor 1/2 of
-          // the averages (normals, velocities, pressure) left out and applied
-          // once at the end: 4 f_rho, 8 f_m, 8 f_E, 2 g_m and 4 g_E, each the
-          // averaged form's value times a power of two, so the sums round as
-          // the averaged form's do
-          const T n0s = jo0 + ja[pn], n1s = jo1 + ja[N3 + pn], n2s = jo2 + ja[2 * N3 + pn];
-          const T vnls = l.v1 * n0s + l.v2 * n1s + l.v3 * n2s;
-          const T vnrs = r.v1 * n0s + r.v2 * n1s + r.v3 * n2s;
-          const T rho_mean = ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho);
-          const T inv_rp = l.p * r.p * inv_ln_mean_logs(l.rho * r.p, r.rho * l.p, l.lrp - r.lrp);
-          const T v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
-          const T ps2 = T(2) * (l.p + r.p);
-          const T vvs = l.v1 * r.v1 + l.v2 * r.v2 + l.v3 * r.v3;
-          const T F = rho_mean * (vnls + vnrs);
-          acc[0].add(ds * F);
-          acc[1].add(ds * (F * v1s + ps2 * n0s));
-          acc[2].add(ds * (F * v2s + ps2 * n1s));
-          acc[3].add(ds * (F * v3s + ps2 * n2s));
-          acc[4].add(ds * (F * (vvs + inv_rp * T(2.0 * q.inv_gm1)) +
-                           T(2) * (l.p * vnrs + r.p * vnls)));
-          if constexpr (NC == 1) {
-            const T sj = rho_mean * dphi;
-            acc_nc[0].add(ds * (n0s * sj));
-            acc_nc[1].add(ds * (n1s * sj));
-            acc_nc[2].add(ds * (n2s * sj));
-            acc_nc[3].add(ds * (n0s * sj * v1s + n1s * sj * v2s + n2s * sj * v3s));
-          }
-        } else {
-          const T n0 = T(0.5) * (jo0 + ja[pn]);
-          const T n1 = T(0.5) * (jo1 + ja[N3 + pn]);
-          const T n2 = T(0.5) * (jo2 + ja[2 * N3 + pn]);
-          T f[5], g[5];
-          pair_flux<VOL, NC, T>(q, l, r, n0, n1, n2, dphi, bg, f, g);
 #pragma unroll
-          for (int v = 0; v < 5; ++v) acc[v].add(ds * f[v]);
-          if constexpr (NC != 0) {
-            acc_nc[0].add(ds * g[0]);
-            acc_nc[1].add(ds * g[1]);
-            acc_nc[2].add(ds * g[2]);
-            acc_nc[3].add(ds * g[3]);
-          }
-        }
-      }
-    }
-    if constexpr (KG_SUMS) {
-      constexpr T sc[5] = {T(0.125), T(0.0625), T(0.0625), T(0.0625), T(0.0625)};
-      constexpr T scn[4] = {T(0.5), T(0.5), T(0.5), T(0.25)};
-#pragma unroll
-      for (int v = 0; v < 5; ++v) acc[v].scale(sc[v]);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc_nc[v].scale(scn[v]);
-    } else if constexpr (RANOCHA_SUMS) {
-      constexpr T sc[5] = {T(0.25), T(0.125), T(0.125), T(0.125), T(0.125)};
-      constexpr T scn[4] = {T(0.5), T(0.5), T(0.5), T(0.25)};
-#pragma unroll
-      for (int v = 0; v < 5; ++v) acc[v].scale(sc[v]);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc_nc[v].scale(scn[v]);
-    }
+    for (int d = 0; d < 3; ++d)
+      volume_direction<N, VOL, NC, T, KAHAN>(q, l, s_w, s_phi, s_buf, s_ds, tl, ti, tj, tk, d,
+                                             phi_own, bg, acc, acc_nc);
+    volume_scale<VOL, NC, T, KAHAN>(acc, acc_nc);
   }
   // the links of the other passes, then the update's inputs, which arrive
   // during the face phase
@@ -1108,6 +1136,119 @@ void e3_stage_direct(
   }
 }
 
+// Split form of the direct form for meshes that do not fill the chip: an
+// element's work shared by sets of waves of one workgroup, so that the chain
+// of dependent operations, which is all that such a stage waits for, is
+// shorter.  Up to polydeg 5 three sets take the volume terms of one direction
+// each (beyond, one set takes all: the workgroup holds 1,024 lanes), another
+// set the face nodes, whose neighbour states and normals are on their way from
+// the start; the first set then adds the directions' sums and updates.
+template <int N>
+struct SplitShape {
+  static constexpr int DIRS = N <= 6 ? 3 : 1;  // sets of waves for the volume terms
+  static constexpr int FACE0 = DIRS * Shape<N>::BLOCK;
+  static constexpr int LANES = FACE0 + FacePrefetch<N, 0>::GB;
+};
+
+template <int N, int VOL, int NC, typename G>
+__global__ __launch_bounds__(SplitShape<N>::LANES) void e3_stage_split(
+    E3Params q, DsplitTable dst, double inv_w, int n_elements, const double* __restrict__ u,
+    double* __restrict__ out, double* __restrict__ kreg, const G* __restrict__ cv,
+    const double* __restrict__ invJ, const int* __restrict__ nbr,
+    const int* __restrict__ face_info, int surf, int snc, int mode, double rk_a, double rk_dt,
+    ResidentLink res, double rk_b, double coriolis, Background bg) {
+  using T = double;
+  using S = SplitShape<N>;
+  constexpr int N2 = Shape<N>::N2, N3 = Shape<N>::N3, BE = Shape<N>::BLOCK;
+  constexpr int NW = NodeFields<VOL, NC, T>::NW;
+  __shared__ T s_w[NW * N3];
+  __shared__ T s_cv[9 * N3];
+  __shared__ T s_sf[36 * N2];
+  __shared__ T s_vol[S::DIRS > 1 ? (S::DIRS - 1) * 5 * N3 : 1];
+  __shared__ T s_ds[N * N];
+  __shared__ double s_red[S::LANES / 64][3];
+
+  bg.on = 0;
+  const int e = blockIdx.x;
+  const int role = __builtin_amdgcn_readfirstlane(
+      threadIdx.x < (unsigned)S::FACE0 ? threadIdx.x / BE : S::DIRS);
+  const bool faces = role == S::DIRS;
+  const int tl = threadIdx.x - role * BE;
+  const bool active = !faces && tl < N3;
+  const int ti = tl % N, tj = (tl / N) % N, tk = tl / N2;
+  const size_t gnode = (size_t)e * N3 + tl;
+
+  FacePrefetch<N, 0> pf;
+  FaceNormals<N, T, 0> fn;
+  if (faces) {
+    face_links<N, 0, 0, 1>(pf, e, 1, tl, nbr, face_info);
+    if (tl < N * N) s_ds[tl] = dst.ds[tl];
+    face_prefetch_states<N, 0>(pf, u);
+    face_normals<N, T, 0, G, false>(fn, e, 1, tl, cv, nullptr, 0, pf);
+  } else if (active) {
+    // set d brings in the vectors of direction d
+    constexpr int ROWS = 9 / S::DIRS;
+    G ja[ROWS];
+#pragma unroll
+    for (int c = 0; c < ROWS; ++c) ja[c] = cv[((size_t)e * 9 + role * ROWS + c) * N3 + tl];
+    if (role == 0) {
+      double uo[6];
+#pragma unroll
+      for (int v = 0; v < 6; ++v) uo[v] = u[gnode * 6 + v];
+      node_fields_to_lds<N, VOL, NC, T>(q, uo, tl, s_w, nullptr, nullptr, bg);
+    }
+#pragma unroll
+    for (int c = 0; c < ROWS; ++c) s_cv[(role * ROWS + c) * N3 + tl] = T(ja[c]);
+  }
+  // the update's inputs arrive during the flux phase
+  NodeRest rest;
+  double uo[6], vol[5];
+  if (active && role == 0) {
+    rest = load_rest<N>(e, tl, invJ, kreg, mode);
+#pragma unroll
+    for (int v = 0; v < 6; ++v) uo[v] = u[gnode * 6 + v];
+  }
+  __syncthreads();
+  if (faces) {
+    face_fluxes_to_lds<N, T, 0>(q, e, 1, tl, inv_w, u, pf, fn, surf, snc, bg, s_w, 0, nullptr,
+                                s_sf, 0);
+  } else if (active) {
+    Acc<T, false> acc[5], acc_nc[4];
+    const FastPrim<T> l = load_fast_prim<VOL, NC, N3, T>(s_w, tl, bg);
+    if constexpr (S::DIRS > 1) {
+      volume_direction<N, VOL, NC, T, false>(q, l, s_w, nullptr, s_cv, s_ds, tl, ti, tj, tk, role,
+                                             0.0, bg, acc, acc_nc);
+    } else {
+#pragma unroll 1
+      for (int d = 0; d < 3; ++d)
+        volume_direction<N, VOL, NC, T, false>(q, l, s_w, nullptr, s_cv, s_ds, tl, ti, tj, tk, d,
+                                               0.0, bg, acc, acc_nc);
+    }
+    volume_scale<VOL, NC, T, false>(acc, acc_nc);
+    volume_sum(acc, acc_nc, vol);
+    if (role > 0) {
+#pragma unroll
+      for (int v = 0; v < 5; ++v) s_vol[((role - 1) * 5 + v) * N3 + tl] = vol[v];
+    }
+  }
+  __syncthreads();
+  double un[6];
+  const bool update = active && role == 0;
+  if (update) {
+    if constexpr (S::DIRS > 1) {
+#pragma unroll
+      for (int d = 0; d < S::DIRS - 1; ++d)
+#pragma unroll
+        for (int v = 0; v < 5; ++v) vol[v] += s_vol[(d * 5 + v) * N3 + tl];
+    }
+    stage_epilogue<N, T>(vol, s_sf, ti, tj, tk, e, gnode, uo, out, kreg, rest, mode, rk_a,
+                         res.dt ? res.dt[0] : rk_dt, rk_b, coriolis, bg, un);
+  }
+  if (res.speed_partial)
+    element_speed<N>(q, update, un, res.cv64, invJ, gnode, threadIdx.x, e, 1, s_red,
+                     res.speed_partial);
+}
+
 // which volume form a shape runs, from timings on MI355X: the direct form for
 // FP64 at every polydeg and for FP32 at polydeg 3 (6 % faster) and 7 (EC:
 // 1.8x faster than the pair form); the pair form for FP32 at polydeg 4 (2 %
@@ -1124,6 +1265,20 @@ constexpr bool use_direct_form() {
 template <int N, typename T>
 constexpr bool has_two_element_groups() {
   return (N == 4 || N == 5) && use_direct_form<N, 1, T>();
+}
+
+// the FP64 stage takes the split form up to this many elements: where its
+// waves are at most two per SIMD (2,048 on the chip's 256 CUs).  Microseconds
+// per stage of flux_ranocha shells, direct / split: 54 elements at polydeg 1
+// .. 7 6.0/4.8, 7.1/4.8, 8.3/5.0, 9.7/6.4, 10.4/8.9, 15.2/13.9, 17.2/17.5; near the line
+// polydeg 2 (648 elements) 7.5/6.6, polydeg 3 (300) 9.0/7.6, polydeg 4 (192)
+// 10.0/7.1, polydeg 5 (192) 11.1/10.4, polydeg 6 (192) 16.2/15.9; beyond it
+// polydeg 3 (648) 9.7/10.7, polydeg 4 (648) 14.6/17.0, polydeg 5 (300)
+// 14.9/18.2.  Polydeg 7, whose volume terms one set of waves has to take,
+// gains nothing.
+template <int N>
+constexpr int split_max_elements() {
+  return N <= 7 ? 2048 / (SplitShape<N>::LANES / 64) : 0;
 }
 
 template <int N, int VOL, int NC, typename T, bool KAHAN, int EPB, typename G>
@@ -1145,6 +1300,16 @@ void launch_stage_inst(const E3Launch& L, hipStream_t s) {
   const int grid = 8 * ((L.n_elements + 7) / 8);
   static_assert(std::is_same<G, T>::value || use_direct_form<N, VOL, T>(),
                 "geometry storage other than T needs the direct form");
+  if constexpr (std::is_same<T, double>::value && split_max_elements<N>() > 0) {
+    if (L.n_elements <= split_max_elements<N>()) {
+      hipLaunchKernelGGL((e3_stage_split<N, VOL, NC, G>), dim3(L.n_elements),
+                         dim3(SplitShape<N>::LANES), 0, s, L.q, dst, L.inv_w, L.n_elements, L.u,
+                         L.out, L.k, reinterpret_cast<const G*>(L.cv_t), L.invJ, L.nbr,
+                         L.face_info, L.surface_flux, L.surface_noncons, L.mode, L.rk_a, L.rk_dt,
+                         L.res, L.rk_b, L.coriolis, L.bg);
+      return;
+    }
+  }
   if constexpr (use_direct_form<N, VOL, T>()) {
     if constexpr (has_two_element_groups<N, T>()) {
       if (L.epb == 2) {
