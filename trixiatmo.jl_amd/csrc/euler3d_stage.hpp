@@ -870,17 +870,152 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
   }
 }
 
-// flux_kennedy_gruber (with or without a gravity term) takes a sum form in the
-// volume terms, and so does the FP64 flux_ranocha (alone or with the Waruszewski
-// term): the averages' powers of two are applied once, by volume_scale
-template <int VOL, int NC, typename T>
-struct VolumeForm {
-  static constexpr bool MIXED = sizeof(T) == 4;
-  static constexpr bool KG_SUMS = VOL == 1;
-  static constexpr bool RANOCHA_SUMS = VOL == 0 && !MIXED && NC != 2;
-};
+// Volume terms of the FP64 form: one pair's term as the own node sees it (a) and,
+// with BOTH, as its partner does (b), times the powers of two that
+// volume_scale64 takes out again.  f# is symmetric in the two nodes and the
+// gravity term g antisymmetric, so a = f# + g / 2 and b = f# - g / 2; in
+// flux_kennedy_gruber and flux_ranocha the gravity term's momentum and energy
+// entries have the shape of the pressure's, so both enter with the sum of the
+// nodes' pressures plus or minus rho_mean [phi] (for flux_ranocha twice that),
+// and the averages' factors 1/2 are left out: 8 f_rho, 16 f_m, 16 f_E, or
+// 4 f_rho, 8 f_m, 8 f_E.
+template <int VOL, int NC, bool BOTH>
+__device__ __forceinline__ void pair_terms64(const E3Params& q, const FastPrim<double>& l,
+                                             const FastPrim<double>& r, double n0s, double n1s,
+                                             double n2s, double* a, double* b) {
+  const double dphi = r.phi - l.phi;
+  if constexpr (VOL == 1) {  // flux_kennedy_gruber
+    const double rs = l.rho + r.rho, ps = l.p + r.p, es = l.e + r.e;
+    const double v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
+    const double vns = v1s * n0s + v2s * n1s + v3s * n2s;
+    const double F = rs * vns, Fe = F * es;
+    const double m1 = F * v1s, m2 = F * v2s, m3 = F * v3s;
+    double sj = 0.0;
+    if constexpr (NC == 1) sj = ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho) * dphi;
+    if constexpr (NC == 2) sj = 0.5 * rs * dphi;
+    const double p = ps + sj, p4 = 4.0 * p;
+    a[0] = F;
+    a[1] = m1 + p4 * n0s;
+    a[2] = m2 + p4 * n1s;
+    a[3] = m3 + p4 * n2s;
+    a[4] = Fe + (2.0 * p) * vns;
+    if constexpr (BOTH) {
+      const double pb = ps - sj, pb4 = 4.0 * pb;
+      b[0] = F;
+      b[1] = m1 + pb4 * n0s;
+      b[2] = m2 + pb4 * n1s;
+      b[3] = m3 + pb4 * n2s;
+      b[4] = Fe + (2.0 * pb) * vns;
+    }
+  } else if constexpr (VOL == 0) {  // flux_ranocha
+    const double vnls = l.v1 * n0s + l.v2 * n1s + l.v3 * n2s;
+    const double vnrs = r.v1 * n0s + r.v2 * n1s + r.v3 * n2s;
+    const double rho_mean = ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho);
+    const double inv_rp = l.p * r.p * inv_ln_mean_logs(l.rho * r.p, r.rho * l.p, l.lrp - r.lrp);
+    const double v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
+    const double ps2 = 2.0 * (l.p + r.p);
+    const double vvs = l.v1 * r.v1 + l.v2 * r.v2 + l.v3 * r.v3;
+    const double vns = vnls + vnrs, F = rho_mean * vns;
+    const double Fe = F * (vvs + inv_rp * (2.0 * q.inv_gm1)) + 2.0 * (l.p * vnrs + r.p * vnls);
+    const double m1 = F * v1s, m2 = F * v2s, m3 = F * v3s;
+    double sj = 0.0;
+    if constexpr (NC == 1) sj = rho_mean * dphi;
+    if constexpr (NC == 2) sj = 0.5 * (l.rho + r.rho) * dphi;
+    const double p = ps2 + 2.0 * sj;
+    a[0] = F;
+    a[1] = m1 + p * n0s;
+    a[2] = m2 + p * n1s;
+    a[3] = m3 + p * n2s;
+    a[4] = Fe + sj * vns;
+    if constexpr (BOTH) {
+      const double pb = ps2 - 2.0 * sj;
+      b[0] = F;
+      b[1] = m1 + pb * n0s;
+      b[2] = m2 + pb * n1s;
+      b[3] = m3 + pb * n2s;
+      b[4] = Fe - sj * vns;
+    }
+  } else {  // flux_shima_etal, on the averaged normal
+    double f[5], g[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const Background none{0, 0.0, 0.0, nullptr};
+    pair_flux<VOL, NC, double>(q, l, r, 0.5 * n0s, 0.5 * n1s, 0.5 * n2s, dphi, none, f, g);
+    a[0] = f[0];
+#pragma unroll
+    for (int v = 1; v < 5; ++v) a[v] = f[v] + 0.5 * g[v - 1];
+    if constexpr (BOTH) {
+      b[0] = f[0];
+#pragma unroll
+      for (int v = 1; v < 5; ++v) b[v] = f[v] - 0.5 * g[v - 1];
+    }
+  }
+}
 
-// the volume terms of one node along direction d, added to acc and acc_nc
+template <int VOL>
+__device__ __forceinline__ void volume_scale64(double* vol) {
+  constexpr double s0 = VOL == 1 ? 0.125 : VOL == 0 ? 0.25 : 1.0;
+  constexpr double s1 = VOL == 2 ? 1.0 : 0.5 * s0;
+  vol[0] *= s0;
+#pragma unroll
+  for (int v = 1; v < 5; ++v) vol[v] *= s1;
+}
+
+// whether all nodes of a line along direction d belong to one wave
+template <int N>
+__device__ constexpr bool line_in_wave(int d) {
+  return N <= 4 || (N == 8 && d < 2);
+}
+
+// the volume terms of one node along direction d, added to vol.  The partners
+// in cyclic order own + 1, own + 2, ... (mod n): every lane has one in each
+// step (a loop over the line's n nodes that skips the own one leaves a lane in n
+// idle).  SHARE (the line's nodes belong to one wave): a lane evaluates the pairs
+// with its next floor(n / 2) nodes only and hands each partner its side of the
+// pair by a lane exchange (with n even the last step pairs opposite nodes,
+// which evaluate it both).  Measured, with the gravity term folded into the
+// pressure: resident runs, ms, polydeg 7 flux_ranocha (two of three directions
+// shared) 47.5 -> 42.2, polydeg 5 (none) 12.15 -> 11.7, polydeg 4
+// flux_kennedy_gruber (none) 95.2 -> 94.6; a right-hand side of a polydeg 3
+// brick (all three) 12.7 -> 11.85 us.
+template <int N, int VOL, int NC, bool SHARE>
+__device__ __forceinline__ void volume_direction64(const E3Params& q, const FastPrim<double>& l,
+                                                   const double* s_w, const double* s_buf,
+                                                   const double* s_ds, int tl, int ti, int tj,
+                                                   int tk, int d, const Background& bg,
+                                                   double* vol) {
+  constexpr int N2 = Shape<N>::N2, N3 = Shape<N>::N3;
+  const int stride = d == 0 ? 1 : (d == 1 ? N : N2);
+  const int own = d == 0 ? ti : (d == 1 ? tj : tk);
+  const double* ja = s_buf + 3 * d * N3;
+  const double jo0 = ja[tl], jo1 = ja[N3 + tl], jo2 = ja[2 * N3 + tl];
+  // per lane: the step from which the partner index wraps, and the
+  // Dsplit row of the own node
+  const int lim = N - own;
+  const double* ds_row = s_ds + own * (N + 1);
+#pragma unroll 1
+  for (int j = 1; j <= (SHARE ? N / 2 : N - 1); ++j) {
+    const int step = j >= lim ? j - N : j;  // partner index minus own index
+    const int pn = tl + step * stride;      // the partner node
+    const FastPrim<double> r = load_fast_prim<VOL, NC, N3, double>(s_w, pn, bg);
+    double a[5], b[5];
+    pair_terms64<VOL, NC, SHARE>(q, l, r, jo0 + ja[pn], jo1 + ja[N3 + pn], jo2 + ja[2 * N3 + pn],
+                                 a, b);
+    const double ds = ds_row[step];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) vol[v] += ds * a[v];
+    if constexpr (SHARE) {
+      if (2 * j < N) {
+        const int back = own < j ? N - j : -j;
+        const double db = ds_row[back];
+        const int from = (tl & 63) + back * stride;
+#pragma unroll
+        for (int v = 0; v < 5; ++v) vol[v] += db * __shfl(b[v], from, 64);
+      }
+    }
+  }
+}
+
+// the FP32 forms' volume terms of one node along direction d, added to acc and
+// acc_nc; flux_kennedy_gruber in sum form (volume_scale)
 template <int N, int VOL, int NC, typename T, bool KAHAN>
 __device__ __forceinline__ void volume_direction(const E3Params& q, const FastPrim<T>& l,
                                                  const T* s_w, const double* s_phi,
@@ -889,9 +1024,6 @@ __device__ __forceinline__ void volume_direction(const E3Params& q, const FastPr
                                                  const Background& bg, Acc<T, KAHAN>* acc,
                                                  Acc<T, KAHAN>* acc_nc) {
   constexpr int N2 = Shape<N>::N2, N3 = Shape<N>::N3;
-  constexpr bool MIXED = sizeof(T) == 4;
-  constexpr bool KG_SUMS = VolumeForm<VOL, NC, T>::KG_SUMS;
-  constexpr bool RANOCHA_SUMS = VolumeForm<VOL, NC, T>::RANOCHA_SUMS;
   const int stride = d == 0 ? 1 : (d == 1 ? N : N2);
   const int own_d = d == 0 ? ti : (d == 1 ? tj : tk);
   const T* ja = s_buf + 3 * d * N3;
@@ -910,11 +1042,9 @@ __device__ __forceinline__ void volume_direction(const E3Params& q, const FastPr
     const int jw = wrap ? j - N : j;  // partner index minus own index
     const int pn = tl + jw * stride;  // the partner node
     const FastPrim<T> r = load_fast_prim<VOL, NC, N3, T>(s_w, pn, bg);
-    T dphi;
-    if constexpr (MIXED) dphi = T(s_phi[pn] - phi_own);
-    else dphi = r.phi - l.phi;
+    const T dphi = T(s_phi[pn] - phi_own);
     const T ds = ds_row[jw];
-    if constexpr (KG_SUMS) {
+    if constexpr (VOL == 1) {
       // flux_kennedy_gruber and the gravity term from sums of the two
       // nodes' values: every average's factor 1/2 is a power of two, so
       // accumulating 8 f_rho, 16 f_m, 16 f_E, 2 g_m and 4 g_E and scaling
@@ -925,11 +1055,7 @@ __device__ __forceinline__ void volume_direction(const E3Params& q, const FastPr
       const T vns = v1s * n0s + v2s * n1s + v3s * n2s;
       const T F = rs * vns;
       // the momentum rows carry p' = p - p_bg when the background is split off
-      T pms = ps;
-      if constexpr (MIXED) {
-        if (bg.on) pms = l.pp + r.pp;
-      }
-      const T ps4 = T(4) * pms;
+      const T ps4 = T(4) * (bg.on ? l.pp + r.pp : ps);
       acc[0].add(ds * F);
       acc[1].add(ds * (F * v1s + ps4 * n0s));
       acc[2].add(ds * (F * v2s + ps4 * n1s));
@@ -939,48 +1065,18 @@ __device__ __forceinline__ void volume_direction(const E3Params& q, const FastPr
         const T ra = NC == 1 ? ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho) : T(0.5) * rs;
         const T sj = ra * dphi;
         T sm = sj;  // momentum part: (rho_avg - rho_avg of the background) [phi]
-        if constexpr (MIXED) {
-          if (bg.on) {
-            const T Ap = r.rp - l.rp, sp = l.rp + r.rp;
-            const T Ab = r.rb - l.rb, sb = l.rb + r.rb;
-            const T dmean = (NC == 1) ? delta_ln_mean(Ap + Ab, sp + sb, Ab, sb, Ap, sp,
-                                                      -dphi * T(bg.inv_RT0), r.lam - l.lam)
-                                      : T(0.5) * sp;
-            sm = dmean * dphi;
-          }
+        if (bg.on) {
+          const T Ap = r.rp - l.rp, sp = l.rp + r.rp;
+          const T Ab = r.rb - l.rb, sb = l.rb + r.rb;
+          const T dmean = (NC == 1) ? delta_ln_mean(Ap + Ab, sp + sb, Ab, sb, Ap, sp,
+                                                    -dphi * T(bg.inv_RT0), r.lam - l.lam)
+                                    : T(0.5) * sp;
+          sm = dmean * dphi;
         }
         acc_nc[0].add(ds * (n0s * sm));
         acc_nc[1].add(ds * (n1s * sm));
         acc_nc[2].add(ds * (n2s * sm));
         acc_nc[3].add(ds * (sj * vns));
-      }
-    } else if constexpr (RANOCHA_SUMS) {
-      // flux_ranocha and the Waruszewski term with every factor 1/2 of
-      // the averages (normals, velocities, pressure) left out and applied
-      // once at the end: 4 f_rho, 8 f_m, 8 f_E, 2 g_m and 4 g_E, each the
-      // averaged form's value times a power of two, so the sums round as
-      // the averaged form's do
-      const T n0s = jo0 + ja[pn], n1s = jo1 + ja[N3 + pn], n2s = jo2 + ja[2 * N3 + pn];
-      const T vnls = l.v1 * n0s + l.v2 * n1s + l.v3 * n2s;
-      const T vnrs = r.v1 * n0s + r.v2 * n1s + r.v3 * n2s;
-      const T rho_mean = ln_mean_logs(l.rho, r.rho, l.lrho, r.lrho);
-      const T inv_rp = l.p * r.p * inv_ln_mean_logs(l.rho * r.p, r.rho * l.p, l.lrp - r.lrp);
-      const T v1s = l.v1 + r.v1, v2s = l.v2 + r.v2, v3s = l.v3 + r.v3;
-      const T ps2 = T(2) * (l.p + r.p);
-      const T vvs = l.v1 * r.v1 + l.v2 * r.v2 + l.v3 * r.v3;
-      const T F = rho_mean * (vnls + vnrs);
-      acc[0].add(ds * F);
-      acc[1].add(ds * (F * v1s + ps2 * n0s));
-      acc[2].add(ds * (F * v2s + ps2 * n1s));
-      acc[3].add(ds * (F * v3s + ps2 * n2s));
-      acc[4].add(ds * (F * (vvs + inv_rp * T(2.0 * q.inv_gm1)) +
-                       T(2) * (l.p * vnrs + r.p * vnls)));
-      if constexpr (NC == 1) {
-        const T sj = rho_mean * dphi;
-        acc_nc[0].add(ds * (n0s * sj));
-        acc_nc[1].add(ds * (n1s * sj));
-        acc_nc[2].add(ds * (n2s * sj));
-        acc_nc[3].add(ds * (n0s * sj * v1s + n1s * sj * v2s + n2s * sj * v3s));
       }
     } else {
       const T n0 = T(0.5) * (jo0 + ja[pn]);
@@ -1000,17 +1096,10 @@ __device__ __forceinline__ void volume_direction(const E3Params& q, const FastPr
   }
 }
 
-template <int VOL, int NC, typename T, bool KAHAN>
+template <int VOL, typename T, bool KAHAN>
 __device__ __forceinline__ void volume_scale(Acc<T, KAHAN>* acc, Acc<T, KAHAN>* acc_nc) {
-  if constexpr (VolumeForm<VOL, NC, T>::KG_SUMS) {
+  if constexpr (VOL == 1) {
     constexpr T sc[5] = {T(0.125), T(0.0625), T(0.0625), T(0.0625), T(0.0625)};
-    constexpr T scn[4] = {T(0.5), T(0.5), T(0.5), T(0.25)};
-#pragma unroll
-    for (int v = 0; v < 5; ++v) acc[v].scale(sc[v]);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc_nc[v].scale(scn[v]);
-  } else if constexpr (VolumeForm<VOL, NC, T>::RANOCHA_SUMS) {
-    constexpr T sc[5] = {T(0.25), T(0.125), T(0.125), T(0.125), T(0.125)};
     constexpr T scn[4] = {T(0.5), T(0.5), T(0.5), T(0.25)};
 #pragma unroll
     for (int v = 0; v < 5; ++v) acc[v].scale(sc[v]);
@@ -1091,28 +1180,34 @@ void e3_stage_direct(
   }
   __syncthreads();
 
-  Acc<T, KAHAN> acc[5], acc_nc[4];
+  double vol[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (active) {
     const FastPrim<T> l = load_fast_prim<VOL, NC, N3, T>(s_w, tl, bg);
-    double phi_own = 0.0;
-    if constexpr (MIXED) phi_own = s_phi[tl];
+    if constexpr (MIXED) {
+      Acc<T, KAHAN> acc[5], acc_nc[4];
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-      volume_direction<N, VOL, NC, T, KAHAN>(q, l, s_w, s_phi, s_buf, s_ds, tl, ti, tj, tk, d,
-                                             phi_own, bg, acc, acc_nc);
-    volume_scale<VOL, NC, T, KAHAN>(acc, acc_nc);
+      for (int d = 0; d < 3; ++d)
+        volume_direction<N, VOL, NC, T, KAHAN>(q, l, s_w, s_phi, s_buf, s_ds, tl, ti, tj, tk, d,
+                                               s_phi[tl], bg, acc, acc_nc);
+      volume_scale<VOL, T, KAHAN>(acc, acc_nc);
+      volume_sum(acc, acc_nc, vol);
+    } else {
+      volume_direction64<N, VOL, NC, line_in_wave<N>(0)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 0,
+                                                         bg, vol);
+      volume_direction64<N, VOL, NC, line_in_wave<N>(1)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 1,
+                                                         bg, vol);
+      volume_direction64<N, VOL, NC, line_in_wave<N>(2)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 2,
+                                                         bg, vol);
+      volume_scale64<VOL>(vol);
+    }
   }
   // the links of the other passes, then the update's inputs, which arrive
   // during the face phase
   face_links<N, EPB, FacePrefetch<N, EPB>::PF, FacePrefetch<N, EPB>::PASSES>(pf, e0, n_valid, t,
                                                                              nbr, face_info);
   constexpr bool LATE = FacePrefetch<N, EPB>::PASSES > 1;
-  double vol[5];
   NodeRest rest;
-  if (active) {
-    volume_sum(acc, acc_nc, vol);
-    if (!LATE) rest = load_rest<N>(e, tl, invJ, kreg, mode);
-  }
+  if (!LATE && active) rest = load_rest<N>(e, tl, invJ, kreg, mode);
   FaceNormals<N, T, EPB> fn;
   face_normals<N, T, EPB, G>(fn, e0, n_valid, t, cv, s_buf_all[0], BUF, pf);
   __syncthreads();  // contravariant vectors consumed; the buffer takes the face fluxes
@@ -1213,19 +1308,17 @@ __global__ __launch_bounds__(SplitShape<N>::LANES) void e3_stage_split(
     face_fluxes_to_lds<N, T, 0>(q, e, 1, tl, inv_w, u, pf, fn, surf, snc, bg, s_w, 0, nullptr,
                                 s_sf, 0);
   } else if (active) {
-    Acc<T, false> acc[5], acc_nc[4];
     const FastPrim<T> l = load_fast_prim<VOL, NC, N3, T>(s_w, tl, bg);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) vol[v] = 0.0;
     if constexpr (S::DIRS > 1) {
-      volume_direction<N, VOL, NC, T, false>(q, l, s_w, nullptr, s_cv, s_ds, tl, ti, tj, tk, role,
-                                             0.0, bg, acc, acc_nc);
+      volume_direction64<N, VOL, NC, N <= 4>(q, l, s_w, s_cv, s_ds, tl, ti, tj, tk, role, bg, vol);
     } else {
 #pragma unroll 1
       for (int d = 0; d < 3; ++d)
-        volume_direction<N, VOL, NC, T, false>(q, l, s_w, nullptr, s_cv, s_ds, tl, ti, tj, tk, d,
-                                               0.0, bg, acc, acc_nc);
+        volume_direction64<N, VOL, NC, false>(q, l, s_w, s_cv, s_ds, tl, ti, tj, tk, d, bg, vol);
     }
-    volume_scale<VOL, NC, T, false>(acc, acc_nc);
-    volume_sum(acc, acc_nc, vol);
+    volume_scale64<VOL>(vol);
     if (role > 0) {
 #pragma unroll
       for (int v = 0; v < 5; ++v) s_vol[((role - 1) * 5 + v) * N3 + tl] = vol[v];
