@@ -197,17 +197,26 @@ __device__ __forceinline__ double flux_n(const RNode& a, double n1, double n2, d
 __device__ __forceinline__ void surface_flux(const RainyLaunch& L, const double* uo,
                                              const double* un, double n1, double n2, double sgn,
                                              double w, double* f) {
-  const RNode l = rnode(uo), r = rnode(un);
+  const RNode r = rnode(un);
   if (L.surface_flux == 1) {
+    const RNode l = rnode(uo);
     flux_ec_rain(l, r, n1, n2, f);
 #pragma unroll
     for (int v = 0; v < 6; ++v) f[v] *= sgn * w;
     f[6] = f[7] = f[8] = 0.0;
     return;
   }
-  double fl[6], fr[6];
-  const double sl = flux_n(l, n1, n2, fl), sr = flux_n(r, n1, n2, fr);
-  const double lam = fmax(sl, sr) + fmax(l.c, r.c) * (n1 + n2);
+  double fr[6];
+  const double sr = flux_n(r, n1, n2, fr);
+  const double rc = r.c;
+  // the own side after the neighbour's is reduced to its flux: formed together the
+  // two take more than the 128 registers of four waves per SIMD (36 B of
+  // scratch per lane)
+  __builtin_amdgcn_sched_barrier(0);
+  double fl[6];
+  const RNode l = rnode(uo);
+  const double sl = flux_n(l, n1, n2, fl);
+  const double lam = fmax(sl, sr) + fmax(l.c, rc) * (n1 + n2);
   const double c = 0.5 * sgn * w, d = -0.5 * lam * w;
 #pragma unroll
   for (int v = 0; v < 6; ++v) f[v] = c * (fl[v] + fr[v]) + d * (un[v] - uo[v]);
