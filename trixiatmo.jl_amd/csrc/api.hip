@@ -718,8 +718,7 @@ int atmo_rhs(atmo_handle* h, double* du, const double* u, double t) {
     rc = run_rhs(h, h->d_duio, h->d_uio);
   }
   if (rc != ATMO_OK) return rc;
-  HIP_TRY(h, hipMemcpyAsync(du, h->d_duio, sb, hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(h, hipStreamSynchronize(h->stream));
+  HIP_TRY(h, copy_to_host(h, du, h->d_duio, sb));
   return ATMO_OK;
 }
 
@@ -749,8 +748,7 @@ int atmo_set_state(atmo_handle* h, const double* u) {
 
 int atmo_get_state(atmo_handle* h, double* u) {
   if (!h || !u) return fail(h ? &h->err : nullptr, ATMO_ERR_INVALID, "null argument");
-  HIP_TRY(h, hipMemcpyAsync(u, h->d_u, sizeof(double) * h->len, hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(h, hipStreamSynchronize(h->stream));
+  HIP_TRY(h, copy_to_host(h, u, h->d_u, sizeof(double) * h->len));
   return ATMO_OK;
 }
 

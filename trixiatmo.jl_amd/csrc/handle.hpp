@@ -13,6 +13,14 @@
 
 namespace atmo {
 
+// the handles in use: the last one to go gives back the pinned transfer slots
+struct HandleCount {
+  HandleCount();
+  ~HandleCount();
+  HandleCount(const HandleCount&) = delete;
+  HandleCount& operator=(const HandleCount&) = delete;
+};
+
 struct TimerPair {
   hipEvent_t a, b;
   int cls;
@@ -29,6 +37,7 @@ inline int fail(std::string* slot, int code, const std::string& msg) {
 }  // namespace atmo
 
 struct atmo_handle {
+  atmo::HandleCount counted;
   int eq = ATMO_EQ_EULER_ENERGY_GRAVITY_3D;
   atmo_config cfg;
   int n = 0, n3 = 0, nv = 6;
@@ -97,6 +106,9 @@ struct atmo_handle {
   } while (0)
 
 namespace atmo {
+// copy from the device to caller memory on the handle's stream, complete on
+// return (transfer.hip)
+hipError_t copy_to_host(atmo_handle* h, void* dst, const void* src, size_t bytes);
 // h_result / d_result of n doubles
 bool alloc_result(atmo_handle* h, size_t n);
 void timer_begin(atmo_handle* h, int cls, TimerPair* tp);

@@ -143,10 +143,7 @@ int atmo_solution_variables(atmo_handle* h, int32_t kind, double* out, int32_t* 
                        d_out);
   }
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(out, d_out, sizeof(double) * V_out * (size_t)n_nodes, hipMemcpyDeviceToHost,
-                       h->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  if (e == hipSuccess) e = copy_to_host(h, out, d_out, sizeof(double) * V_out * (size_t)n_nodes);
   (void)hipFree(d_out);
   if (e != hipSuccess) return fail(&h->err, ATMO_ERR_DEVICE, hipGetErrorString(e));
   if (n_vars) *n_vars = V_out;
