@@ -690,6 +690,8 @@ void atmo_destroy(atmo_handle* h) {
   if (h->d_fxf32) hipFree(h->d_fxf32);
   if (h->d_hs64) hipFree(h->d_hs64);
   if (h->d_clock) hipFree(h->d_clock);
+  if (h->h_clock) hipHostFree(h->h_clock);
+  if (h->solve_graph) hipGraphExecDestroy(h->solve_graph);
   if (h->d_step_dt) hipFree(h->d_step_dt);
   if (h->e3_graph) hipGraphExecDestroy(h->e3_graph);
   if (h->d_member) hipFree(h->d_member);

@@ -78,6 +78,13 @@ struct atmo_handle {
   atmo::RainyLaunch rainy_base{};
   double time = 0.0;                       // time of the resident state
   double* d_clock = nullptr;               // device clock of the resident time loop
+  double *h_clock = nullptr, *d_hclock = nullptr;  // its copy in pinned host memory
+  // two resident steps captured for replay, and the launch parameters (bytes of
+  // swe_base or rainy_base) and state buffer they were captured with
+  hipGraphExec_t solve_graph = nullptr;
+  double* solve_graph_u = nullptr;
+  int solve_graph_epb = 0;
+  std::vector<unsigned char> solve_graph_key;
   // 3D atmo_step: two RK steps captured for replay, their step size read from d_step_dt
   hipGraphExec_t e3_graph = nullptr;
   double* e3_graph_u = nullptr;            // state buffer the graph was captured with

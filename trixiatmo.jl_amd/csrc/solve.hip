@@ -154,11 +154,45 @@ void launch_step_control(const double* max_speed, int n_members, int n, double* 
 }
 
 namespace {
+// a clock at time t before its first step; dt: the step sizes the stages read
+__global__ void init_clock_kernel(double* clock, double* dt, int M, double t, double t_end,
+                                  double cfl) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < M) {
+    clock[m] = t;
+    clock[M + m] = 0.0;
+    clock[2 * M + m] = 0.0;
+    dt[m] = 0.0;
+  }
+  if (m == 0) {
+    clock[3 * M] = 0.0;
+    clock[3 * M + 1] = t_end;
+    clock[3 * M + 2] = cfl;
+  }
+}
+
+// t, the step sizes the stages read, the steps and the status
+__global__ void read_clock_kernel(const double* __restrict__ clock, const double* __restrict__ dt,
+                                  int M, double* __restrict__ out) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= 3 * M) out[i] = i >= M && i < 2 * M ? dt[i - M] : clock[i];
+}
+
 __global__ void fill_kernel(double* ptr, double value, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) ptr[i] = value;
 }
 }  // namespace
+
+void launch_init_clock(double* clock, double* dt, int M, double t, double t_end, double cfl,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(init_clock_kernel, dim3((M + 63) / 64), dim3(64), 0, s, clock, dt, M, t,
+                     t_end, cfl);
+}
+
+void launch_read_clock(const double* clock, const double* dt, int M, double* out, hipStream_t s) {
+  hipLaunchKernelGGL(read_clock_kernel, dim3((3 * M + 64) / 64), dim3(64), 0, s, clock, dt, M, out);
+}
 
 void launch_fill(double* ptr, double value, int n, hipStream_t s) {
   hipLaunchKernelGGL(fill_kernel, dim3((n + 63) / 64), dim3(64), 0, s, ptr, value, n);
@@ -189,6 +223,8 @@ void launch_step_control_reduce(const double* partial, int n_items, int n, doubl
 namespace {
 
 using atmo::fail;
+using atmo::launch_init_clock;
+using atmo::launch_read_clock;
 
 int enqueue_resident_steps(atmo_handle* h, int n_steps) {
   for (int s = 0; s < n_steps; ++s) {
@@ -201,8 +237,23 @@ int enqueue_resident_steps(atmo_handle* h, int n_steps) {
 }
 
 // two resident steps as one graph (the ping-pong state buffers return to
-// their places after an even number of stages)
-int capture_two_steps(atmo_handle* h, hipGraphExec_t* exec) {
+// their places after an even number of stages), kept for the next call with
+// the same buffers and launch parameters (capturing and instantiating it takes
+// about 60 us, which two steps on a small mesh take too)
+int ensure_solve_graph(atmo_handle* h) {
+  std::vector<unsigned char> key;
+  auto bytes = [&](const void* p, size_t n) {
+    key.assign(static_cast<const unsigned char*>(p), static_cast<const unsigned char*>(p) + n);
+  };
+  if (h->eq == ATMO_EQ_COVARIANT_SWE_2D) bytes(&h->swe_base, sizeof(h->swe_base));
+  if (h->eq == ATMO_EQ_RAINY_EULER_2D) bytes(&h->rainy_base, sizeof(h->rainy_base));
+  if (h->solve_graph && h->solve_graph_u == h->d_u && h->solve_graph_epb == h->e3_epb &&
+      h->solve_graph_key == key)
+    return ATMO_OK;
+  if (h->solve_graph) {
+    HIP_TRY(h, hipGraphExecDestroy(h->solve_graph));
+    h->solve_graph = nullptr;
+  }
   hipGraph_t g = nullptr;
   HIP_TRY(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
   const int rc = enqueue_resident_steps(h, 2);
@@ -212,9 +263,21 @@ int capture_two_steps(atmo_handle* h, hipGraphExec_t* exec) {
     return rc;
   }
   HIP_TRY(h, ec);
-  const hipError_t ei = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
+  const hipError_t ei = hipGraphInstantiate(&h->solve_graph, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   HIP_TRY(h, ei);
+  h->solve_graph_u = h->d_u;
+  h->solve_graph_epb = h->e3_epb;
+  h->solve_graph_key = std::move(key);
+  return ATMO_OK;
+}
+
+// the clock as it stands after everything enqueued, in h->h_clock: by a kernel
+// that writes pinned host memory (a copy into pageable memory takes 12 us more)
+int read_clock(atmo_handle* h, const double* d_dt, int M) {
+  launch_read_clock(h->d_clock, d_dt, M, h->d_hclock, h->stream);
+  HIP_TRY(h, hipGetLastError());
+  HIP_TRY(h, hipStreamSynchronize(h->stream));
   return ATMO_OK;
 }
 
@@ -234,25 +297,25 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
   // the step-size array the stages read: the shallow-water stage reads its
   // per-member array, the others the clock's
   double* d_dt = swe ? h->d_dt_member : h->d_clock + M;
-  std::vector<double> clk(clock_len, 0.0);
-  for (int m = 0; m < M; ++m) clk[m] = h->time;
-  clk[3 * M + 1] = t_end;
-  clk[3 * M + 2] = cfl;
-  HIP_TRY(h, hipMemcpyAsync(h->d_clock, clk.data(), sizeof(double) * clock_len,
-                            hipMemcpyHostToDevice, h->stream));
-  if (swe) {
-    HIP_TRY(h, hipMemcpyAsync(h->d_dt_member, clk.data() + M, sizeof(double) * M,
-                              hipMemcpyHostToDevice, h->stream));
-    if (!h->swe_tuned) {
-      const int rc = atmo::swe_autotune(h, nullptr);
-      if (rc != ATMO_OK) return rc;
-    }
+  if (!h->d_hclock) {
+    void* p = nullptr;
+    if (!h->h_clock)
+      HIP_TRY(h, hipHostMalloc(reinterpret_cast<void**>(&h->h_clock), sizeof(double) * clock_len,
+                               hipHostMallocDefault));
+    HIP_TRY(h, hipHostGetDevicePointer(&p, h->h_clock, 0));
+    h->d_hclock = static_cast<double*>(p);
+  }
+  if (swe && !h->swe_tuned) {
+    const int rc = atmo::swe_autotune(h, nullptr);
+    if (rc != ATMO_OK) return rc;
   }
   if (h->eq == ATMO_EQ_EULER_ENERGY_GRAVITY_3D && !h->e3_tuned) {
     const int rc = atmo::e3_autotune(h, nullptr);
     if (rc != ATMO_OK) return rc;
   }
   h->du_valid = false;
+  launch_init_clock(h->d_clock, d_dt, M, h->time, t_end, cfl, h->stream);
+  HIP_TRY(h, hipGetLastError());
   bool done = !(h->time < t_end);
   if (!done) {
     const int rc = h->eq == ATMO_EQ_EULER_ENERGY_GRAVITY_3D ? atmo::e3_resident_prologue(h)
@@ -262,10 +325,17 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
   }
   hipGraphExec_t graph = nullptr;
   if (!h->timing && !done) {
-    const int rc = capture_two_steps(h, &graph);
+    const int rc = ensure_solve_graph(h);
+    if (rc != ATMO_OK) return rc;
+    graph = h->solve_graph;
+  }
+  // the clock as last read (before the first step: where it starts)
+  const double* back = h->h_clock;
+  const double* dt_back = h->h_clock + M;
+  if (done) {
+    const int rc = read_clock(h, d_dt, M);
     if (rc != ATMO_OK) return rc;
   }
-  std::vector<double> back(clock_len), dt_back(M);
   int rc = ATMO_OK;
   // a first short chunk gives the step size the later chunks are sized by
   int64_t chunk = std::min<int64_t>(check_every, 2);
@@ -282,15 +352,8 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
       rc = enqueue_resident_steps(h, (int)chunk);
     }
     if (rc != ATMO_OK) break;
-    hipError_t e = hipMemcpyAsync(back.data(), h->d_clock, sizeof(double) * clock_len,
-                                  hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess && swe)
-      e = hipMemcpyAsync(dt_back.data(), d_dt, sizeof(double) * M, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) {
-      rc = fail(&h->err, ATMO_ERR_DEVICE, std::string("clock read-back: ") + hipGetErrorString(e));
-      break;
-    }
+    rc = read_clock(h, d_dt, M);
+    if (rc != ATMO_OK) break;
     if (back[3 * M] != 0.0) {
       rc = fail(&h->err, ATMO_ERR_NONFINITE, "non-finite wave speed in state");
       break;
@@ -300,7 +363,7 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
     done = true;
     double need = 0.0;
     for (int m = 0; m < M; ++m) {
-      const double dtm = swe ? dt_back[m] : back[M + m];
+      const double dtm = dt_back[m];
       const double tm = back[m] + dtm;
       if (tm < t_end) {
         done = false;
@@ -310,14 +373,8 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
     chunk = (int64_t)std::min<double>(std::max(need, 1.0), (double)check_every);
     if (graph) chunk += chunk & 1;
   }
-  if (graph) (void)hipGraphExecDestroy(graph);
   if (rc != ATMO_OK && rc != ATMO_ERR_NONFINITE) return rc;
-  // final clock: each member's time is t + dt of its last step
-  HIP_TRY(h, hipMemcpyAsync(back.data(), h->d_clock, sizeof(double) * clock_len,
-                            hipMemcpyDeviceToHost, h->stream));
-  HIP_TRY(h, hipMemcpyAsync(dt_back.data(), d_dt, sizeof(double) * M, hipMemcpyDeviceToHost,
-                            h->stream));
-  HIP_TRY(h, hipStreamSynchronize(h->stream));
+  // each member's time is t + dt of its last step
   double t_min = 0.0;
   for (int m = 0; m < M; ++m) {
     const double tm = back[m] + dt_back[m];
