@@ -138,8 +138,13 @@ int swe_resident_prologue(atmo_handle* h) {
 // one step: every member's step size from its elements' speeds in d_partial,
 // then the five stages, the last of which writes the new speeds there
 int swe_enqueue_resident_step(atmo_handle* h) {
-  launch_step_control_members_reduce(h->d_partial, h->d_member_first, h->n_members, h->n,
-                                     h->d_clock, h->d_dt_member, h->stream);
+  // a single member needs no look at where its elements begin
+  if (h->n_members == 1)
+    launch_step_control_reduce(h->d_partial, h->swe_base.n_elements, h->n, h->d_clock,
+                               h->d_dt_member, h->stream);
+  else
+    launch_step_control_members_reduce(h->d_partial, h->d_member_first, h->n_members, h->n,
+                                       h->d_clock, h->d_dt_member, h->stream);
   HIP_TRY(h, hipGetLastError());
   return enqueue_steps(h, 1, h->d_partial);
 }

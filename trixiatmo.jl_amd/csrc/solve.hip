@@ -27,22 +27,30 @@ namespace atmo {
 
 namespace {
 
+// what the control of member m reads, loaded while the partials are in flight
+struct ClockIn {
+  double t, dt, steps, t_end, cfl;
+};
+
+__device__ __forceinline__ ClockIn load_clock(const double* clock, const double* dt, int m, int M) {
+  return {clock[m], dt[m], clock[2 * M + m], clock[3 * M + 1], clock[3 * M + 2]};
+}
+
 // the step just taken is added to t, then the next step size is
 // dt = min(cfl * (2 / (n * max speed)), t_end - t) as atmo_max_dt and the host
 // loop compute it (same operations in the same order), or 0 once t >= t_end
-__device__ __forceinline__ void step_control_kernel_body(double max_speed, int m, int M, int n,
-                                                         double* clock, double* dt) {
-  const double t_end = clock[3 * M + 1], cfl = clock[3 * M + 2];
-  const double t = clock[m] + dt[m];
+__device__ __forceinline__ void step_control_kernel_body(double max_speed, const ClockIn& c, int m,
+                                                         int M, int n, double* clock, double* dt) {
+  const double t = c.t + c.dt;
   double d = 0.0;
-  if (t < t_end) {
+  if (t < c.t_end) {
     double mx = max_speed;
     if (!isfinite(mx)) {
       clock[3 * M] = 1.0;  // every member that finds one stores the same value
     } else {
       if (mx < 5e-324) mx = 5e-324;
-      d = fmin(cfl * (2.0 / (n * mx)), t_end - t);
-      clock[2 * M + m] += 1.0;
+      d = fmin(c.cfl * (2.0 / (n * mx)), c.t_end - t);
+      clock[2 * M + m] = c.steps + 1.0;
     }
   }
   clock[m] = t;
@@ -52,7 +60,8 @@ __device__ __forceinline__ void step_control_kernel_body(double max_speed, int m
 __global__ void step_control_kernel(const double* __restrict__ max_speed, int M, int n,
                                     double* clock, double* dt) {
   const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < M) step_control_kernel_body(max_speed[m], m, M, n, clock, dt);
+  if (m < M)
+    step_control_kernel_body(max_speed[m], load_clock(clock, dt, m, M), m, M, n, clock, dt);
 }
 
 // maximum over partial[from .. to) of a workgroup of B lanes, on every lane of
@@ -81,12 +90,16 @@ __device__ __forceinline__ double block_max(const double* __restrict__ partial, 
 }
 
 // the same for one member whose maximum speed is the maximum over per-element
-// partials (written by the last stage of the step just taken)
-__global__ __launch_bounds__(1024) void step_control_reduce_kernel(const double* __restrict__ partial,
-                                                                   int n_items, int n,
-                                                                   double* clock, double* dt) {
-  const double m = block_max<1024>(partial, 0, n_items, 0.0);
-  if (threadIdx.x == 0) step_control_kernel_body(m, 0, 1, n, clock, dt);
+// partials (written by the last stage of the step just taken).  One chain of
+// latencies between two stages: the clock is loaded beside the partials, and
+// the workgroup has as many lanes as one batch of block_max needs
+template <int B>
+__global__ __launch_bounds__(B) void step_control_reduce_kernel(const double* __restrict__ partial,
+                                                                int n_items, int n, double* clock,
+                                                                double* dt) {
+  const ClockIn c = load_clock(clock, dt, 0, 1);
+  const double m = block_max<B>(partial, 0, n_items, 0.0);
+  if (threadIdx.x == 0) step_control_kernel_body(m, c, 0, 1, n, clock, dt);
 }
 
 // one workgroup per ensemble member: its maximum speed is the maximum over the
@@ -95,8 +108,9 @@ __global__ __launch_bounds__(256) void step_control_members_reduce_kernel(
     const double* __restrict__ partial, const int* __restrict__ member_first, int M, int n,
     double* clock, double* dt) {
   const int m = blockIdx.x;
+  const ClockIn c = load_clock(clock, dt, m, M);
   const double mx = block_max<256>(partial, member_first[m], member_first[m + 1], 0.0);
-  if (threadIdx.x == 0) step_control_kernel_body(mx, m, M, n, clock, dt);
+  if (threadIdx.x == 0) step_control_kernel_body(mx, c, m, M, n, clock, dt);
 }
 
 __global__ __launch_bounds__(1024) void reduce_max_kernel(const double* __restrict__ partial, int n,
@@ -214,8 +228,12 @@ void launch_sum_rows(const double* partial, int n, int width, double* result, hi
 
 void launch_step_control_reduce(const double* partial, int n_items, int n, double* clock,
                                 double* dt, hipStream_t s) {
-  hipLaunchKernelGGL(step_control_reduce_kernel, dim3(1), dim3(1024), 0, s, partial, n_items, n,
-                     clock, dt);
+  if (n_items <= 8 * 256)
+    hipLaunchKernelGGL(step_control_reduce_kernel<256>, dim3(1), dim3(256), 0, s, partial, n_items,
+                       n, clock, dt);
+  else
+    hipLaunchKernelGGL(step_control_reduce_kernel<1024>, dim3(1), dim3(1024), 0, s, partial,
+                       n_items, n, clock, dt);
 }
 
 }  // namespace atmo
