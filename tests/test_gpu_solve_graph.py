@@ -56,3 +56,41 @@ def test_pieces_on_one_handle(family):
             np.testing.assert_array_equal(a, b)
         assert np.isfinite(got[0][0]).all() and got[0][1][0] > 2
         u, t = got[0][0].reshape(one.shape, order="F"), got[0][2]
+
+
+@pytest.mark.parametrize("cells,precision", [(1, "fp64"), (9, "fp64"), (9, "fp32_geometry"),
+                                             (10, "fp64")])
+def test_control_inside_the_first_stage(cells, precision):
+    """up to 512 elements the split shapes take the step control into the first
+    stage: the same steps to the same bits as with a kernel of its own (the
+    plain shapes, and launches one by one), a last step cut short and a wave
+    speed that is not a number included"""
+    print(f"case: cells {cells} {precision}", flush=True)
+    case = W.covariant_elixir("rossby_haurwitz", cells=cells, polydeg=3, precision=precision)
+    u0 = case.u0()
+    semi = case.semi()
+    semi.set_state(u0)
+    dt = semi.max_dt(0.4)
+    first = None
+    for variant, timing in ((0, False), (3, False), (3, True), (4, False), (5, False)):
+        semi.enable_timing(timing)
+        semi.set_kernel_variant(variant)
+        semi.set_state(u0)
+        semi.set_time(0.0)
+        a = semi.solve_resident(4.5 * dt, 0.4, 4)
+        b = semi.solve_resident(6.7 * dt, 0.4, 1)
+        got = (semi.get_state(), a[0], a[1], b[0], b[1])
+        assert a[0][0] >= 5 and b[1] == 6.7 * dt
+        if first is None:
+            first = got
+        for x, y in zip(got, first):
+            np.testing.assert_array_equal(x, y)
+    bad = u0.copy()
+    bad[0, 0, 0, -1] = np.nan
+    for variant in (0, 3):
+        semi.enable_timing(False)
+        semi.set_kernel_variant(variant)
+        semi.set_state(bad)
+        semi.set_time(0.0)
+        with pytest.raises(T.AtmoError, match="NONFINITE"):
+            semi.solve_resident(dt, 0.4)

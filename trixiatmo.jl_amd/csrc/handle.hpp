@@ -139,7 +139,11 @@ void rainy_free(atmo_handle* h);
 // the resident time loop: one step (maximum wave speed, step-size control,
 // five stages reading the step size from d_clock) enqueued on the stream
 int e3_enqueue_resident_step(atmo_handle* h);
-int swe_enqueue_resident_step(atmo_handle* h);
+// side: -1 with a control kernel of its own, else the clock (0 or 1) that the
+// first stage reads while it writes the other
+int swe_enqueue_resident_step(atmo_handle* h, int side);
+// whether a resident step's first stage can take the control
+bool swe_fuses_control(const atmo_handle* h);
 int rainy_enqueue_resident_step(atmo_handle* h);
 // ptr[0 .. n) = value, stream-ordered (a value for kernels that read it from memory)
 void launch_fill(double* ptr, double value, int n, hipStream_t s);

@@ -18,43 +18,19 @@
 
 #include "handle.hpp"
 #include "speed_max.hpp"
-
-// clock layout (M members): t[M] (start of the step in flight), dt[M], steps
-// taken [M], status (1: non-finite wave speed), t_end, cfl
-constexpr int kClockExtra = 3;
+#include "step_control.hpp"
 
 namespace atmo {
 
 namespace {
 
-// what the control of member m reads, loaded while the partials are in flight
-struct ClockIn {
-  double t, dt, steps, t_end, cfl;
-};
-
-__device__ __forceinline__ ClockIn load_clock(const double* clock, const double* dt, int m, int M) {
-  return {clock[m], dt[m], clock[2 * M + m], clock[3 * M + 1], clock[3 * M + 2]};
-}
-
-// the step just taken is added to t, then the next step size is
-// dt = min(cfl * (2 / (n * max speed)), t_end - t) as atmo_max_dt and the host
-// loop compute it (same operations in the same order), or 0 once t >= t_end
 __device__ __forceinline__ void step_control_kernel_body(double max_speed, const ClockIn& c, int m,
                                                          int M, int n, double* clock, double* dt) {
-  const double t = c.t + c.dt;
-  double d = 0.0;
-  if (t < c.t_end) {
-    double mx = max_speed;
-    if (!isfinite(mx)) {
-      clock[3 * M] = 1.0;  // every member that finds one stores the same value
-    } else {
-      if (mx < 5e-324) mx = 5e-324;
-      d = fmin(c.cfl * (2.0 / (n * mx)), c.t_end - t);
-      clock[2 * M + m] = c.steps + 1.0;
-    }
-  }
-  clock[m] = t;
-  dt[m] = d;
+  const ClockOut o = step_control(max_speed, c, n);
+  if (o.failed) clock[3 * M] = 1.0;  // every member that finds one stores the same value
+  clock[2 * M + m] = o.steps;
+  clock[m] = o.t;
+  dt[m] = o.dt;
 }
 
 __global__ void step_control_kernel(const double* __restrict__ max_speed, int M, int n,
@@ -241,12 +217,13 @@ void launch_step_control_reduce(const double* partial, int n_items, int n, doubl
 namespace {
 
 using atmo::fail;
+using atmo::kClockExtra;
 using atmo::launch_init_clock;
 using atmo::launch_read_clock;
 
-int enqueue_resident_steps(atmo_handle* h, int n_steps) {
+int enqueue_resident_steps(atmo_handle* h, int n_steps, bool fused) {
   for (int s = 0; s < n_steps; ++s) {
-    const int rc = h->eq == ATMO_EQ_COVARIANT_SWE_2D ? atmo::swe_enqueue_resident_step(h)
+    const int rc = h->eq == ATMO_EQ_COVARIANT_SWE_2D ? atmo::swe_enqueue_resident_step(h, fused ? s & 1 : -1)
                    : h->eq == ATMO_EQ_RAINY_EULER_2D ? atmo::rainy_enqueue_resident_step(h)
                                                      : atmo::e3_enqueue_resident_step(h);
     if (rc != ATMO_OK) return rc;
@@ -258,7 +235,7 @@ int enqueue_resident_steps(atmo_handle* h, int n_steps) {
 // their places after an even number of stages), kept for the next call with
 // the same buffers and launch parameters (capturing and instantiating it takes
 // about 60 us, which two steps on a small mesh take too)
-int ensure_solve_graph(atmo_handle* h) {
+int ensure_solve_graph(atmo_handle* h, bool fused) {
   std::vector<unsigned char> key;
   auto bytes = [&](const void* p, size_t n) {
     key.assign(static_cast<const unsigned char*>(p), static_cast<const unsigned char*>(p) + n);
@@ -274,7 +251,7 @@ int ensure_solve_graph(atmo_handle* h) {
   }
   hipGraph_t g = nullptr;
   HIP_TRY(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-  const int rc = enqueue_resident_steps(h, 2);
+  const int rc = enqueue_resident_steps(h, 2, fused);
   const hipError_t ec = hipStreamEndCapture(h->stream, &g);
   if (rc != ATMO_OK) {
     if (g) (void)hipGraphDestroy(g);
@@ -311,10 +288,7 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
   const bool swe = h->eq == ATMO_EQ_COVARIANT_SWE_2D;
   const int M = swe ? h->n_members : 1;
   const size_t clock_len = 3 * (size_t)M + kClockExtra;
-  if (!h->d_clock) HIP_TRY(h, hipMalloc(&h->d_clock, sizeof(double) * clock_len));
-  // the step-size array the stages read: the shallow-water stage reads its
-  // per-member array, the others the clock's
-  double* d_dt = swe ? h->d_dt_member : h->d_clock + M;
+  if (!h->d_clock) HIP_TRY(h, hipMalloc(&h->d_clock, sizeof(double) * 2 * clock_len));
   if (!h->d_hclock) {
     void* p = nullptr;
     if (!h->h_clock)
@@ -331,6 +305,12 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
     const int rc = atmo::e3_autotune(h, nullptr);
     if (rc != ATMO_OK) return rc;
   }
+  // the control as part of the first stage (an even number of steps, which the
+  // graph takes, ends on the clock it began with)
+  const bool fused = swe && !h->timing && atmo::swe_fuses_control(h);
+  // the step-size array the stages read: the shallow-water stage reads its
+  // per-member array, the others the clock's
+  double* d_dt = swe && !fused ? h->d_dt_member : h->d_clock + M;
   h->du_valid = false;
   launch_init_clock(h->d_clock, d_dt, M, h->time, t_end, cfl, h->stream);
   HIP_TRY(h, hipGetLastError());
@@ -343,7 +323,7 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
   }
   hipGraphExec_t graph = nullptr;
   if (!h->timing && !done) {
-    const int rc = ensure_solve_graph(h);
+    const int rc = ensure_solve_graph(h, fused);
     if (rc != ATMO_OK) return rc;
     graph = h->solve_graph;
   }
@@ -367,7 +347,7 @@ int atmo_solve(atmo_handle* h, double t_end, double cfl, int32_t check_every, in
         }
       }
     } else {
-      rc = enqueue_resident_steps(h, (int)chunk);
+      rc = enqueue_resident_steps(h, (int)chunk, false);
     }
     if (rc != ATMO_OK) break;
     rc = read_clock(h, d_dt, M);

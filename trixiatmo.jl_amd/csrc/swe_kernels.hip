@@ -45,6 +45,7 @@
 #include "handle.hpp"
 #include "swe_kernels.hpp"
 #include "speed_max.hpp"
+#include "step_control.hpp"
 
 namespace atmo {
 
@@ -333,7 +334,10 @@ __device__ __forceinline__ void swe_node_speeds(const double* u, double gcon11, 
 // SPEED: the RK stage also writes L.speed_partial (the last stage of a
 // resident step); a variant of its own, so the other stages keep their
 // register budget
-template <int N, int WAVES, bool SPLIT, bool SPEED, typename GT>
+// CONTROL: the first stage of a resident step forms its step size itself: the
+// loads of its node waves go out with the node's own, the reduction follows
+// the volume terms, while the face waves are still busy
+template <int N, int WAVES, bool SPLIT, bool SPEED, bool CONTROL, typename GT>
 __global__ __launch_bounds__((SPLIT ? 3 : 1) * 64 * WAVES)
 __attribute__((amdgpu_waves_per_eu(N == 4 && !SPLIT ? 5 : 1)))
 void swe_stage(SweLaunch L) {
@@ -405,14 +409,41 @@ void swe_stage(SweLaunch L) {
     if (L.mode != 0) {
 #pragma unroll
       for (int v = 0; v < NV; ++v) kreg[v] = L.k[v * NN + g];
-      if (L.dt_member) dt = L.dt_member[L.member[e]];
+      if (!CONTROL && L.dt_member) dt = L.dt_member[L.member[e]];
     }
   };
   if (SPLIT && node_role && active) load_rest();
+  double speeds[CONTROL ? 8 : 1];
+  ClockIn clk{};
+  if (CONTROL && node_role) {
+    clk = load_clock(L.clock_in, L.clock_in + 1, 0, 1);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int i = (t & 63) + 64 * k;
+      speeds[CONTROL ? k : 0] = i < L.n_elements ? L.control_partial[i] : 0.0;
+    }
+  }
   __syncthreads();
 
   double du[NV], d1[NV];
   if (node_role && active) volume_terms<N, UNROLL>(L, s_n[es], s_ds, q, 0, du);
+  if (CONTROL && node_role) {  // each wave for itself
+    double m = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m = speed_max(m, speeds[CONTROL ? k : 0]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = speed_max(m, __shfl_xor(m, o, 64));
+    const ClockOut next = step_control(m, clk, N);
+    dt = next.dt;
+    if (blockIdx.x == 0 && t == 0) {
+      L.clock_out[0] = next.t;
+      L.clock_out[1] = next.dt;
+      L.clock_out[2] = next.steps;
+      L.clock_out[3] = next.failed ? 1.0 : L.clock_in[3];
+      L.clock_out[4] = clk.t_end;
+      L.clock_out[5] = clk.cfl;
+    }
+  }
   if (dir1_role && active) {
     volume_terms<N, UNROLL>(L, s_n[es], s_ds, q, 1, d1);
     if constexpr (SPLIT) {
@@ -564,15 +595,21 @@ void launch_variant(const SweLaunch& L, hipStream_t s) {
   using S = SweShape<N, WAVES>;
   const dim3 grid((L.n_elements + S::EPB - 1) / S::EPB), block((SPLIT ? 3 : 1) * S::LANES);
   const bool speed = L.speed_partial && L.mode == 1;
+  auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, s, L); };
+  if constexpr (SPLIT) {
+    if (L.control_partial) {
+      if (L.geo32) go(swe_stage<N, WAVES, SPLIT, false, true, float>);
+      else go(swe_stage<N, WAVES, SPLIT, false, true, double>);
+      return;
+    }
+  }
   if (L.geo32) {
-    if (speed)
-      hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, true, float>), grid, block, 0, s, L);
-    else
-      hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, false, float>), grid, block, 0, s, L);
+    if (speed) go(swe_stage<N, WAVES, SPLIT, true, false, float>);
+    else go(swe_stage<N, WAVES, SPLIT, false, false, float>);
   } else if (speed) {
-    hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, true, double>), grid, block, 0, s, L);
+    go(swe_stage<N, WAVES, SPLIT, true, false, double>);
   } else {
-    hipLaunchKernelGGL((swe_stage<N, WAVES, SPLIT, false, double>), grid, block, 0, s, L);
+    go(swe_stage<N, WAVES, SPLIT, false, false, double>);
   }
 }
 

@@ -44,11 +44,20 @@ struct SweLaunch {
   const double* dt_member;  // per-member time steps (NULL: rk_dt for all)
   double* speed_partial;    // RK stage, if set: per element the StepsizeCallback sum over
                             // directions of the maximum scaled speed of the new state
+  // first stage of a resident step, if set: the per-element speeds and the
+  // clock that its step size comes from, and the clock it writes (the split
+  // shapes, one member, at most kSweControlMax elements)
+  const double* control_partial;
+  const double* clock_in;
+  double* clock_out;
   const int* member;        // [E] member of each element
   int topography;           // 0: h_s is zero at every node and its row is not read
   int variant;              // workgroup shape: node lanes of 1, 2, 4 waves (0..2), split (3..5)
 };
 constexpr int kSweVariants = 6;
+constexpr int kSweSplitVariant = 3;  // the first of the split shapes
+// one batch of eight loads per lane of a wave
+constexpr int kSweControlMax = 512;
 
 // init_auxiliary_node_variables! on the device (swe_geometry.hip): aux
 // [26,n,n,E] from the node coordinates X [3,n,n,E] (LGL nodes x_lgl[n],
