@@ -35,8 +35,8 @@ METRIC = "GDOF\u00b7RHS/s, mixed vs FP64 on 1 GPU at stated rel. err; % of VALU 
 # stage issues 128 B read requests, counted as 64 B, as for a plain device
 # copy of known size) and the executed flops per node
 # (64 x (ADD + MUL + TRANS) + 128 x FMA wave instructions / nodes).
-STAGE_FETCH_KIB, STAGE_WRITE_KIB, FETCH_FACTOR = 2.020e5, 1.258e5, 2.0
-EXEC_FP64_FLOPS_PER_NODE = 1383.0
+STAGE_FETCH_KIB, STAGE_WRITE_KIB, FETCH_FACTOR = 2.049e5, 1.263e5, 2.0
+EXEC_FP64_FLOPS_PER_NODE = 1159.0
 COUNTER_PASSES = (("FETCH_SIZE",), ("WRITE_SIZE",),
                   ("SQ_INSTS_VALU_FMA_F64", "SQ_INSTS_VALU_MUL_F64", "SQ_INSTS_VALU_ADD_F64",
                    "SQ_INSTS_VALU_TRANS_F64"))
@@ -47,7 +47,7 @@ CALIBRATION_COPY_BYTES = 256 << 20
 # + - * / sqrt log exp pow one each), every node pair of a line evaluated once
 # as the reference does
 ALG_FP64_FLOPS_PER_NODE = 1680.4
-EXEC_MIXED_FLOPS_PER_NODE = {"fp32": 1703.0, "fp64": 298.0}
+EXEC_MIXED_FLOPS_PER_NODE = {"fp32": 1695.0, "fp64": 298.0}
 
 
 def log(msg):
