@@ -357,15 +357,17 @@ __device__ __forceinline__ void face_prefetch_states(FacePrefetch<N, EPB>& pf,
 
 // face-node geometry of pass ps: element slot es, face node fid of that
 // element, face f, direction d, own node; false when the lane has no face
-// node in that pass
+// node in that pass (es is then a slot of the workgroup all the same:
+// face_normals reads that slot's LDS copy on every lane)
 template <int N, int EPB = 1>
-__device__ __forceinline__ bool face_node_of(int t, int ps, int n_valid, int& es, int& fid, int& f,
-                                             int& d, int& node) {
+__host__ __device__ __forceinline__ bool face_node_of(int t, int ps, int n_valid, int& es,
+                                                      int& fid, int& f, int& d, int& node) {
   using F = FacePrefetch<N, EPB>;
   constexpr int N2 = Shape<N>::N2, NF = F::NF;
   const int fg = t + ps * F::GB;
-  es = EPB <= 1 ? 0 : fg / NF;
-  if (fg >= F::SLOTS * NF || es >= n_valid) return false;
+  const int slot = EPB <= 1 ? 0 : fg / NF;
+  es = slot < F::SLOTS ? slot : F::SLOTS - 1;
+  if (fg >= F::SLOTS * NF || slot >= n_valid) return false;
   fid = fg - es * NF;
   f = fid / N2;
   const int ab = fid - f * N2;
