@@ -36,7 +36,7 @@ def test_rhs_on_both_sides_of_the_line(oracle, polydeg, beyond, fluxes):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "fp32_geometry"])
-@pytest.mark.parametrize("polydeg", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("polydeg", [1, 2, 3, 4, 5, 6])
 def test_split_form_steps_and_resident_loop(polydeg, precision):
     mesh, eq, solver, bcs, u0 = T.workloads.periodic_cube(trees=3, polydeg=polydeg, seed=4,
                                                           precision=precision)

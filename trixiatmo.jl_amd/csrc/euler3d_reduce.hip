@@ -14,6 +14,9 @@ template <int N>
 struct Shape {
   static constexpr int N3 = N * N * N;
   static constexpr int BLOCK = ((N3 + 63) / 64) * 64;
+  // first step of a halving reduction over BLOCK lanes: the largest power of
+  // two below it (at polydeg 6 the 384 lanes fold 128 into 256 first)
+  static constexpr int FOLD = BLOCK > 256 ? 256 : BLOCK / 2;
 };
 
 struct WeightTable {
@@ -48,8 +51,8 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_max_speed(E3Params q, cons
   }
   s[0][t] = l1; s[1][t] = l2; s[2][t] = l3;
   __syncthreads();
-  for (int w = B / 2; w > 0; w >>= 1) {
-    if (t < w) {
+  for (int w = Shape<N>::FOLD; w > 0; w >>= 1) {
+    if (t < w && t + w < B) {
       s[0][t] = speed_max(s[0][t], s[0][t + w]);
       s[1][t] = speed_max(s[1][t], s[1][t + w]);
       s[2][t] = speed_max(s[2][t], s[2][t + w]);
@@ -96,8 +99,8 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_integrals(E3Params q, Weig
   }
   for (int c = 0; c < K; ++c) s[c][t] = val[c];
   __syncthreads();
-  for (int w = B / 2; w > 0; w >>= 1) {
-    if (t < w)
+  for (int w = Shape<N>::FOLD; w > 0; w >>= 1) {
+    if (t < w && t + w < B)
       for (int c = 0; c < K; ++c) s[c][t] += s[c][t + w];
     __syncthreads();
   }
