@@ -1194,12 +1194,23 @@ void e3_stage_direct(
       volume_scale<VOL, T, KAHAN>(acc, acc_nc);
       volume_sum(acc, acc_nc, vol);
     } else {
-      volume_direction64<N, VOL, NC, line_in_wave<N>(0)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 0,
-                                                         bg, vol);
-      volume_direction64<N, VOL, NC, line_in_wave<N>(1)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 1,
-                                                         bg, vol);
-      volume_direction64<N, VOL, NC, line_in_wave<N>(2)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 2,
-                                                         bg, vol);
+      if constexpr (N <= 3) {
+        // a direction is a single step here: written one after the other, the
+        // scheduler interleaves all three and spills up to 116 B of scratch per
+        // lane (microseconds per stage of shells, one after the other / looped:
+        // polydeg 2, 12,288 elements, flux_ranocha 58.1/29.9, flux_kennedy_gruber
+        // 54.5/26.5; polydeg 1, 49,152 elements 89.0/82.5, 72.0/69.4)
+#pragma unroll 1
+        for (int d = 0; d < 3; ++d)
+          volume_direction64<N, VOL, NC, true>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, d, bg, vol);
+      } else {
+        volume_direction64<N, VOL, NC, line_in_wave<N>(0)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 0,
+                                                           bg, vol);
+        volume_direction64<N, VOL, NC, line_in_wave<N>(1)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 1,
+                                                           bg, vol);
+        volume_direction64<N, VOL, NC, line_in_wave<N>(2)>(q, l, s_w, s_buf, s_ds, tl, ti, tj, tk, 2,
+                                                           bg, vol);
+      }
       volume_scale64<VOL>(vol);
     }
   }
