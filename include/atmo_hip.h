@@ -311,10 +311,13 @@ int atmo_swe_create(const atmo_swe_config* config, const atmo_geometry2d* geomet
  * fastest; `ms` (may be NULL, else room for ATMO_SWE_VARIANTS values)
  * receives the time of each shape.  Covariant form: node lanes of 1, 2
  * or 4 waves per workgroup that do all the work (0..2) or share it with two
- * more sets of waves (3..5; ATMO_SWE_VARIANTS shapes).  3D Euler: one or two elements per workgroup (variants 0 and 1;
- * the second is built for polydeg 3 and 4 of the direct volume form, elsewhere
- * variant 0 is the only shape and its time is reported as 0).  atmo_step and
- * atmo_solve tune by themselves on their first call; every shape gives
+ * more sets of waves (3..5; ATMO_SWE_VARIANTS shapes).  3D Euler: one or two
+ * elements per workgroup (variants 0 and 1; the second is built for polydeg 3
+ * and 4 of the direct volume form, elsewhere variant 0 is the only shape and
+ * its time is reported as 0).  Up to 409 elements at polydeg 3 and 227 at
+ * polydeg 4 the FP64 forms have one shape for either variant: its time is
+ * reported for both, 0 is chosen, and pinning 1 changes nothing.  atmo_step
+ * and atmo_solve tune by themselves on their first call; every shape gives
  * bit-identical results. */
 #define ATMO_SWE_VARIANTS 6
 int atmo_autotune(atmo_handle* handle, int32_t* variant, double* ms);

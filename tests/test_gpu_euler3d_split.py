@@ -76,3 +76,26 @@ def test_direct_form_shapes_are_bit_identical(polydeg, trees):
         got.append((du, u, semi.get_state()))
     for a, b in zip(*got):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("polydeg,trees,one_shape", [(3, (409, 1, 1), True), (3, (410, 1, 1), False),
+                                                     (4, (227, 1, 1), True), (4, (228, 1, 1), False)])
+def test_autotuner_on_both_sides_of_the_line(polydeg, trees, one_shape):
+    """the split form is one kernel for either variant: the tuner chooses 0 and
+    reports its one time for both; beyond the line each shape has a time of its
+    own"""
+    mesh = T.P4estMesh(trees, polydeg=polydeg, coordinates_min=(0.0, 0.0, 0.0),
+                       coordinates_max=(float(trees[0]), 1.0, 1.0))
+    eq = T.CompressibleEulerEnergyEquationsWithGravity3D(c_p=1004.0, c_v=717.0, gravity=9.81)
+    solver = T.DGSEM(polydeg=polydeg, surface_flux=("flux_lax_friedrichs", "flux_zero"),
+                     volume_integral=T.VolumeIntegralFluxDifferencing(("flux_ranocha",
+                                                                       "flux_zero")))
+    semi = T.SemidiscretizationHyperbolic(mesh, eq, solver)
+    semi.set_state(T.initial_condition_periodic_modes(mesh, eq, 3))
+    runs = [semi.autotune() for _ in range(3)]
+    assert all(ms[0] > 0 and ms[1] > 0 for _, ms in runs)
+    if one_shape:
+        assert all(chosen == 0 and ms[0] == ms[1] for chosen, ms in runs), runs
+    else:
+        assert any(ms[0] != ms[1] for _, ms in runs), runs
+    semi.set_kernel_variant(1)  # accepted on both sides

@@ -250,10 +250,13 @@ namespace atmo {
 // workgroup on the RK stage (the launch the time loops make) and keeps the
 // faster.  The resident state is read; the scratch buffers d_u2 (the stage
 // output) and d_du (as the register) are written.  Every shape gives the same
-// bits (each element's arithmetic does not depend on its workgroup).
+// bits (each element's arithmetic does not depend on its workgroup).  On a mesh
+// that runs the split form both variants launch that one kernel: there is
+// nothing to choose, and only a caller who asks for times has it timed.
 int e3_autotune(atmo_handle* h, double* ms_per_variant) {
   if (ms_per_variant) ms_per_variant[0] = ms_per_variant[1] = 0.0;
-  if (!e3_has_two_element_groups(h->n, h->cfg.precision)) {
+  const bool split = e3_takes_split_form(h->n, h->cfg.precision, h->cfg.n_elements);
+  if (!e3_has_two_element_groups(h->n, h->cfg.precision) || (split && !ms_per_variant)) {
     h->e3_epb = 1;
     h->e3_tuned = true;
     return ATMO_OK;
@@ -269,7 +272,7 @@ int e3_autotune(atmo_handle* h, double* ms_per_variant) {
   L.rk_a = L.rk_dt = L.rk_b = 0.0;
   float best_of[2] = {1e30f, 1e30f};
   for (int round = 0; round < 3; ++round)
-    for (int v = 0; v < 2; ++v) {
+    for (int v = 0; v < (split ? 1 : 2); ++v) {
       L.epb = v + 1;
       if (!launch_stage_only(h, L)) continue;
       HIP_TRY(h, hipEventRecord(a, h->stream));
@@ -284,6 +287,7 @@ int e3_autotune(atmo_handle* h, double* ms_per_variant) {
   hipEventDestroy(a);
   hipEventDestroy(b);
   HIP_TRY(h, hipGetLastError());
+  if (split) best_of[1] = best_of[0];
   // two only where they win by more than a tie: at polydeg 4 on 12,288 elements
   // both measure 102.1 +- 0.3 us here, while a loop of steps takes 110.4 a stage
   // with one and 112.5 with two (on 1,536 elements 18.2 and 17.9 here, 18.3 and

@@ -15,4 +15,17 @@ bool e3_has_two_element_groups(int n, int precision) {
     default: return false;
   }
 }
+
+bool e3_takes_split_form(int n, int precision, int n_elements) {
+  if (precision != 0 && precision != 3) return false;
+  switch (n) {
+    case 2: return n_elements <= split_max_elements<2>();
+    case 3: return n_elements <= split_max_elements<3>();
+    case 4: return n_elements <= split_max_elements<4>();
+    case 5: return n_elements <= split_max_elements<5>();
+    case 6: return n_elements <= split_max_elements<6>();
+    case 7: return n_elements <= split_max_elements<7>();
+    default: return false;
+  }
+}
 }  // namespace atmo

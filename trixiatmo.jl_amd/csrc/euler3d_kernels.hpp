@@ -51,6 +51,8 @@ struct E3Launch {
 // whether the stage kernel of this polydeg / precision has a two-element
 // workgroup shape (the 3D autotuner's choice)
 bool e3_has_two_element_groups(int n, int precision);
+// whether a mesh of n_elements runs the split form, which has one shape
+bool e3_takes_split_form(int n, int precision, int n_elements);
 
 // background state from the geopotential of u: (rho_bg, 0, 0, 0, p_bg/(gamma-1), phi)
 void e3_launch_background_state(const E3Launch& L, const double* u, double* ubg, hipStream_t s);

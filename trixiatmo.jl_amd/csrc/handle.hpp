@@ -130,6 +130,8 @@ int swe_autotune(atmo_handle* h, double* ms_per_variant);
 int e3_autotune(atmo_handle* h, double* ms_per_variant);
 // whether the 3D stage of this polydeg / precision has the two-element shape
 bool e3_has_two_element_groups(int n, int precision);
+// whether a mesh of n_elements runs the split form, which has one shape
+bool e3_takes_split_form(int n, int precision, int n_elements);
 // rainy Euler paths of the generic entry points
 int rainy_rhs_device(atmo_handle* h, double* du, const double* u, double t);
 int rainy_step(atmo_handle* h, double dt, int n_steps);
