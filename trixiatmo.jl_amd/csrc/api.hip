@@ -616,28 +616,19 @@ int atmo_create(const atmo_config* cfg, const atmo_geometry3d* g, atmo_handle** 
     h->weights = b.w;
   }
   const size_t sb = sizeof(double) * h->len;
+  const size_t cb = sizeof(double) * 9 * n3 * (size_t)E, nb = sizeof(double) * n3 * (size_t)E;
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipMalloc(&h->d_u, sb) != hipSuccess || hipMalloc(&h->d_u2, sb) != hipSuccess ||
-      hipMalloc(&h->d_k, sb) != hipSuccess || hipMalloc(&h->d_du, sb) != hipSuccess ||
-      hipMalloc(&h->d_uio, sb) != hipSuccess || hipMalloc(&h->d_duio, sb) != hipSuccess ||
-      hipMalloc(&h->d_cv, sizeof(double) * 9 * n3 * (size_t)E) != hipSuccess ||
-      hipMalloc(&h->d_invJ, sizeof(double) * n3 * (size_t)E) != hipSuccess ||
-      hipMalloc(&h->d_nbr, sizeof(int32_t) * nbr.size()) != hipSuccess ||
-      hipMalloc(&h->d_face_info, sizeof(int32_t) * face_info.size()) != hipSuccess ||
-      hipMalloc(&h->d_partial, sizeof(double) * 9 * (size_t)E) != hipSuccess ||
-      !alloc_result(h, 16) ||
-      (cfg->precision != ATMO_PREC_FP64 &&
-       hipMalloc(&h->d_cv32, sizeof(float) * 9 * n3 * (size_t)E) != hipSuccess) ||
-      (h->bg_on && (hipMalloc(&h->d_ubg, sb) != hipSuccess || hipMalloc(&h->d_dubg, sb) != hipSuccess ||
-                    hipMalloc(&h->d_B, sizeof(float) * 3 * n3 * (size_t)E) != hipSuccess))) {
+      hipMalloc(&h->d_cv, cb) != hipSuccess || hipMalloc(&h->d_invJ, nb) != hipSuccess ||
+      (cfg->precision != ATMO_PREC_FP64 && hipMalloc(&h->d_cv32, cb / 2) != hipSuccess)) {
     fail(nullptr, ATMO_ERR_DEVICE, "device allocation failed");
     return cleanup_fail(ATMO_ERR_DEVICE);
   }
   {
     // the vectors in the caller's layout, uploaded or computed on the device
-    // from the node coordinates alone, then as the rows the stages read
+    // from the node coordinates alone, then as the rows the stages read; before
+    // the states take their memory, so that this second copy adds nothing to
+    // the largest amount a handle holds at once
     double *d_xyz = nullptr, *d_cv9 = nullptr;
-    const size_t cb = sizeof(double) * 9 * n3 * (size_t)E, nb = sizeof(double) * n3 * (size_t)E;
     bool ok = hipMalloc(&d_cv9, cb) == hipSuccess;
     if (ok && metric_on_device) {
       Basis b(n);
@@ -660,6 +651,18 @@ int atmo_create(const atmo_config* cfg, const atmo_geometry3d* g, atmo_handle** 
            metric_on_device ? "metric terms on the device failed" : "device upload failed");
       return cleanup_fail(ATMO_ERR_DEVICE);
     }
+  }
+  if (hipMalloc(&h->d_u, sb) != hipSuccess || hipMalloc(&h->d_u2, sb) != hipSuccess ||
+      hipMalloc(&h->d_k, sb) != hipSuccess || hipMalloc(&h->d_du, sb) != hipSuccess ||
+      hipMalloc(&h->d_uio, sb) != hipSuccess || hipMalloc(&h->d_duio, sb) != hipSuccess ||
+      hipMalloc(&h->d_nbr, sizeof(int32_t) * nbr.size()) != hipSuccess ||
+      hipMalloc(&h->d_face_info, sizeof(int32_t) * face_info.size()) != hipSuccess ||
+      hipMalloc(&h->d_partial, sizeof(double) * 9 * (size_t)E) != hipSuccess ||
+      !alloc_result(h, 16) ||
+      (h->bg_on && (hipMalloc(&h->d_ubg, sb) != hipSuccess || hipMalloc(&h->d_dubg, sb) != hipSuccess ||
+                    hipMalloc(&h->d_B, sizeof(float) * 3 * n3 * (size_t)E) != hipSuccess))) {
+    fail(nullptr, ATMO_ERR_DEVICE, "device allocation failed");
+    return cleanup_fail(ATMO_ERR_DEVICE);
   }
   if (hipMemcpy(h->d_nbr, nbr.data(), sizeof(int32_t) * nbr.size(), hipMemcpyHostToDevice) !=
           hipSuccess ||
