@@ -645,7 +645,8 @@ int atmo_swe_create(const atmo_swe_config* cfg, const atmo_geometry2d* g, atmo_h
   L.n_elements = E;
   L.volume_flux = cfg->volume_flux;
   L.surface_flux = cfg->surface_flux;
-  L.surface_noncons = cfg->surface_noncons;
+  // surface_noncons: with one set of auxiliary variables on both sides of a face
+  // the two nonconservative surface terms are the same (face_flux)
   L.source_terms = cfg->source_terms;
   L.gravity = cfg->gravity;
   L.rotation_rate = cfg->rotation_rate;

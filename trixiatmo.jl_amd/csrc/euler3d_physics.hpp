@@ -246,25 +246,6 @@ __device__ __forceinline__ void flux_kennedy_gruber(const Prim<T>& l, const Prim
   f[4] = f1 * ea + pa * vna;
 }
 
-// flux_shima_etal, :248-276
-template <typename T>
-__device__ __forceinline__ void flux_shima(const E3Params& q, const Prim<T>& l, const Prim<T>& r,
-                                           const T n0, const T n1, const T n2, T f[5]) {
-  const T vnl = l.v1 * n0 + l.v2 * n1 + l.v3 * n2;
-  const T vnr = r.v1 * n0 + r.v2 * n1 + r.v3 * n2;
-  const T ra = T(0.5) * (l.rho + r.rho);
-  const T v1a = T(0.5) * (l.v1 + r.v1), v2a = T(0.5) * (l.v2 + r.v2), v3a = T(0.5) * (l.v3 + r.v3);
-  const T vna = T(0.5) * (vnl + vnr);
-  const T pa = T(0.5) * (l.p + r.p);
-  const T vsq = T(0.5) * (l.v1 * r.v1 + l.v2 * r.v2 + l.v3 * r.v3);
-  const T f1 = ra * vna;
-  f[0] = f1;
-  f[1] = f1 * v1a + pa * n0;
-  f[2] = f1 * v2a + pa * n1;
-  f[3] = f1 * v3a + pa * n2;
-  f[4] = f1 * vsq + pa * vna * T(q.inv_gm1) + T(0.5) * (l.p * vnr + r.p * vnl);
-}
-
 // pointwise flux, :77-91.  The reference takes `rho_e = last(u)`, the sixth
 // entry (phi), for the energy flux; kept as the reference has it.
 template <typename T>
@@ -321,21 +302,6 @@ __device__ __forceinline__ void flux_lmars(const E3Params& q, const T* ul, const
   f[3] = v * us[3] + p * n2;
   f[4] = v * us[4] + ps * v;
   f[5] = T(0);
-}
-
-// flux_nonconservative_waruszewski_etal (:135-159) / souza_etal (:206-230):
-// g = rho_avg [phi] (0, n, n.v_avg, 0); only entries 1..4 are nonzero.
-template <int NC, typename T>
-__device__ __forceinline__ void noncons_gravity(const Prim<T>& l, const Prim<T>& r, const T n0,
-                                                const T n1, const T n2, T g[4]) {
-  const T ra = (NC == 1) ? ln_mean(l.rho, r.rho) : T(0.5) * (l.rho + r.rho);
-  const T jump = r.phi - l.phi;
-  const T s = ra * jump;
-  const T v1a = T(0.5) * (l.v1 + r.v1), v2a = T(0.5) * (l.v2 + r.v2), v3a = T(0.5) * (l.v3 + r.v3);
-  g[0] = n0 * s;
-  g[1] = n1 * s;
-  g[2] = n2 * s;
-  g[3] = n0 * s * v1a + n1 * s * v2a + n2 * s * v3a;
 }
 
 }  // namespace atmo

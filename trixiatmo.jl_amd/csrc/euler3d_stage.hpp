@@ -136,13 +136,6 @@ __device__ __forceinline__ void surface_flux(const E3Params& q, int surf, const 
   }
 }
 
-template <typename T>
-__device__ __forceinline__ void surface_noncons(int snc, const Prim<T>& l, const Prim<T>& r, T n0,
-                                                T n1, T n2, T g[4]) {
-  if (snc == 1) noncons_gravity<1>(l, r, n0, n1, n2, g);
-  else noncons_gravity<2>(l, r, n0, n1, n2, g);
-}
-
 // Per-node quantities of the two-point fluxes, with the divisions and
 // logarithms done once per node instead of once per pair.
 template <typename T>
@@ -733,8 +726,8 @@ __device__ __forceinline__ void element_speed(const E3Params& q, bool active, co
   }
 }
 
-// Pair-record form: per direction the unordered pairs of every line are
-// evaluated once into LDS records, then gathered by both nodes.
+// Pair-record form of the FP32 fluxes: per direction the unordered pairs of
+// every line are evaluated once into LDS records, then gathered by both nodes.
 template <int N, int VOL, int NC, typename T, bool KAHAN>
 __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
     E3Params q, DsplitTable dst, double inv_w, int n_elements, const double* __restrict__ u,
@@ -745,18 +738,16 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
   using S = Shape<N>;
   using C = Chunking<N, T, NC>;
   constexpr int N2 = S::N2, N3 = S::N3, P = S::P, B = S::BLOCK;
-  constexpr bool MIXED = sizeof(T) == 4;
+  static_assert(sizeof(T) == 4, "FP64 takes the direct and split forms");
   constexpr int NW = NodeFields<VOL, NC, T>::NW;
   __shared__ T s_w[NW * N3];
-  __shared__ double s_phi[MIXED ? N3 : 1];  // FP64 phi for the jumps of the mixed path
-  __shared__ double s_pb[MIXED ? N3 : 1];   // FP64 background pressure
+  __shared__ double s_phi[N3];  // FP64 phi for the jumps
+  __shared__ double s_pb[N3];   // FP64 background pressure
   __shared__ T s_ja[3][N3];
   __shared__ T s_fl[C::FLEN];  // pair terms [9][NPC], later face fluxes [6][6 n^2]
   __shared__ T s_ds[N * N];
   __shared__ unsigned char s_pa[P], s_pm[P];  // node pair (a, m), a < m, of each pair slot
 
-  // the FP64 form never splits off a background: make that a compile-time fact
-  if constexpr (!MIXED) bg.on = 0;
   const int e = xcd_element(blockIdx.x, n_elements);
   if (e >= n_elements) return;  // whole workgroup: padding of the XCD mapping
   const int t = threadIdx.x;
@@ -803,9 +794,7 @@ __global__ __launch_bounds__(Shape<N>::BLOCK) void e3_stage(
         const int na = base + a * stride, nm = base + m * stride;
         const FastPrim<T> l = load_fast_prim<VOL, NC, N3, T>(s_w, na, bg);
         const FastPrim<T> r = load_fast_prim<VOL, NC, N3, T>(s_w, nm, bg);
-        T dphi;
-        if constexpr (MIXED) dphi = T(s_phi[nm] - s_phi[na]);
-        else dphi = r.phi - l.phi;
+        const T dphi = T(s_phi[nm] - s_phi[na]);
         const T n0 = T(0.5) * (s_ja[0][na] + s_ja[0][nm]);
         const T n1 = T(0.5) * (s_ja[1][na] + s_ja[1][nm]);
         const T n2 = T(0.5) * (s_ja[2][na] + s_ja[2][nm]);
@@ -1139,6 +1128,7 @@ void e3_stage_direct(
   __shared__ T s_buf_all[EPB][BUF];  // contravariant vectors [9][n^3], later face fluxes [6][6 n^2]
   __shared__ T s_ds[N * N + 1];  // and a slot for the lanes past the table
 
+  // the FP64 form never splits off a background: make that a compile-time fact
   if constexpr (!MIXED) bg.on = 0;
   const int n_groups = (n_elements + EPB - 1) / EPB;
   const int grp = xcd_element(blockIdx.x, n_groups);

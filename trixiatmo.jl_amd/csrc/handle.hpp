@@ -149,10 +149,7 @@ bool swe_fuses_control(const atmo_handle* h);
 int rainy_enqueue_resident_step(atmo_handle* h);
 // ptr[0 .. n) = value, stream-ordered (a value for kernels that read it from memory)
 void launch_fill(double* ptr, double value, int n, hipStream_t s);
-// dt[m] and the clock of n_members members from their maximum wave speeds
-void launch_step_control(const double* max_speed, int n_members, int n, double* clock, double* dt,
-                         hipStream_t s);
-// the same for one member from per-element partial maxima
+// dt and the clock of one member from its elements' wave speeds
 void launch_step_control_reduce(const double* partial, int n_items, int n, double* clock,
                                 double* dt, hipStream_t s);
 // result[0] = the maximum of floor and the n partials (NaN propagates)

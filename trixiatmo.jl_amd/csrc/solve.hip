@@ -1,15 +1,16 @@
 // The time loop of the examples' solve(ode, CarpenterKennedy2N54(williamson_condition
 // = false); callback = StepsizeCallback(cfl)) (e.g.
 // examples/shallow_water/covariant/elixir_barotropic_instability.jl:79-80)
-// kept on the device.  Every step is the maximum-wave-speed reduction of the
-// resident state, a one-thread-per-member control kernel that turns it into
-// the step size (cut to end at t_end, as OrdinaryDiffEq's tstop handling
-// does) and the five fused stages, which read the step size from device
-// memory.  Two steps are captured as one graph and replayed; the host reads
-// the clock back only every `check_every` steps.  A member that has reached
-// t_end takes steps of size 0, which leave its state unchanged, so the
-// members of an ensemble each follow their own step sizes and finish
-// together.
+// kept on the device.  Every step begins with its control, a workgroup per
+// member that reduces the elements' wave speeds and turns them into the step
+// size (cut to end at t_end, as OrdinaryDiffEq's tstop handling does); the five
+// fused stages read the step size from device memory, and the last of them
+// writes the new state's speeds.  On small covariant meshes the control is part
+// of the first stage instead.  Two steps are captured as one graph and
+// replayed; the host reads the clock back only every `check_every` steps.  A
+// member that has reached t_end takes steps of size 0, which leave its state
+// unchanged, so the members of an ensemble each follow their own step sizes
+// and finish together.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,20 +25,13 @@ namespace atmo {
 
 namespace {
 
-__device__ __forceinline__ void step_control_kernel_body(double max_speed, const ClockIn& c, int m,
-                                                         int M, int n, double* clock, double* dt) {
+__device__ __forceinline__ void store_step_control(double max_speed, const ClockIn& c, int m,
+                                                   int M, int n, double* clock, double* dt) {
   const ClockOut o = step_control(max_speed, c, n);
   if (o.failed) clock[3 * M] = 1.0;  // every member that finds one stores the same value
   clock[2 * M + m] = o.steps;
   clock[m] = o.t;
   dt[m] = o.dt;
-}
-
-__global__ void step_control_kernel(const double* __restrict__ max_speed, int M, int n,
-                                    double* clock, double* dt) {
-  const int m = blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < M)
-    step_control_kernel_body(max_speed[m], load_clock(clock, dt, m, M), m, M, n, clock, dt);
 }
 
 // maximum over partial[from .. to) of a workgroup of B lanes, on every lane of
@@ -65,7 +59,7 @@ __device__ __forceinline__ double block_max(const double* __restrict__ partial, 
   return m;
 }
 
-// the same for one member whose maximum speed is the maximum over per-element
+// the control of one member whose maximum speed is the maximum over per-element
 // partials (written by the last stage of the step just taken).  One chain of
 // latencies between two stages: the clock is loaded beside the partials, and
 // the workgroup has as many lanes as one batch of block_max needs
@@ -75,7 +69,7 @@ __global__ __launch_bounds__(B) void step_control_reduce_kernel(const double* __
                                                                 double* dt) {
   const ClockIn c = load_clock(clock, dt, 0, 1);
   const double m = block_max<B>(partial, 0, n_items, 0.0);
-  if (threadIdx.x == 0) step_control_kernel_body(m, c, 0, 1, n, clock, dt);
+  if (threadIdx.x == 0) store_step_control(m, c, 0, 1, n, clock, dt);
 }
 
 // one workgroup per ensemble member: its maximum speed is the maximum over the
@@ -86,7 +80,7 @@ __global__ __launch_bounds__(256) void step_control_members_reduce_kernel(
   const int m = blockIdx.x;
   const ClockIn c = load_clock(clock, dt, m, M);
   const double mx = block_max<256>(partial, member_first[m], member_first[m + 1], 0.0);
-  if (threadIdx.x == 0) step_control_kernel_body(mx, c, m, M, n, clock, dt);
+  if (threadIdx.x == 0) store_step_control(mx, c, m, M, n, clock, dt);
 }
 
 __global__ __launch_bounds__(1024) void reduce_max_kernel(const double* __restrict__ partial, int n,
@@ -135,12 +129,6 @@ void launch_step_control_members_reduce(const double* partial, const int* member
                                         hipStream_t s) {
   hipLaunchKernelGGL(step_control_members_reduce_kernel, dim3(n_members), dim3(256), 0, s, partial,
                      member_first, n_members, n, clock, dt);
-}
-
-void launch_step_control(const double* max_speed, int n_members, int n, double* clock, double* dt,
-                         hipStream_t s) {
-  hipLaunchKernelGGL(step_control_kernel, dim3((n_members + 63) / 64), dim3(64), 0, s, max_speed,
-                     n_members, n, clock, dt);
 }
 
 namespace {

@@ -11,7 +11,6 @@ struct SweLaunch {
   int volume_flux;      // 0 flux_ec, 1 flux_central, 2 weak form of the standard form
   int surface_flux;     // 0 FluxPlusDissipation(flux_ec, LLF), 1 flux_lax_friedrichs, 2 flux_ec,
                         // 3 flux_lax_friedrichs of the standard form
-  int surface_noncons;  // 0 surface_simplified, 1 flux_nonconservative_ec (split form only)
   int source_terms;     // 1 source_terms_geometric_coriolis, 2 the same of the standard form
   double gravity, rotation_rate;
   double dsplit[64];    // Dsplit[i * n + m]
