@@ -196,13 +196,39 @@ def test_mixed_precision_rhs_error(oracle, precision, case):
             assert diff[v] <= 1e-10 * umax[v], (v, diff, umax)
 
 
-@pytest.mark.parametrize("case", ["shell_p4", "cube_odd_p4", "cube_odd_p3"])
+def beyond_the_split_line(polydeg, precision="fp64"):
+    """moving air under gravity between walls on more elements than the split form
+    takes (227 at polydeg 4, 409 at polydeg 3): a shell of 294, a brick of 867"""
+    if polydeg == 4:
+        mesh, eq, solver, bcs, u0 = T.workloads.shell(7, 1, polydeg=4, seed=1, precision=precision)
+        u0 = u0.copy()
+        u0[1:4] += 10.0 * np.sin(mesh.node_coordinates / 1e6) * u0[0]
+        return mesh, eq, solver, bcs, u0
+    _, eq, solver, _, _ = T.workloads.shell(1, 1, polydeg=polydeg, precision=precision)
+    mesh = T.P4estMesh((17, 17, 3), polydeg=polydeg, coordinates_min=(0.0, 0.0, 0.0),
+                       coordinates_max=(17e3, 17e3, 3e3), periodicity=(True, True, False))
+    x = mesh.node_coordinates
+    phi, R = eq.gravity * x[2], eq.c_p - eq.c_v
+    p = 1e5 * np.exp(-phi / (R * 250.0))
+    rho = p / (R * 250.0)
+    v = 10.0 * np.sin(2.0 * np.pi * x[[1, 2, 0]] / np.array([17e3, 3e3, 17e3])[:, None, None, None, None])
+    E = p / (eq.c_p / eq.c_v - 1.0) + 0.5 * rho * (v ** 2).sum(axis=0)
+    return mesh, eq, solver, None, np.stack([rho, *(rho * v), E, phi])
+
+
+@pytest.mark.parametrize("case", ["shell_p4", "cube_odd_p4", "cube_odd_p3",
+                                  "direct_shell_p4", "direct_brick_p3"])
 def test_autotuner_shapes_are_bit_identical(case):
     """the 3D stage's workgroup shapes (one or two elements per workgroup,
     chosen by the autotuner) give the same bits: rhs!, RK steps replayed from
-    the captured graph, and the resident loop; an odd element count leaves the
-    last two-element workgroup half filled"""
-    if case == "shell_p4":
+    the captured graph, and the resident loop.  The two direct cases lie beyond
+    the split form's line, with walls and the gravity term: a shell, and a brick
+    of an odd element count, which leaves the last two-element workgroup half
+    filled.  The other three run the split form for either shape and check that
+    pinning one changes nothing"""
+    if case.startswith("direct"):
+        mesh, eq, solver, bcs, u0 = beyond_the_split_line(4 if case.endswith("p4") else 3)
+    elif case == "shell_p4":
         mesh, eq, solver, bcs, u0 = T.workloads.shell(3, 2, polydeg=4, seed=1)
         u0 = u0.copy()
         u0[1:4] += 10.0 * np.sin(mesh.node_coordinates / 1e6) * u0[0]

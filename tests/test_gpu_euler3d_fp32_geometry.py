@@ -22,6 +22,7 @@ import pytest
 import trixiatmo_hip as T
 from trixiatmo_hip import workloads as W
 from oracle_lib import params_for
+from test_gpu_euler3d import beyond_the_split_line
 
 pytestmark = pytest.mark.gpu
 
@@ -96,9 +97,14 @@ def test_entropy_rate_of_the_ec_shell():
     assert abs(rate) <= 1e-6 * scale
 
 
-@pytest.mark.parametrize("name", ["shell_p4", "cube_p3"])
+@pytest.mark.parametrize("name", ["shell_p4", "cube_p3", "direct_shell_p4", "direct_brick_p3"])
 def test_shapes_and_resident_loop_are_bit_identical(name):
-    if name == "shell_p4":
+    """one and two elements per workgroup and the host and resident loops; the
+    direct cases lie beyond the split form's line, the other two run the split
+    form for either shape"""
+    if name.startswith("direct"):
+        mesh, eq, solver, bcs, u0 = beyond_the_split_line(int(name[-1]), GEO)
+    elif name == "shell_p4":
         mesh, eq, solver, bcs, u0 = _case("shell_flow", GEO)
     else:
         mesh, eq, solver, bcs, u0 = W.periodic_cube(trees=3, polydeg=3, seed=2, precision=GEO)

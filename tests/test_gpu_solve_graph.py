@@ -20,11 +20,13 @@ def make(family):
         mesh, eq, solver, src, lim, u0, _ = W.rainy_bubble(cells=(8, 4), polydeg=3, seed=3)
         return (lambda: T.SemidiscretizationRainy(mesh, eq, solver, source_terms=src,
                                                   stage_limiter=lim)), u0
-    mesh, eq, solver, bcs, u0 = W.shell(trees_per_face=2, layers=2, polydeg=3, seed=1)
+    # 48 elements, either shape the split form, or 486 beyond its line
+    trees, layers = (9, 1) if family.endswith("direct") else (2, 2)
+    mesh, eq, solver, bcs, u0 = W.shell(trees, layers, polydeg=3, seed=1)
     return (lambda: T.SemidiscretizationHyperbolic(mesh, eq, solver, bcs)), u0
 
 
-@pytest.mark.parametrize("family", ["covariant", "rainy", "euler3d"])
+@pytest.mark.parametrize("family", ["covariant", "rainy", "euler3d", "euler3d_direct"])
 def test_pieces_on_one_handle(family):
     print(f"case: {family}", flush=True)
     build, u0 = make(family)
