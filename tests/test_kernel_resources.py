@@ -1,7 +1,9 @@
-"""Scratch memory of the stage kernels in the built library, from the metadata
-the compiler leaves in its code objects: a stage that spills registers loses
-10 to 100 % of its speed, so the one-element FP64 forms of the 3D stage, the
-covariant and the rainy stages take none, at any polydeg and flux."""
+"""Scratch memory and registers of the stage kernels in the built library, from
+the metadata the compiler leaves in its code objects.  A stage that spills loses
+10 to 100 % of its speed: the one-element FP64 forms of the 3D stage, the
+covariant and the rainy stages take no scratch, at any polydeg and flux.  The
+FP32 direct form keeps within the 96 registers of five waves per SIMD, without
+which a third workgroup of polydeg 6 no longer fits a CU."""
 import os
 import re
 import struct
@@ -51,24 +53,39 @@ def kernels(code):
             at += desc + 3 & ~3
 
 
-def test_stage_kernels_take_no_scratch():
+@pytest.fixture(scope="module")
+def metadata():
     if not os.path.exists(LIB):
         raise FileNotFoundError(f"{LIB} is missing: run __graft_entry__.build()")
     with open(LIB, "rb") as f:
         lib = f.read()
+    return {k[".name"]: k for code in code_objects(lib) for k in kernels(code)}
+
+
+def test_stage_kernels_take_no_scratch(metadata):
     # template arguments: nodes, volume flux, gravity term, FP64, no Kahan, one
     # element a workgroup, either geometry storage
     direct = re.compile(r"e3_stage_directILi(\d)ELi\dELi\dEdLb0ELi1E[df]EE")
     seen, scratch = set(), {}
-    for code in code_objects(lib):
-        for k in kernels(code):
-            name = k[".name"]
-            m = direct.search(name)
-            kind = "e3 " + m[1] if m else next((s for s in ("9swe_stageI", "11rainy_stageI")
-                                                if s in name), None)
-            if kind:
-                seen.add(kind)
-                if k[".private_segment_fixed_size"]:
-                    scratch[name] = k[".private_segment_fixed_size"]
+    for name, k in metadata.items():
+        m = direct.search(name)
+        kind = "e3 " + m[1] if m else next((s for s in ("9swe_stageI", "11rainy_stageI")
+                                            if s in name), None)
+        if kind:
+            seen.add(kind)
+            if k[".private_segment_fixed_size"]:
+                scratch[name] = k[".private_segment_fixed_size"]
     assert seen == {f"e3 {n}" for n in range(2, 9)} | {"9swe_stageI", "11rainy_stageI"}
     assert not scratch, scratch
+
+
+def test_fp32_direct_form_runs_five_waves_per_simd(metadata):
+    direct = re.compile(r"e3_stage_directILi(\d)ELi\dELi\dEfLb[01]ELi1EfEE")
+    seen, large = set(), {}
+    for name, k in metadata.items():
+        if m := direct.search(name):
+            seen.add(int(m[1]))
+            if k[".vgpr_count"] > 96 or k[".private_segment_fixed_size"]:
+                large[name] = k[".vgpr_count"], k[".private_segment_fixed_size"]
+    assert seen == {2, 3, 4, 6, 7, 8}  # polydeg 4 runs the pair-record form
+    assert not large, large

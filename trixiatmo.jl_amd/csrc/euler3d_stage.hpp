@@ -1208,7 +1208,11 @@ void e3_stage_direct(
   // during the face phase
   face_links<N, EPB, FacePrefetch<N, EPB>::PF, FacePrefetch<N, EPB>::PASSES>(pf, e0, n_valid, t,
                                                                              nbr, face_info);
-  constexpr bool LATE = FacePrefetch<N, EPB>::PASSES > 1;
+  // (not where the face phase takes two passes, nor in the FP32 forms: held
+  // through it they take 98 registers instead of 86 to 96, four waves per SIMD
+  // instead of five; polydeg 6, 926,100 nodes, flux_ranocha 122.3 against 107.8 us
+  // a stage, flux_kennedy_gruber 97.8 against 86.2)
+  constexpr bool LATE = FacePrefetch<N, EPB>::PASSES > 1 || MIXED;
   NodeRest rest;
   if (!LATE && active) rest = load_rest<N>(e, tl, invJ, kreg, mode);
   FaceNormals<N, T, EPB> fn;
