@@ -32,9 +32,14 @@ __device__ __forceinline__ float rcp_refined(float x) { return __builtin_amdgcn_
 // a / b from a reciprocal refined by one Newton step and one correction of
 // the quotient by its residual: six VALU operations instead of the eleven of
 // the IEEE division sequence, within one unit in the last place of the
-// IEEE quotient (no special operands reach it: b is a nonzero difference
-// of two values or of their logarithms, a positive series denominator or a
-// sum of positive terms)
+// IEEE quotient for normal operands and quotients.  Special operands do not
+// follow IEEE: where b is zero, infinite or subnormal the result is a NaN or
+// worthless.  The callers' denominators are nonzero in a valid state
+// (densities, depths, temperatures, determinants, sums of positive terms,
+// differences of values or of their logarithms away from the series branch,
+// pivots of the saturation solve); in an invalid one the NaN reaches the state
+// or the wave speed, and the step-size control refuses it as it does an
+// infinity
 __device__ __forceinline__ double div_nr(double a, double b) {
   const double r = rcp_refined(b);
   const double q = a * r;
@@ -47,7 +52,7 @@ __device__ __forceinline__ float div_nr(float a, float b) { return div_(a, b); }
 // (Markstein, IA-64 and Elementary Functions, 2000, ch. 9), without the
 // exponent scaling that keeps a library square root exact near the ends of
 // the exponent range (the speeds and normals here are far from them);
-// sqrt(0) = 0
+// sqrt(0) = 0, NaN for a negative or infinite operand
 __device__ __forceinline__ double sqrt_(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;

@@ -42,7 +42,7 @@
 // 12.2, polydeg 7 49.5 -> 47.2 (with the logarithmic means).  The register
 // budget decides what can be asked for early: 28 B of scratch per lane cost
 // 10 % (106 against 96 ms), so polydeg 3 and 4, whose faces take two passes,
-// ask for the register after the faces.
+// and the FP32 forms ask for the register after the faces.
 #ifndef ATMO_EULER3D_STAGE_HPP
 #define ATMO_EULER3D_STAGE_HPP
 
@@ -1099,13 +1099,17 @@ __device__ __forceinline__ void volume_scale(Acc<T, KAHAN>* acc, Acc<T, KAHAN>* 
   }
 }
 
-// Direct form: every node evaluates the two-point flux with each of its n-1
-// partners on each line itself (each unordered pair is evaluated by both of
-// its nodes).  The fluxes are symmetric and the gravity terms antisymmetric
-// under exchanging the two states bit for bit, so the result equals the
-// pair-record form's exactly; in exchange for twice the flux arithmetic the
-// volume phase needs no pair buffer and no barrier, which leaves LDS for more
-// resident workgroups.
+// Direct form: a node sums its volume terms itself, from the node fields in
+// LDS, so that the volume phase needs no pair buffer and no barrier, which
+// leaves LDS for more resident workgroups.  FP32 (volume_direction): every node
+// evaluates the two-point flux with each of its n-1 partners on each line, so
+// each unordered pair is evaluated by both of its nodes; the fluxes are symmetric
+// and the gravity terms antisymmetric under exchanging the two states bit for
+// bit, so the result equals the pair-record form's exactly.  FP64
+// (volume_direction64): the gravity term is folded into the pressure, and where
+// a line's nodes belong to one wave each pair is evaluated once and handed over
+// by a lane exchange (polydeg 1 to 3, two directions of polydeg 7); elsewhere
+// both nodes evaluate it.
 // G: storage type of the contravariant vectors in memory (T, or float for the
 // FP64 form with FP32 geometry storage: widened to T where they are read)
 template <int N, int VOL, int NC, typename T, bool KAHAN, int EPB = 1, typename G = T>
@@ -1374,8 +1378,9 @@ constexpr bool has_two_element_groups() {
 // polydeg 2 (648 elements) 7.5/6.6, polydeg 3 (300) 9.0/7.6, polydeg 4 (192)
 // 10.0/7.1, polydeg 5 (192) 11.1/10.4, polydeg 6 (192) 16.2/15.9; beyond it
 // polydeg 3 (648) 9.7/10.7, polydeg 4 (648) 14.6/17.0, polydeg 5 (300)
-// 14.9/18.2.  Polydeg 7, whose volume terms one set of waves has to take,
-// gains nothing.
+// 14.9/18.2.  At polydeg 6 one set of waves has to take the volume terms of all
+// three directions, so only the faces leave the chain; polydeg 7, of which the
+// same holds, gains nothing.
 template <int N>
 constexpr int split_max_elements() {
   return N <= 7 ? 2048 / (SplitShape<N>::LANES / 64) : 0;
